@@ -9,11 +9,14 @@
 // fp32 scales cannot ride in the MFMA's e8m0 scale operands, so every K group
 // is "promoted" on the VALU: per 32x32 sub-tile two chained MFMAs (the group's
 // two 64-deep K-steps) produce a fresh partial P, then acc += P * sa * sb.
-// M > 192 runs the 8-wave K loop of blockscale_core.h over 256 x 256 tiles;
-// narrow M streams the weights through registers (blockscale_narrow_kernel).
+// Large products run the 8-wave K loop of blockscale_core.h over 256 x 256
+// tiles, fewer rows smaller tiles with K split over the workgroup's waves
+// (gemm_kgroup.h), and a few rows of short K stream the weights through
+// registers (blockscale_narrow_kernel).
 #include <cstdlib>
 
 #include "blockscale_core.h"
+#include "gemm_kgroup.h"
 #include "hkq_host.h"
 
 namespace hkq {
@@ -168,48 +171,26 @@ __global__ __launch_bounds__(64 * BS_NW, 1) void blockscale_gemm_kernel(const Bl
 }
 
 // ---------------------------------------------------------------------------
-// Narrow M (M <= 64): the streaming layout of the dense GEMMs' narrow path
+// Narrow M (M <= 16): the streaming layout of the dense GEMMs' narrow path
 // (workgroup = 16*NT columns for all rows, 4 waves splitting K, fragments
 // loaded straight into registers for the 16x16x128 MFMA; lane l supplies row
 // l % 16, bytes [16q, 16q+16) and [64+16q, 64+16q+16) of the step, q = l/16,
 // and holds D[4q + i][l % 16]). A 128-value K-step is exactly one scale
 // group, so each step's MFMA starts from zero and is promoted at once:
-// acc += P * sa[m, g] * sb[g, n / GN]. Rows come in MT tiles of 16. The
-// 256 x 256 tiles of the main kernel would give M <= 64 only N/256
-// workgroups.
-constexpr int BSN_WAVES = 4, BSN_MAX_M = 64;
+// acc += P * sa[m, g] * sb[g, n / GN].
+constexpr int BSN_WAVES = 4, BSN_MAX_M = 16;
 
-template <bool GN1, int MT, int NT>
+template <bool GN1, int NT>
 struct BsNarrowFrag {
-    v4i b0[NT], b1[NT], a0[MT], a1[MT];
-    float sa[MT];                // sa[m, g] of the lane's rows
+    v4i b0[NT], b1[NT], a0, a1;
+    float sa;                    // sa[m, g] of the lane's row
     float sb[NT][GN1 ? 4 : 1];   // sb[g, n] of the lane's 4 columns (GN 1) or of the tile's column block
 };
 
-// Rows [64 * blockIdx.y, 64 * blockIdx.y + 64) of the GEMM as a GEMM of their own.
-__device__ __forceinline__ BlockScaleParams bs_row_slice(const BlockScaleParams& pb) {
-    BlockScaleParams p = pb;
-    const int m0 = blockIdx.y * BSN_MAX_M;
-    if (m0 > 0) {
-        p.A += (int64_t)m0 * p.lda;
-        p.sa += (int64_t)m0 * p.lsa;
-        p.C += (int64_t)m0 * p.ldc;
-        if (p.ca) {
-            p.ca += (int64_t)m0 * p.ldca;
-            p.cb += (int64_t)m0 * p.ldcb;
-        }
-    }
-    // every row group (the first included) spans at most 64 rows, which keeps
-    // its buffer ranges within the host's 64-row 2^31-byte bound
-    p.M = min(BSN_MAX_M, p.M - m0);
-    return p;
-}
-
-template <bool GN1, int MT, int NT>
-__global__ __launch_bounds__(64 * BSN_WAVES) void blockscale_narrow_kernel(const BlockScaleParams pb) {
-    const BlockScaleParams p = bs_row_slice(pb);
-    constexpr int DEPTH = MT * NT == 1 ? 6 : 4;
-    __shared__ v4f red[BSN_WAVES][NT][MT][64];
+template <bool GN1, int NT>
+__global__ __launch_bounds__(64 * BSN_WAVES) void blockscale_narrow_kernel(const BlockScaleParams p) {
+    constexpr int DEPTH = NT == 1 ? 6 : 4;
+    __shared__ v4f red[BSN_WAVES][NT][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, q = lane >> 4;
@@ -222,12 +203,8 @@ __global__ __launch_bounds__(64 * BSN_WAVES) void blockscale_narrow_kernel(const
     // scales: rows of sa past M and groups past S read zero
     const auto rsa = make_rsrc(p.sa, (uint32_t)(((int64_t)(p.M - 1) * p.lsa + S) * 4));
     const auto rsb = make_rsrc(p.sb, (uint32_t)(((int64_t)(S - 1) * p.lsb + (GN1 ? p.N : (p.N + 127) / 128)) * 4));
-    uint32_t a_off[MT], sa_row[MT];
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        a_off[t] = (uint32_t)((t * 16 + r) * p.lda + 16 * q);
-        sa_row[t] = t * 16 + r < p.M ? (uint32_t)((t * 16 + r) * p.lsa) * 4 : OOB;
-    }
+    const uint32_t a_off = (uint32_t)(r * p.lda + 16 * q);
+    const uint32_t sa_row = r < p.M ? (uint32_t)(r * p.lsa) * 4 : OOB;
     uint32_t b_off[NT], sb_col[NT];
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
@@ -235,7 +212,7 @@ __global__ __launch_bounds__(64 * BSN_WAVES) void blockscale_narrow_kernel(const
         sb_col[i] = (uint32_t)(GN1 ? n0 + 16 * i + 4 * q : (n0 + 16 * i) / 128) * 4;
     }
 
-    auto load = [&](int s, BsNarrowFrag<GN1, MT, NT>& f) {
+    auto load = [&](int s, BsNarrowFrag<GN1, NT>& f) {
         const uint32_t kill = s < s1 ? 0u : OOB;
         const uint32_t kb = (uint32_t)s * 128 | kill;
 #pragma unroll
@@ -243,13 +220,9 @@ __global__ __launch_bounds__(64 * BSN_WAVES) void blockscale_narrow_kernel(const
             f.b0[i] = __builtin_amdgcn_raw_buffer_load_b128(rb, b_off[i] + kb, 0, 0);
             f.b1[i] = __builtin_amdgcn_raw_buffer_load_b128(rb, b_off[i] + kb + 64, 0, 0);
         }
-#pragma unroll
-        for (int t = 0; t < MT; ++t) {
-            f.a0[t] = __builtin_amdgcn_raw_buffer_load_b128(ra, a_off[t] + kb, 0, 0);
-            f.a1[t] = __builtin_amdgcn_raw_buffer_load_b128(ra, a_off[t] + kb + 64, 0, 0);
-            f.sa[t] = __builtin_bit_cast(float,
-                                         __builtin_amdgcn_raw_buffer_load_b32(rsa, (sa_row[t] + 4 * (uint32_t)s) | kill, 0, 0));
-        }
+        f.a0 = __builtin_amdgcn_raw_buffer_load_b128(ra, a_off + kb, 0, 0);
+        f.a1 = __builtin_amdgcn_raw_buffer_load_b128(ra, a_off + kb + 64, 0, 0);
+        f.sa = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsa, (sa_row + 4 * (uint32_t)s) | kill, 0, 0));
         const uint32_t srow = ((uint32_t)s * (uint32_t)p.lsb * 4) | kill;
 #pragma unroll
         for (int i = 0; i < NT; ++i)
@@ -257,28 +230,23 @@ __global__ __launch_bounds__(64 * BSN_WAVES) void blockscale_narrow_kernel(const
             for (int e = 0; e < (GN1 ? 4 : 1); ++e)
                 f.sb[i][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsb, srow + sb_col[i] + 4 * e, 0, 0));
     };
-    v4f acc[NT][MT];
+    v4f acc[NT];
 #pragma unroll
-    for (int i = 0; i < NT; ++i)
+    for (int i = 0; i < NT; ++i) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
+    auto mma = [&](const BsNarrowFrag<GN1, NT>& f) {
+        const v8i b = v8i{f.a0[0], f.a0[1], f.a0[2], f.a0[3], f.a1[0], f.a1[1], f.a1[2], f.a1[3]};
 #pragma unroll
-        for (int t = 0; t < MT; ++t) acc[i][t] = v4f{0.f, 0.f, 0.f, 0.f};
-    auto mma = [&](const BsNarrowFrag<GN1, MT, NT>& f) {
+        for (int i = 0; i < NT; ++i) {
+            const v8i a = v8i{f.b0[i][0], f.b0[i][1], f.b0[i][2], f.b0[i][3],
+                              f.b1[i][0], f.b1[i][1], f.b1[i][2], f.b1[i][3]};
+            const v4f P =
+                __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 127, 0, 127);
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
-            const v8i b = v8i{f.a0[t][0], f.a0[t][1], f.a0[t][2], f.a0[t][3], f.a1[t][0], f.a1[t][1], f.a1[t][2], f.a1[t][3]};
-#pragma unroll
-            for (int i = 0; i < NT; ++i) {
-                const v8i a = v8i{f.b0[i][0], f.b0[i][1], f.b0[i][2], f.b0[i][3],
-                                  f.b1[i][0], f.b1[i][1], f.b1[i][2], f.b1[i][3]};
-                const v4f P =
-                    __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 127, 0, 127);
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    acc[i][t][e] = __builtin_fmaf(P[e], f.sa[t] * f.sb[i][GN1 ? e : 0], acc[i][t][e]);
-            }
+            for (int e = 0; e < 4; ++e)
+                acc[i][e] = __builtin_fmaf(P[e], f.sa * f.sb[i][GN1 ? e : 0], acc[i][e]);
         }
     };
-    BsNarrowFrag<GN1, MT, NT> f[DEPTH];
+    BsNarrowFrag<GN1, NT> f[DEPTH];
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) load(s0 + d, f[d]);
     for (int s = s0; s < s1; s += DEPTH) {
@@ -289,20 +257,16 @@ __global__ __launch_bounds__(64 * BSN_WAVES) void blockscale_narrow_kernel(const
         }
     }
 #pragma unroll
-    for (int i = 0; i < NT; ++i)
-#pragma unroll
-        for (int t = 0; t < MT; ++t) red[wave][i][t][lane] = acc[i][t];
+    for (int i = 0; i < NT; ++i) red[wave][i][lane] = acc[i];
     __syncthreads();
     if (wave != 0) return;
 #pragma unroll
-    for (int i = 0; i < NT; ++i)
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        const int n = n0 + 16 * i + 4 * q, m = t * 16 + r;
+    for (int i = 0; i < NT; ++i) {
+        const int n = n0 + 16 * i + 4 * q, m = r;
         if (n >= p.N || m >= p.M) continue;  // N % 4 == 0: n .. n+3 all in or all out
-        v4f v = red[0][i][t][lane];
+        v4f v = red[0][i][lane];
 #pragma unroll
-        for (int w = 1; w < BSN_WAVES; ++w) v += red[w][i][t][lane];
+        for (int w = 1; w < BSN_WAVES; ++w) v += red[w][i][lane];
         if (p.ca) {
             const uint2 x = *reinterpret_cast<const uint2*>(p.ca + (int64_t)m * p.ldca + n);
             const uint2 y = *reinterpret_cast<const uint2*>(p.cb + (int64_t)m * p.ldcb + n);
@@ -315,27 +279,118 @@ __global__ __launch_bounds__(64 * BSN_WAVES) void blockscale_narrow_kernel(const
     }
 }
 
-// M <= 64 in MT = 1, 2 or 4 row tiles, with 16-column (NT = 1) or 32-column
-// (NT = 2, when N/16 workgroups exceed the CUs) slices; larger M in row groups
-// of 64 (grid.y), each streaming the weights again. 32 weight rows and 64
-// activation rows must span less than 2 GiB (32-bit buffer offsets).
-template <bool GN1, int MT>
-static int launch_blockscale_narrow_mt(const BlockScaleParams& p, hipStream_t stream) {
+// 16-column (NT = 1) or 32-column (NT = 2, when N/16 workgroups exceed the
+// CUs) slices.
+template <bool GN1>
+static int launch_blockscale_narrow(const BlockScaleParams& p, hipStream_t stream) {
     const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
     const int64_t wgs16 = (p.N + 15) / 16;
-    const unsigned row_groups = (unsigned)((p.M + BSN_MAX_M - 1) / BSN_MAX_M);
     if (wgs16 > ncu)
-        blockscale_narrow_kernel<GN1, MT, 2><<<dim3((unsigned)((p.N + 31) / 32), row_groups), 64 * BSN_WAVES, 0, stream>>>(p);
+        blockscale_narrow_kernel<GN1, 2><<<dim3((unsigned)((p.N + 31) / 32)), 64 * BSN_WAVES, 0, stream>>>(p);
     else
-        blockscale_narrow_kernel<GN1, MT, 1><<<dim3((unsigned)wgs16, row_groups), 64 * BSN_WAVES, 0, stream>>>(p);
+        blockscale_narrow_kernel<GN1, 1><<<dim3((unsigned)wgs16), 64 * BSN_WAVES, 0, stream>>>(p);
     return hkq_launch_status();
 }
 
-template <bool GN1>
-static int launch_blockscale_narrow(const BlockScaleParams& p, hipStream_t stream) {
-    if (p.M <= 16) return launch_blockscale_narrow_mt<GN1, 1>(p, stream);
-    if (p.M <= 32) return launch_blockscale_narrow_mt<GN1, 2>(p, stream);
-    return launch_blockscale_narrow_mt<GN1, 4>(p, stream);
+// ---------------------------------------------------------------------------
+// Small tiles (gemm_kgroup.h): 32 x 32 .. 128 x 256, chosen by bs_plan below.
+// Bound by the weights' way from memory where the tiles fill the CUs once
+// (measured on MI355X: with its MFMAs taken out, 24 x 7168 x 18432 runs as
+// long as with them), and from 128 x 64 up by the wave's own chain of LDS
+// reads, MFMAs and promotions (0.32, 0.56 and 0.82 us per K-tile of 128 x 64,
+// 128 x 128 and 128 x 256 against 0.24, 0.41 and 0.55 for the loads alone).
+// Against the 256 x 256 tiles (or, up to 192 rows, the 16-column streaming
+// kernel in groups of 64 rows) that served these shapes before: 24x7168x18432
+// 46.0 -> 29 us, 64x2112x7168 26.6 -> 8.7, 500x7168x2048 25.3 -> 13.7,
+// 256x7168x18432 299 -> 73, 1024x7168x18432 276 -> 152.
+template <class Cfg, bool GN1>
+__global__ __launch_bounds__(Cfg::THREADS, 1) void blockscale_tile_kernel(const BlockScaleParams p) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
+    HKQ_LDS uint8_t* smem = (HKQ_LDS uint8_t*)smem_raw;
+    constexpr int BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TMO = Cfg::TMO;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wg = wave % Cfg::GW, kg = wave / Cfg::GW;
+    int tm, tn;
+    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, p.group_m, tm, tn);
+    const int m0 = tm * BM, n0 = tn * BN;
+    const int rows_a = min(p.M - m0, BM), rows_b = min(p.N - n0, BN);
+    const int S = p.K / 128;
+
+    KgSrc<Cfg> src;
+    src.a = buffer_desc(p.A + (int64_t)m0 * p.lda, clamp_bytes((int64_t)rows_a * p.lda));
+    src.b = buffer_desc(p.B + (int64_t)n0 * p.ldb, clamp_bytes((int64_t)rows_b * p.ldb));
+    src.as = buffer_desc(p.sa + (int64_t)m0 * p.lsa, clamp_bytes(((int64_t)(rows_a - 1) * p.lsa + S) * 4));
+    src.bs = buffer_desc(p.sb, clamp_bytes(((int64_t)(S - 1) * p.lsb + (GN1 ? p.N : (p.N + 127) / 128)) * 4));
+    src.bs_step = (uint32_t)p.lsb * 4u;
+    src.sc_shift = 0;
+    src.KT = S;
+#pragma unroll
+    for (int i = 0; i < Cfg::SWP; ++i) {
+        const int r = kg_row<Cfg>(i, wg, lane);
+        src.a_off[i] = (uint32_t)(r * p.lda) + kg_chunk<Cfg>(r, lane);
+        src.b_off[i] = (uint32_t)(r * p.ldb) + kg_chunk<Cfg>(r, lane);
+    }
+    src.a_step = (uint32_t)(8 * Cfg::GW * Cfg::SWP * p.lda);
+    src.b_step = (uint32_t)(8 * Cfg::GW * Cfg::SWP * p.ldb);
+    // scale pieces: 64 rows of sa each, then (one scale per 128 columns) the
+    // n-tiles' column scales; n-tiles past N repeat the last one
+#pragma unroll
+    for (int i = 0; i < Cfg::PW; ++i) {
+        const int q = i * Cfg::GW + wg;
+        const int r = kg_piece_row<Cfg>(q, lane);
+        src.s_off[i] = q < Cfg::PA ? (r < rows_a ? (uint32_t)(r * p.lsa) * 4u : OOB)
+                                   : (uint32_t)(min(n0 + (lane >> 2) * 32, p.N - 1) / 128) * 4u + (uint32_t)(lane & 3) * src.bs_step;
+    }
+#pragma unroll
+    for (int i = 0; i < Cfg::LC; ++i) {
+        const int c = ((i * Cfg::GW + wg) % Cfg::PC) * 64 + lane;
+        src.c_off[i] = c < rows_b ? (uint32_t)(n0 + c) * 4u : OOB;
+    }
+
+    v16f acc[TN][TMO];
+    kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
+    if (!Cfg::SPREAD && kg != 0) return;
+
+    const int mw = m0 + (wg / Cfg::WN * Cfg::TM + (Cfg::SPREAD ? kg * TMO : 0)) * 32, nw = n0 + wg % Cfg::WN * TN * 32;
+    auto one = [](int) { return 1.0f; };
+    auto ones = [](int, int) { return make_float4(1.f, 1.f, 1.f, 1.f); };
+    const int ep = Cfg::SPREAD ? wave : wg;
+    if (p.ca) {
+        MulAddElem<TMO> e;
+        e.ca = p.ca;
+        e.cb = p.cb;
+        e.ldca = p.ldca;
+        e.ldcb = p.ldcb;
+        e.M = p.M;
+        e.N = p.N;
+        e.mw = mw;
+        e.nw = nw;
+        e.lane = lane;
+        store_tile_bf16<TMO, TN>(acc, smem, ep, lane, p.C, p.ldc, p.M, p.N, mw, nw, p.c16 != 0, one, ones, NoBias{}, e);
+    } else {
+        store_tile_bf16<TMO, TN>(acc, smem, ep, lane, p.C, p.ldc, p.M, p.N, mw, nw, p.c16 != 0, one, ones, NoBias{});
+    }
+}
+
+template <class Cfg, bool GN1>
+static int launch_blockscale_tile(BlockScaleParams& p, hipStream_t stream) {
+    auto kern = blockscale_tile_kernel<Cfg, GN1>;
+    static bool attr_set = false;
+    if (!attr_set) {
+        hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS);
+        if (e != hipSuccess) {
+            set_error("hipFuncSetAttribute(MaxDynamicSharedMemorySize=%d) failed: %s", Cfg::LDS, hipGetErrorString(e));
+            return (int)e;
+        }
+        attr_set = true;
+    }
+    p.tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM;
+    p.tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
+    if (p.group_m <= 0) p.group_m = 8;
+    p.c16 = (p.ldc % 8 == 0) && (reinterpret_cast<uintptr_t>(p.C) % 16 == 0);
+    kern<<<dim3((unsigned)(p.tiles_m * p.tiles_n)), Cfg::THREADS, Cfg::LDS, stream>>>(p);
+    return hkq_launch_status();
 }
 
 template <bool GN1, int BN>
@@ -361,18 +416,56 @@ static int launch_blockscale_bn(BlockScaleParams& p, hipStream_t stream) {
     return hkq_launch_status();
 }
 
-// 224-column tiles when they take fewer SIMD-steps: rounds of tiles over the
-// CUs times the n-tiles a SIMD computes per tile (8 for 256 columns, 7 for
-// 224). HKQ_BLOCKSCALE_W224=0 (read at each call) keeps the 256-column tiles.
-template <bool GN1>
-static int launch_blockscale(BlockScaleParams& p, hipStream_t stream) {
+// Tile size of a block-scale GEMM: the least estimated time,
+//   rounds of tiles over the CUs * (K-tiles * us per K-tile + 2.3 us) + 2.3 us,
+// with the us per K-tile measured on MI355X as the mean of operands that lie
+// in the last-level cache (N, K = 2112, 7168 and 7168, 2048: 0.05, 0.12, 0.17,
+// 0.32, 0.56, 0.82, 1.3 in the order below) and in HBM (7168, 18432: 0.15,
+// 0.26, 0.33, 0.5, 0.67, 1.03, 1.9). It picks the fastest size at 24 .. 2048
+// rows of those shapes and of 24576, 1536 (the runner-up within 6% in all but
+// the clear cases). 224-column tiles of 256 rows do 7/8 of a 256-column
+// tile's work (they fill CUs that 256 columns leave idle: 2048 x 7168 is 224
+// tiles of 256 columns, 256 of 224). Column scales per column (GN 1) need 64
+// columns for a whole load and leave 128 x 256 no registers.
+// HKQ_BLOCKSCALE_W224=0 (read at each call) keeps 256-column tiles.
+enum BsTile { BST_32x32, BST_32x64, BST_64x64, BST_128x64, BST_128x128, BST_128x256, BST_256x256, BST_256x224, BST_COUNT };
+static int bs_plan(int64_t M, int64_t N, int64_t K, bool gn1, bool small_ok) {
+    static const struct { int bm, bn; float us; bool gn1; } T[BST_COUNT] = {
+        {32, 32, 0.10f, false},  {32, 64, 0.18f, true},    {64, 64, 0.24f, true},   {128, 64, 0.38f, true},
+        {128, 128, 0.60f, true}, {128, 256, 0.97f, false}, {256, 256, 1.5f, true}, {256, 224, 1.3125f, true}};
     const char* w224_env = std::getenv("HKQ_BLOCKSCALE_W224");
     const bool w224_on = !(w224_env && w224_env[0] == '0');
     const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
-    const int64_t tm = (p.M + BS_BM - 1) / BS_BM;
-    const int64_t r256 = (tm * ((p.N + BS_BN - 1) / BS_BN) + ncu - 1) / ncu;
-    const int64_t r224 = (tm * ((p.N + BS_BN - 33) / (BS_BN - 32)) + ncu - 1) / ncu;
-    if (w224_on && 7 * r224 < 8 * r256) return launch_blockscale_bn<GN1, BS_BN - 32>(p, stream);
+    int best = BST_256x256;
+    float best_us = 0.f;
+    for (int t = BST_COUNT - 1; t >= 0; --t) {
+        if ((t < BST_256x256 && (!small_ok || (gn1 && !T[t].gn1))) || (t == BST_256x224 && !w224_on)) continue;
+        const int64_t tiles = ((M + T[t].bm - 1) / T[t].bm) * ((N + T[t].bn - 1) / T[t].bn);
+        const float us = (float)((tiles + ncu - 1) / ncu) * ((float)(K / 128) * T[t].us + 2.3f);
+        if (best_us == 0.f || us < best_us) {
+            best = t;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
+template <bool GN1>
+static int launch_blockscale(BlockScaleParams& p, bool small_ok, hipStream_t stream) {
+    constexpr int B = MODE_BLOCKSCALE;
+    switch (bs_plan(p.M, p.N, p.K, GN1, small_ok)) {
+        case BST_32x32:
+            if constexpr (!GN1) return launch_blockscale_tile<KgCfg<B, 1, 1, 4, 1, 1, 4>, false>(p, stream);
+            break;
+        case BST_32x64: return launch_blockscale_tile<KgCfg<B, 1, 1, 4, 1, 2, 3, GN1>, GN1>(p, stream);
+        case BST_64x64: return launch_blockscale_tile<KgCfg<B, 1, 1, 4, 2, 2, 2, GN1>, GN1>(p, stream);
+        case BST_128x64: return launch_blockscale_tile<KgCfg<B, 4, 1, 2, 1, 2, 3, GN1>, GN1>(p, stream);
+        case BST_128x128: return launch_blockscale_tile<KgCfg<B, 4, 2, 1, 1, 2, 4, GN1>, GN1>(p, stream);
+        case BST_128x256:
+            if constexpr (!GN1) return launch_blockscale_tile<KgCfg<B, 2, 4, 1, 2, 2, 3>, false>(p, stream);
+            break;
+        case BST_256x224: return launch_blockscale_bn<GN1, BS_BN - 32>(p, stream);
+    }
     return launch_blockscale_bn<GN1, BS_BN>(p, stream);
 }
 
@@ -434,14 +527,15 @@ static int blockscale_call(const void* A, const void* B, const float* sa, const 
     p.cb = static_cast<const uint16_t*>(cb);
     p.ldca = ldca; p.ldcb = ldcb;
     if (M == 0 || N == 0) return 0;
-    // M <= 64; up to 192 rows (row groups of 64) while the 256 x 256 tiles
-    // would give fewer than a quarter of the CUs work (at N = 7168, 28 tiles:
-    // 16x7168x18432 took 321 us tiled, 31 us streamed; 128x7168x18432 325 vs
-    // 140 us; at 256 rows the tiles win for K <= 7168)
-    const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
-    const bool few_tiles = M <= 192 && ((N + 255) / 256) * 4 < ncu;
-    if ((M <= BSN_MAX_M || few_tiles) && 32 * ldb < (1ll << 31) && BSN_MAX_M * lda < (1ll << 31) &&
-        (int64_t)M * lsa < (1ll << 28) && (K / 128) * lsb < (1ll << 28))
+    // M <= 16 with at most 32 K groups streams the weights through registers
+    // (16 x 7168 x 2048: 6.1 us against 5.8 on small tiles, 1 x 24576 x 1536
+    // 10.3 against 11; with long K the tiles' deeper rings win: 8 x 7168 x
+    // 18432 29.2 against 25.7, 8 x 2112 x 7168 9.5 against 7.4). The streaming
+    // kernel's 32 weight rows and 16 activation rows, the small tiles' 256
+    // and 128, and the scales must span less than 2 GiB (32-bit offsets).
+    const bool scales32 = 128 * lsa < (1ll << 28) && (K / 128) * lsb < (1ll << 28);
+    if (M <= BSN_MAX_M && K / 128 <= 32 && 32 * ldb < (1ll << 31) && BSN_MAX_M * lda < (1ll << 31) && scales32)
         return group_n == 1 ? launch_blockscale_narrow<true>(p, stream) : launch_blockscale_narrow<false>(p, stream);
-    return group_n == 1 ? launch_blockscale<true>(p, stream) : launch_blockscale<false>(p, stream);
+    const bool small_ok = 256 * ldb < (1ll << 31) && 128 * lda < (1ll << 31) && scales32;
+    return group_n == 1 ? launch_blockscale<true>(p, small_ok, stream) : launch_blockscale<false>(p, small_ok, stream);
 }

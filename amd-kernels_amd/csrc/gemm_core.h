@@ -221,7 +221,6 @@ __device__ __forceinline__ HKQ_LDS uint8_t* stage_tile_bf16(v16f (&acc)[TN][TM],
                                                             int lane, RowScale row_scale, ColScale4 col_scale4,
                                                             ColBias4 col_bias4, Elem elem = Elem{}) {
     constexpr int PITCH = TN * 32 * 2 + 16;
-    static_assert((TN * 32 * 2) % 128 == 0, "rows are whole 128-byte segments");
     HKQ_LDS uint8_t* ep = smem + wave * (TM * 32) * PITCH;
     const int khalf = lane >> 5;
     float rs[TM];

@@ -373,6 +373,33 @@ def test_gemm_blockscale_tile_widths(orc, monkeypatch, M, N, K, group_n):
     assert_gemm_close(C224, orc.gemm_blockscale_ref_f32(A, B, sa, sb, 128, group_n), f"blockscale {M}x{N}x{K}")
 
 
+# The small tiles, each at ragged M and N with an odd count of K groups (uneven
+# splits over the wave groups, a last scale block of 1 or 3 columns): on 256
+# CUs 32x32 / 32x64 (GN 1), 64x64, 128x64, 128x128, 128x256 / 256x224 (GN 1);
+# then 256-row tiles with a ragged last tile. Row strides of A, sa, sb and C
+# hold more than a row; the padding of C stays untouched and that of sa is NaN
+# (a scale read across its row's end would show). Tolerance: that of every
+# GEMM here.
+@pytest.mark.parametrize("group_n", [128, 1])
+@pytest.mark.parametrize("M,N,K", [(17, 300, 640), (40, 1000, 128), (97, 4100, 384), (161, 7172, 384), (333, 7172, 640),
+                                   (1000, 7172, 384), (1000, 8196, 896)])
+def test_gemm_blockscale_small_tiles(orc, M, N, K, group_n):
+    require_gpu()
+    A, B, sa, sb = blockscale_inputs(orc, M, N, K, M + N + K + 5, group_n)
+    Ap = torch.full((M, K + 64), 0x7F, dtype=torch.uint8, device="cuda")
+    Ap[:, :K] = dev_u8(A)
+    sap = torch.full((M, K // 128 + 3), float("nan"), dtype=torch.float32, device="cuda")
+    sap[:, :K // 128] = dev_f32(sa)
+    sbp = torch.full((K // 128, sb.shape[1] + 5), float("nan"), dtype=torch.float32, device="cuda")
+    sbp[:, :sb.shape[1]] = dev_f32(sb)
+    Cp = torch.full((M, N + 4), 7.0, dtype=torch.bfloat16, device="cuda")
+    C = hkq.gemm_blockscale(Ap[:, :K], dev_u8(B), sap[:, :K // 128], sbp[:, :sb.shape[1]], Cp[:, :N], group_n=group_n)
+    torch.cuda.synchronize()
+    assert bool((Cp[:, N:] == 7.0).all()), "stores past N reached the row padding"
+    assert_gemm_close(host_bf16_f32(C), orc.gemm_blockscale_ref_f32(A, B, sa, sb, 128, group_n),
+                      f"blockscale small tiles {M}x{N}x{K} gn{group_n}")
+
+
 def test_gemm_blockscale_uniform_scales_reduce_to_a8w8(orc):
     """Scales constant over K groups: the block-scale GEMM equals the A8W8 GEMM
     with the same per-row / per-column factors."""
