@@ -19,6 +19,7 @@
 
 #include <cstdlib>
 
+#include "gemm_kgroup.h"
 #include "gemm_stream.h"
 #include "hkq_host.h"
 
@@ -39,7 +40,7 @@ struct DenseParams {
     int n_whole;          // workgroups [0, n_whole) compute whole tiles 0 .. n_whole-1
     int n_split;          // tiles n_whole .. n_whole+n_split-1 are computed as two M halves
     int c16;              // rows of C are 16-byte aligned (ldc % 8 == 0, C 16-byte aligned)
-    int splits;           // K splits of the split/skinny path (1: none)
+    int splits;           // K splits of the split path (1: none)
     int kt_split;         // K-tiles per split
     float* ws;            // split partials (splits > 1)
     uint64_t* split_cnt;  // splits > 1: per tile, the arrival counter of its splits
@@ -81,9 +82,6 @@ __device__ __forceinline__ float4 bias4(const DenseParams& p, int n) {
 // else 64 bytes in a 4-stage ring.
 constexpr int DENSE_WAVES_M = 2, DENSE_WAVES_N = 2, DENSE_TM = 4, DENSE_TN = 4;
 constexpr int DENSE_BM = DENSE_WAVES_M * DENSE_TM * 32, DENSE_BN = DENSE_WAVES_N * DENSE_TN * 32;
-// Skinny geometry (M <= 64): one row of (TM*32) x 256 tiles, 4 waves of
-// (TM*32) x 64 side by side.
-constexpr int SKINNY_WAVES_N = 4, SKINNY_TN = 2, SKINNY_BN = SKINNY_WAVES_N * SKINNY_TN * 32;
 template <int KTB>
 constexpr int dense_ns() { return KTB == 128 ? 2 : 4; }
 
@@ -373,11 +371,9 @@ __global__ __launch_bounds__(64 * DENSE_WAVES_M * DENSE_WAVES_N, 1) void dense_s
 }
 
 // ---------------------------------------------------------------------------
-// Smaller tiles and split K. A grid of 256 x 256 tiles that would fill at most
-// half of the CUs runs on 128 x 128 tiles (4 waves of 64 x 64; FP8 with
-// M <= 128 and K <= 16384: 128 x 64 tiles, 4 waves of 32 x 64), and M <= 64
-// on one row of (32 or 64) x 256 tiles (4 waves side by side); if that still
-// fills at most half of the CUs, K is split as well: workgroup u computes tile
+// 128 x 128 tiles (4 waves of 64 x 64; FP8 with M <= 128 and K <= 16384: 128 x
+// 64 tiles, 4 waves of 32 x 64) with two workgroups per CU or with K split over
+// the workgroups of one launch. A split's workgroup u computes tile
 // u % tiles over K-tiles [s * kt_split, (s+1) * kt_split), s = u / tiles, and
 // writes its fp32 sums to the workspace in register order (per wave, float4 q
 // of lane l at (q * 64 + l) * 16 bytes: every store is a contiguous 1 KB).
@@ -573,152 +569,88 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void dense_tile_kernel(const De
 }
 
 // ---------------------------------------------------------------------------
-// Narrow M (M <= 32, FP8 and FP4): a streaming path on the 16x16x128 MFMA.
-// Workgroup u owns the 16*NT columns [16*NT*u, 16*NT*(u+1)) of C for all M
-// rows; its 4 waves split K (wave w takes the 128-value K-steps
+// Narrow M (M <= 16 and short K, where 16-column workgroups pay): a streaming
+// path on the 16x16x128 MFMA. Workgroup u owns the 16 columns [16u, 16u + 16) of C for all
+// M rows; its 4 waves split K (wave w takes the 128-value K-steps
 // [w*S/4, (w+1)*S/4) of S) and load their operand fragments from memory
-// straight into registers, DEPTH steps ahead. The waves' sums meet in LDS, and
-// wave 0 adds them in wave order, applies the scales and writes C. Each weight
-// byte is read once, by one workgroup, in a single launch (no split-K
-// partials, no second kernel). NT > 1 reuses each activation fragment for NT
-// weight tiles when N gives more workgroups than CUs.
+// straight into registers, all steps at once. The waves' sums meet in LDS, and
+// wave 0 adds them in wave order, applies the scales and writes C.
 //
 // Fragment layout of the 16x16x128 MFMA (verified on gfx950): lane l supplies
-// row l % 16 and the 32 K-values [32*(l/16), 32*(l/16) + 32) of the 128-deep
-// slice (FP8: 32 bytes; FP4: 16 bytes in the low 4 VGPRs, scaled per lane by
-// its 32-value block's e8m0); lane l, register i of the result holds
-// D[4*(l/16) + i][l % 16]. The MFMA A operand is the weight rows (n), B the
-// activation rows (m): a lane holds 4 consecutive n of one m. An FP8 sum over
-// K does not depend on which lane supplies which K-value as long as both
-// operands agree, so an FP8 lane takes bytes [16q, 16q+16) and [64+16q,
-// 64+16q+16) of the step (q = l/16): each 16-byte load covers 64 contiguous
-// bytes of 16 rows.
-constexpr int NARROW_WAVES = 4, NARROW_MAX_M = 32;
+// row l % 16 and 32 K-values of the 128-deep slice; lane l, register i of the
+// result holds D[4*(l/16) + i][l % 16]. The MFMA A operand is the weight rows
+// (n), B the activation rows (m): a lane holds 4 consecutive n of one m. A sum
+// over K does not depend on which lane supplies which K-value as long as both
+// operands agree, so a lane takes bytes [16q, 16q+16) and [64+16q, 64+16q+16)
+// of the step (q = l/16): each 16-byte load covers 64 contiguous bytes of 16
+// rows.
+//
+// Bound by latency: one memory round trip for everything, then the sums'
+// exchange. All of a wave's steps (at most 8) are in flight at once, the
+// epilogue's scales before them, and no look-ahead load is issued past them:
+// 4x4096x4096 5.75 -> 4.9 us against a loop of 8-step rings whose look-ahead
+// read nothing and whose scales were fetched after the sums.
+constexpr int NARROW_WAVES = 4, NARROW_MAX_M = 16, NARROW_MAX_STEPS = 32;
 
-template <int MODE, int MT, int NT>
 struct NarrowFrag {
-    v4i b0[NT], b1[NT];  // weight rows (b1: FP8 only)
-    v4i a0[MT], a1[MT];  // activation rows (a1: FP8 only)
-    uint32_t sb[NT], sa[MT];  // FP4: e8m0 scales of the step's 4 blocks (byte q is the lane's)
+    v4i b0, b1, a0, a1;  // weight row, activation row
 };
 
-// K-steps of loads in flight per wave (measured on MI355X: FP8 with two
-// column tiles per workgroup 8 rather than 6, 1x6144x4096 8.33 -> 7.94 us;
-// deeper rings for one or four column tiles, and for FP4, were slower)
-template <int MODE, int MT, int NT>
-constexpr int narrow_depth() { return NT >= 4 ? 4 : NT == 2 ? (MODE == MODE_MXFP4 ? 6 : 8) : 8; }
-
-template <int MODE, int MT, int NT>
 __global__ __launch_bounds__(64 * NARROW_WAVES) void narrow_gemm_kernel(const DenseParams pb) {
-    constexpr bool FP4 = MODE == MODE_MXFP4;
-    constexpr int SB = FP4 ? 64 : 128;  // bytes of a row per 128-value K-step
-    constexpr int DEPTH = narrow_depth<MODE, MT, NT>();
-    __shared__ v4f red[NARROW_WAVES][NT][MT][64];
+    constexpr int DEPTH = NARROW_MAX_STEPS / NARROW_WAVES;  // K-steps of a wave at most, all in flight together
+    __shared__ v4f red[NARROW_WAVES][64];
     const DenseParams p = batch_slice(pb);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, q = lane >> 4;
-    const int n0 = blockIdx.x * 16 * NT;
-    const int S = p.kbytes / SB;
+    const int n0 = blockIdx.x * 16;
+    const int S = p.kbytes / 128;
     const int s0 = wave * S / NARROW_WAVES, s1 = (wave + 1) * S / NARROW_WAVES;
-    const int rows_b = min(16 * NT, p.N - n0);
+    const int rows_b = min(16, p.N - n0);
     const auto rb = make_rsrc(p.B + (int64_t)n0 * p.ldb, (uint32_t)(rows_b * p.ldb));
     const auto ra = make_rsrc(p.A, (uint32_t)(p.M * p.lda));
-    const uint8_t* bs = static_cast<const uint8_t*>(p.sb);
-    const auto rsb = make_rsrc(FP4 ? bs + (int64_t)n0 * p.lsb : p.B, FP4 ? (uint32_t)(rows_b * p.lsb) : 0u);
-    const auto rsa = make_rsrc(FP4 ? p.sa : p.A, FP4 ? (uint32_t)(p.M * p.lsa) : 0u);
-    uint32_t b_off[NT], a_off[MT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) b_off[t] = (uint32_t)((t * 16 + r) * p.ldb + 16 * q);
-#pragma unroll
-    for (int t = 0; t < MT; ++t) a_off[t] = (uint32_t)((t * 16 + r) * p.lda + 16 * q);
+    const uint32_t b_off = (uint32_t)(r * p.ldb + 16 * q), a_off = (uint32_t)(r * p.lda + 16 * q);
 
     // Steps at or past s1 read zeros (their MFMAs add nothing): offsets with
     // the OOB bit set are past every buffer's range.
-    auto load = [&](int s, NarrowFrag<MODE, MT, NT>& f) {
-        const uint32_t kb = (uint32_t)s * SB | (s < s1 ? 0u : OOB);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            f.b0[t] = __builtin_amdgcn_raw_buffer_load_b128(rb, b_off[t] + kb, 0, 0);
-            if constexpr (!FP4) f.b1[t] = __builtin_amdgcn_raw_buffer_load_b128(rb, b_off[t] + kb + 64, 0, 0);
-        }
-#pragma unroll
-        for (int t = 0; t < MT; ++t) {
-            f.a0[t] = __builtin_amdgcn_raw_buffer_load_b128(ra, a_off[t] + kb, 0, 0);
-            if constexpr (!FP4) f.a1[t] = __builtin_amdgcn_raw_buffer_load_b128(ra, a_off[t] + kb + 64, 0, 0);
-        }
-        if constexpr (FP4) {
-            const uint32_t ks = 4 * (uint32_t)s | (s < s1 ? 0u : OOB);
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-                f.sb[t] = __builtin_amdgcn_raw_buffer_load_b32(rsb, (uint32_t)((t * 16 + r) * p.lsb) + ks, 0, 0);
-#pragma unroll
-            for (int t = 0; t < MT; ++t)
-                f.sa[t] = __builtin_amdgcn_raw_buffer_load_b32(rsa, (uint32_t)((t * 16 + r) * p.lsa) + ks, 0, 0);
-        }
+    auto load = [&](int s, NarrowFrag& f) {
+        const uint32_t kb = (uint32_t)s * 128 | (s < s1 ? 0u : OOB);
+        f.b0 = __builtin_amdgcn_raw_buffer_load_b128(rb, b_off + kb, 0, 0);
+        f.b1 = __builtin_amdgcn_raw_buffer_load_b128(rb, b_off + kb + 64, 0, 0);
+        f.a0 = __builtin_amdgcn_raw_buffer_load_b128(ra, a_off + kb, 0, 0);
+        f.a1 = __builtin_amdgcn_raw_buffer_load_b128(ra, a_off + kb + 64, 0, 0);
     };
-    v4f acc[NT][MT];
-#pragma unroll
-    for (int i = 0; i < NT; ++i)
-#pragma unroll
-        for (int t = 0; t < MT; ++t) acc[i][t] = v4f{0.f, 0.f, 0.f, 0.f};
-    auto mma = [&](const NarrowFrag<MODE, MT, NT>& f) {
-#pragma unroll
-        for (int i = 0; i < NT; ++i)
-#pragma unroll
-            for (int t = 0; t < MT; ++t) {
-                if constexpr (FP4) {
-                    const v8i a = v8i{f.b0[i][0], f.b0[i][1], f.b0[i][2], f.b0[i][3], 0, 0, 0, 0};
-                    const v8i b = v8i{f.a0[t][0], f.a0[t][1], f.a0[t][2], f.a0[t][3], 0, 0, 0, 0};
-                    acc[i][t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                        a, b, acc[i][t], 4, 4, 0, (int)(f.sb[i] >> (8 * q)), 0, (int)(f.sa[t] >> (8 * q)));
-                } else {
-                    const v8i a = v8i{f.b0[i][0], f.b0[i][1], f.b0[i][2], f.b0[i][3],
-                                      f.b1[i][0], f.b1[i][1], f.b1[i][2], f.b1[i][3]};
-                    const v8i b = v8i{f.a0[t][0], f.a0[t][1], f.a0[t][2], f.a0[t][3],
-                                      f.a1[t][0], f.a1[t][1], f.a1[t][2], f.a1[t][3]};
-                    acc[i][t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, acc[i][t], 0, 0, 0, 127, 0, 127);
-                }
-            }
+    v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
+    auto mma = [&](const NarrowFrag& f) {
+        const v8i a = v8i{f.b0[0], f.b0[1], f.b0[2], f.b0[3], f.b1[0], f.b1[1], f.b1[2], f.b1[3]};
+        const v8i b = v8i{f.a0[0], f.a0[1], f.a0[2], f.a0[3], f.a1[0], f.a1[1], f.a1[2], f.a1[3]};
+        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, acc, 0, 0, 0, 127, 0, 127);
     };
-    NarrowFrag<MODE, MT, NT> f[DEPTH];
+    // the epilogue's scales go out before the operands: no memory latency
+    // follows the K loop
+    const int n = n0 + 4 * q, m = r;
+    const bool in = n < p.N && m < p.M;  // N % 4 == 0: n .. n+3 all in or all out
+    float4 cs = make_float4(0.f, 0.f, 0.f, 0.f);
+    float a = 0.f;
+    if (in) {
+        cs = *reinterpret_cast<const float4*>(static_cast<const float*>(p.sb) + n);
+        a = static_cast<const float*>(p.sa)[m];
+    }
+    const float4 c = bias4(p, n);
+    NarrowFrag f[DEPTH];
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) load(s0 + d, f[d]);
-    for (int s = s0; s < s1; s += DEPTH) {
 #pragma unroll
-        for (int d = 0; d < DEPTH; ++d) {
-            mma(f[d]);
-            load(s + d + DEPTH, f[d]);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < NT; ++i)
-#pragma unroll
-        for (int t = 0; t < MT; ++t) red[wave][i][t][lane] = acc[i][t];
+    for (int d = 0; d < DEPTH; ++d) mma(f[d]);
+    red[wave][lane] = acc;
     __syncthreads();
-    if (wave != 0) return;
-    const float* sa = static_cast<const float*>(p.sa);
-    const float* sb = static_cast<const float*>(p.sb);
+    if (wave != 0 || !in) return;
+    v4f v = red[0][lane];
 #pragma unroll
-    for (int i = 0; i < NT; ++i) {
-        const int n = n0 + 16 * i + 4 * q;
-        if (n >= p.N) break;  // N % 4 == 0: n .. n+3 all in or all out
-        float4 cs = make_float4(1.f, 1.f, 1.f, 1.f);
-        if constexpr (MODE == MODE_A8W8) cs = *reinterpret_cast<const float4*>(sb + n);
-        const float4 c = bias4(p, n);
-#pragma unroll
-        for (int t = 0; t < MT; ++t) {
-            const int m = t * 16 + r;
-            if (m >= p.M) break;
-            v4f v = red[0][i][t][lane];
-#pragma unroll
-            for (int w = 1; w < NARROW_WAVES; ++w) v += red[w][i][t][lane];
-            const float a = MODE == MODE_A8W8 ? sa[m] : 1.f;
-            *reinterpret_cast<v2i*>(p.C + (int64_t)m * p.ldc + n) =
-                v2i{(int)pk_bf16(v[0] * a * cs.x + c.x, v[1] * a * cs.y + c.y),
-                    (int)pk_bf16(v[2] * a * cs.z + c.z, v[3] * a * cs.w + c.w)};
-        }
-    }
+    for (int w = 1; w < NARROW_WAVES; ++w) v += red[w][lane];
+    *reinterpret_cast<v2i*>(p.C + (int64_t)m * p.ldc + n) =
+        v2i{(int)pk_bf16(v[0] * a * cs.x + c.x, v[1] * a * cs.y + c.y),
+            (int)pk_bf16(v[2] * a * cs.z + c.z, v[3] * a * cs.w + c.w)};
 }
 
 template <typename K>
@@ -733,39 +665,111 @@ static int set_lds(K kern, int lds, bool& done) {
     return 0;
 }
 
-// Plan of a dense GEMM: the tile geometry, how many K splits, and the
-// workspace the splits need (bytes). The same function answers the workspace
-// query, so a caller's workspace always matches the launch.
+// ---------------------------------------------------------------------------
+// Small tiles with K split over the workgroup's waves (gemm_kgroup.h), chosen
+// by dense_tile_plan below. Bound by the way into LDS: a CU takes 95-100 GB/s
+// from the caches while it computes (125 GB/s when it only loads from L2), so
+// a K-tile of a BM x BN tile costs about its (BM + BN) * 128 bytes at that
+// rate. Measured on MI355X against the (32 or 64) x 256 tiles, split-K
+// 128 x 64 tiles and streaming kernel that served these shapes before: A8W8
+// 48x4096x4096 17.1 -> 6.6 us, 160x4096x4096 15.0 -> 9.9, 64x4096x14336
+// 29.6 -> 13.6, 64x28672x4096 42 -> 26; MXFP4 64x8192x8192 19.9 -> 9.1,
+// 1x8192x8192 11.9 -> 8.0; bf16 64x4096x4096 25.8 -> 9.0, 1x4096x4096
+// 17.1 -> 7.9, 300x4096x4096 22.9 -> 19.1.
+template <class Cfg>
+__global__ __launch_bounds__(Cfg::THREADS, 1) void dense_kgroup_kernel(const DenseParams pb) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
+    HKQ_LDS uint8_t* smem = (HKQ_LDS uint8_t*)smem_raw;
+    constexpr int MODE = Cfg::MODE, BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TMO = Cfg::TMO;
+    const DenseParams p = batch_slice(pb);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wg = wave % Cfg::GW, kg = wave / Cfg::GW;
+    int tm, tn;
+    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, p.group_m, tm, tn);
+    const int m0 = tm * BM, n0 = tn * BN;
+    const int rows_a = min(p.M - m0, BM), rows_b = min(p.N - n0, BN);
+
+    KgSrc<Cfg> src;
+    src.KT = (p.kbytes + 64) / 128;
+    src.half_tail = p.kbytes % 128 != 0;
+    src.a = buffer_desc(p.A + (int64_t)m0 * p.lda, clamp_bytes((int64_t)rows_a * p.lda));
+    src.b = buffer_desc(p.B + (int64_t)n0 * p.ldb, clamp_bytes((int64_t)rows_b * p.ldb));
+#pragma unroll
+    for (int i = 0; i < Cfg::SWP; ++i) {
+        const int r = kg_row<Cfg>(i, wg, lane);
+        src.a_off[i] = (uint32_t)(r * p.lda) + kg_chunk<Cfg>(r, lane);
+        src.b_off[i] = (uint32_t)(r * p.ldb) + kg_chunk<Cfg>(r, lane);
+    }
+    src.a_step = (uint32_t)(8 * Cfg::GW * Cfg::SWP * p.lda);
+    src.b_step = (uint32_t)(8 * Cfg::GW * Cfg::SWP * p.ldb);
+    src.bs_step = 0;
+    src.sc_shift = 0;
+    if constexpr (Cfg::FP4) {
+        src.as = buffer_desc(static_cast<const uint8_t*>(p.sa) + (int64_t)m0 * p.lsa,
+                             clamp_bytes((int64_t)(rows_a - 1) * p.lsa + p.K / 32));
+        src.bs = buffer_desc(static_cast<const uint8_t*>(p.sb) + (int64_t)n0 * p.lsb,
+                             clamp_bytes((int64_t)(rows_b - 1) * p.lsb + p.K / 32));
+#pragma unroll
+        for (int i = 0; i < Cfg::PW; ++i) {
+            const int q = i * Cfg::GW + wg;
+            const int r = kg_piece_row<Cfg>(q < Cfg::PA ? q : q - Cfg::PA, lane);
+            src.s_off[i] = (uint32_t)(r * (q < Cfg::PA ? p.lsa : p.lsb)) + kg_piece_half(lane);
+        }
+    }
+    const int mw = m0 + (wg / Cfg::WN * Cfg::TM + (Cfg::SPREAD ? kg * TMO : 0)) * 32, nw = n0 + wg % Cfg::WN * TN * 32;
+    EpiScales<MODE, TMO, TN> sc;
+    sc.load(p, lane, mw, nw);
+
+    v16f acc[TN][TMO];
+    kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
+    if (!Cfg::SPREAD && kg != 0) return;
+    dense_epilogue_global<MODE, 0, 0, TMO, TN>(p, acc, sc, smem, Cfg::SPREAD ? wave : wg, lane, mw, nw);
+}
+
+template <class Cfg>
+static int launch_dense_kgroup(DenseParams& p, hipStream_t stream) {
+    auto kern = dense_kgroup_kernel<Cfg>;
+    static bool attr_set = false;
+    if (int e = set_lds(kern, Cfg::LDS, attr_set)) return e;
+    p.tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM;
+    p.tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
+    if (p.group_m <= 0) p.group_m = 8;
+    kern<<<dim3((unsigned)(p.tiles_m * p.tiles_n), (unsigned)std::max(1, p.batch)), Cfg::THREADS, Cfg::LDS, stream>>>(p);
+    return hkq_launch_status();
+}
+
+// Split plan of a dense GEMM: the tile geometry, how many K splits, and the
+// workspace the splits need (bytes). It answers the workspace queries for all
+// shapes (GEO_SKINNY's included, which now run without one), so a caller's
+// workspace always covers the launch; dense_tile_plan decides where a split
+// runs.
 enum DenseGeo { GEO_256 = 0, GEO_128 = 1, GEO_SKINNY = 2, GEO_128x64 = 3 };
 struct DensePlan {
     int geo;
-    int skinny_tm;  // GEO_SKINNY: TM = 1 or 2
     int64_t tiles;
     int splits, kt_split;
     size_t ws_bytes;
 };
 
-static DensePlan dense_plan(int mode, int64_t M, int64_t N, int64_t kbytes, bool allow_split, int64_t batch = 1) {
+static DensePlan dense_plan(int mode, int64_t M, int64_t N, int64_t kbytes) {
     DensePlan pl{};
     const int ktb = kbytes % 128 == 0 ? 128 : 64;
     const int64_t KT = kbytes / ktb;
     const int ncu = cu_count() > 0 ? cu_count() : 256;
-    // tiles of the whole launch (all batches)
-    auto ntiles = [&](int64_t bm, int64_t bn) { return batch * ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    auto ntiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     int64_t bm = DENSE_BM, bn = DENSE_BN;
     pl.geo = GEO_256;
     if (ktb == 128 && M <= 64) {
         pl.geo = GEO_SKINNY;
-        pl.skinny_tm = M <= 32 ? 1 : 2;
-        bm = 32 * pl.skinny_tm;
-        bn = SKINNY_BN;
+        bm = M <= 32 ? 32 : 64;
+        bn = 256;
     } else if (ktb == 128 && 2 * ntiles(DENSE_BM, DENSE_BN) <= ncu) {
         pl.geo = GEO_128;
         bm = bn = 128;
         // FP8 with M <= 128 and K <= 16384: 128 x 64 tiles (4 waves of 32 x 64),
         // twice the workgroups for the same K split and a quarter of the
-        // partial sums the last split reads (measured on MI355X: 128x4096x4096
-        // 10.0 us, 128x4096x14336 18.0 us against 24.1 on 128 x 128 tiles)
+        // partial sums the last split reads
         if (mode == MODE_A8W8 && M <= 128 && KT <= 128) {
             pl.geo = GEO_128x64;
             bn = 64;
@@ -776,8 +780,7 @@ static DensePlan dense_plan(int mode, int64_t M, int64_t N, int64_t kbytes, bool
     pl.kt_split = (int)KT;
     // split K when the tiles fill at most half of the CUs, keeping at least 4
     // K-tiles per split
-    if (allow_split && pl.geo != GEO_256 && pl.tiles > 0 && 2 * pl.tiles <= ncu && pl.tiles <= SPLIT_MAX_TILES &&
-        KT >= 8) {
+    if (pl.geo != GEO_256 && pl.tiles > 0 && 2 * pl.tiles <= ncu && pl.tiles <= SPLIT_MAX_TILES && KT >= 8) {
         int64_t s = (ncu + pl.tiles - 1) / pl.tiles;
         s = std::min<int64_t>(s, KT / 4);
         if (s > 1) {
@@ -791,8 +794,58 @@ static DensePlan dense_plan(int mode, int64_t M, int64_t N, int64_t kbytes, bool
     return pl;
 }
 
+// Tile size of a dense GEMM: the least estimated time
+// over the sizes below,
+//   rounds of tiles over the CUs * (K-tiles * us + e) + 2.3 us,
+// us and e per size and operand format fitted to MI355X times at 24 .. 2500
+// rows of the benchmark's weights and of 1500 x 1024 (the pick is the fastest
+// size or within 6% of it at all of the 230 shapes). Split K (A8W8 and bf16,
+// a workspace given): one round of its own plan, the partial sums' exchange in
+// the constant. It is still the better one where half of the CUs' worth of
+// tiles meets a long K: 400x4096x14336 31.7 us against 34.7, 128x4096x14336
+// 17.7 against 18.4, bf16 256x2048x14336 29.8 against 32.8.
+enum DenseTile {
+    DT_32x32, DT_32x64, DT_32x128, DT_64x64, DT_128x64, DT_128x128, DT_128x256,
+    DT_128x128_PAIR,  // two workgroups per CU (dense_tile_kernel)
+    DT_256, DT_SPLIT
+};
+struct TileCost { float us, e; };
+static int dense_tile_plan(int mode, int64_t M, int64_t N, int64_t kbytes, int64_t batch, bool small_ok,
+                           const DensePlan* split) {
+    static const int BM[] = {32, 32, 32, 64, 128, 128, 128, 128, 256}, BN[] = {32, 64, 128, 64, 64, 128, 256, 128, 256};
+    static const TileCost A8W8[] = {{0.082f, 1.8f}, {0.118f, 2.3f}, {0.198f, 3.4f}, {0.145f, 3.5f}, {0.245f, 2.5f},
+                                    {0.345f, 2.0f}, {0.54f, 3.0f},  {0.60f, 1.8f}, {0.716f, 4.5f}};
+    // MXFP4's 128 x 256 tile would cost more than the 256 x 256 one
+    static const TileCost FP4[] = {{0.091f, 1.8f}, {0.125f, 1.9f}, {0.233f, 2.7f}, {0.161f, 3.1f}, {0.431f, 2.0f},
+                                   {0.589f, 2.3f}, {-1.f, 0.f},    {0.717f, 1.2f}, {0.909f, 3.4f}};
+    static const TileCost BF16[] = {{0.098f, 1.0f}, {0.132f, 1.5f}, {0.216f, 1.7f}, {0.156f, 2.4f}, {0.259f, 1.7f},
+                                    {0.393f, 0.9f}, {0.605f, 1.3f}, {0.58f, 1.5f},  {0.757f, 3.0f}};
+    const TileCost* T = mode == MODE_A8W8 ? A8W8 : mode == MODE_MXFP4 ? FP4 : BF16;
+    const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
+    const float KT = (float)((kbytes + 64) / 128);
+    int best = DT_256;
+    float best_us = 0.f;
+    for (int t = DT_256; t >= 0; --t) {
+        if (T[t].us < 0.f || (t < DT_256 && !small_ok) || (t == DT_128x128_PAIR && kbytes % 128 != 0)) continue;
+        const int64_t tiles = batch * ((M + BM[t] - 1) / BM[t]) * ((N + BN[t] - 1) / BN[t]);
+        const int64_t slots = t == DT_128x128_PAIR ? 2 * ncu : ncu;
+        const float us = (float)((tiles + slots - 1) / slots) * (KT * T[t].us + T[t].e);
+        if (best_us == 0.f || us < best_us) {
+            best = t;
+            best_us = us;
+        }
+    }
+    if (split != nullptr) {
+        const float kt = (float)split->kt_split;
+        const float us = split->geo == GEO_128x64 ? kt * 0.345f + 5.7f
+                                                  : kt * (mode == MODE_BF16 ? 0.5f : 0.4f) + 4.2f + 1.3f * (float)split->splits;
+        if (us < best_us) best = DT_SPLIT;
+    }
+    return best;
+}
+
 template <int MODE, int WM, int WN, int TM, int TN, int KTB, int MINB, int NS = dense_ns<KTB>()>
-static int launch_dense_tiles(DenseParams& p, const DensePlan& pl, hipStream_t stream) {
+static int launch_dense_tiles(DenseParams& p, int splits, int kt_split, void* ws, hipStream_t stream) {
     using Cfg = DenseCfg<MODE, WM, WN, TM, TN, KTB>;
     constexpr int LDS = Cfg::lds_bytes(NS);
     static_assert(LDS * MINB <= 160 * 1024, "LDS budget of a CDNA4 CU");
@@ -802,13 +855,12 @@ static int launch_dense_tiles(DenseParams& p, const DensePlan& pl, hipStream_t s
     p.tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM;
     p.tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
     if (p.group_m <= 0) p.group_m = 8;
-    p.splits = pl.splits;
-    p.kt_split = pl.kt_split;
+    p.splits = splits;
+    p.kt_split = kt_split;
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
-    if (tiles == 0) return 0;
     if (p.splits > 1) {  // dense_plan's workspace: the arrival counters, then the partial sums
-        p.split_cnt = reinterpret_cast<uint64_t*>(p.ws);
-        p.ws = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(p.ws) + SPLIT_CNT_BYTES);
+        p.split_cnt = static_cast<uint64_t*>(ws);
+        p.ws = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + SPLIT_CNT_BYTES);
     }
     kern<<<dim3((unsigned)(tiles * p.splits), (unsigned)std::max(1, p.batch)), 64 * WM * WN, LDS, stream>>>(p);
     return hkq_launch_status();
@@ -870,104 +922,75 @@ static int launch_dense_whole(DenseParams& p, hipStream_t stream) {
     return hkq_launch_status();
 }
 
-// The narrow path serves the FP8 and FP4 GEMMs whose rows hold whole 128-value
-// K-steps: all of M <= 16, and M <= 32 while the 16-column workgroups number
-// fewer than two per CU and K is at most 32 steps (beyond that, every
-// workgroup re-reading the activation rows costs more than the tiled path's
-// LDS-shared activation tile; measured on MI355X). Its buffer offsets are
-// 32-bit: 16*NT weight rows and 32 activation rows must span less than 2 GiB.
+// The narrow path: A8W8 with at most 32 K-steps, and at most 16 rows where the
+// 16-column workgroups fit one per CU, 4 where they come to more than four
+// rounds, 1 between (measured on MI355X against the small tiles: 1x4096x4096
+// 4.4 us and 5.9, 16x4096x4096 5.7 and 6.1, 4x28672x4096 23.1 and 25.0,
+// 8x28672x4096 26.1 and 25.2, 1x14336x4096 11.4 and 11.7, 4x6144x4096 7.4 and
+// 7.1; with 128 K-steps 4x512x16384 12.0 and 10.4). Its buffer offsets are
+// 32-bit.
 static bool use_narrow(int mode, int64_t M, int64_t N, int64_t kbytes, int64_t lda, int64_t ldb, int64_t batch) {
-    if (mode != MODE_A8W8 && mode != MODE_MXFP4) return false;
-    const int64_t step = mode == MODE_MXFP4 ? 64 : 128;
-    if (M < 1 || M > NARROW_MAX_M || kbytes % step != 0 || 64 * ldb >= (1ll << 31) || NARROW_MAX_M * lda >= (1ll << 31))
-        return false;
-    if (M <= 16) return true;
     const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
-    return std::max<int64_t>(1, batch) * ((N + 15) / 16) < 2 * ncu && kbytes / step <= 32;
-}
-
-template <int MODE, int MT, int NT>
-static int launch_narrow_nt(const DenseParams& p, hipStream_t stream) {
-    const dim3 grid((unsigned)((p.N + 16 * NT - 1) / (16 * NT)), (unsigned)std::max(1, p.batch));
-    narrow_gemm_kernel<MODE, MT, NT><<<grid, 64 * NARROW_WAVES, 0, stream>>>(p);
-    return hkq_launch_status();
-}
-
-// Columns per workgroup: 16 * NT. One round of 16-column workgroups: NT = 1;
-// up to three rounds: NT = 2 (one round, activation fragments used twice);
-// more: NT = 4 (measured on MI355X at N = 4096 .. 28672).
-template <int MODE>
-static int launch_narrow(const DenseParams& p, hipStream_t stream) {
-    if constexpr (MODE == MODE_A8W8 || MODE == MODE_MXFP4) {
-        if (p.N == 0) return 0;
-        const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
-        const int64_t wgs16 = (int64_t)std::max(1, p.batch) * ((p.N + 15) / 16);
-        const int nt = wgs16 <= ncu ? 1 : wgs16 <= 3 * ncu ? 2 : 4;
-        if (p.M <= 16) {
-            if (nt == 4) return launch_narrow_nt<MODE, 1, 4>(p, stream);
-            if (nt == 2) return launch_narrow_nt<MODE, 1, 2>(p, stream);
-            return launch_narrow_nt<MODE, 1, 1>(p, stream);
-        }
-        if (nt == 4) return launch_narrow_nt<MODE, 2, 4>(p, stream);
-        if (nt == 2) return launch_narrow_nt<MODE, 2, 2>(p, stream);
-        return launch_narrow_nt<MODE, 2, 1>(p, stream);
-    }
-    return 0;
-}
-
-// 128-byte K-tiles need whole 128-byte K-tiles in every row: a partial last
-// K-tile would read the next row's bytes instead of zeros.
-template <int MODE, int KTB>
-static int launch_dense_ktb(DenseParams& p, void* ws, size_t ws_bytes, hipStream_t stream) {
-    if (use_narrow(MODE, p.M, p.N, p.kbytes, p.lda, p.ldb, p.batch)) return launch_narrow<MODE>(p, stream);
-    p.c16 = (p.ldc % 8 == 0) && (reinterpret_cast<uintptr_t>(p.C) % 16 == 0);
-    // batches and bias run unsplit (the split partials and their reduction are per 2-D GEMM)
-    const bool plain = p.batch <= 1 && p.bias == nullptr;
-    DensePlan pl = dense_plan(MODE, p.M, p.N, p.kbytes, plain, std::max(1, p.batch));
-    if (pl.splits > 1 && (ws == nullptr || ws_bytes < pl.ws_bytes))
-        pl = dense_plan(MODE, p.M, p.N, p.kbytes, false, std::max(1, p.batch));
-    p.ws = static_cast<float*>(ws);
-    if constexpr (KTB == 128) {  // smaller tiles need a full 16-byte load per lane for their A rows
-        if (pl.geo == GEO_SKINNY) {
-            if (pl.skinny_tm == 1) return launch_dense_tiles<MODE, 1, SKINNY_WAVES_N, 1, SKINNY_TN, KTB, 1>(p, pl, stream);
-            return launch_dense_tiles<MODE, 1, SKINNY_WAVES_N, 2, SKINNY_TN, KTB, 1>(p, pl, stream);
-        }
-        // Grids of at most one workgroup per CU run one workgroup each with a
-        // 3-stage ring (two K-tiles of loads in flight) rather than two per CU
-        // with 2-stage rings (measured on MI355X: 128 x 128 tiles at
-        // 1024x4096x4096 25.8 -> 21.2 us, 1024x4096x14336 75.1 -> 58.1,
-        // 512x4096x4096 21.4 -> 15.8; 128 x 64 tiles at 128x4096x4096 12.7 ->
-        // 11.3, 128x6144x4096 13.3 -> 11.4; at 1.5 rounds, 1024x6144x4096,
-        // two per CU win: 29.6 vs 36.5). MXFP4's scale blocks assume 2 stages.
-        const int ncu = cu_count() > 0 ? cu_count() : 256;
-        const bool one_round = pl.tiles * pl.splits * std::max(1, p.batch) <= ncu;
-        if (pl.geo == GEO_128) {
-            if (one_round) {
-                if constexpr (MODE == MODE_MXFP4) {  // the scale blocks keep 2 stages
-                    return launch_dense_tiles<MODE, 2, 2, 2, 2, KTB, 1, 2>(p, pl, stream);
-                } else {
-                    if (pl.kt_split >= 4) return launch_dense_tiles<MODE, 2, 2, 2, 2, KTB, 1, 4>(p, pl, stream);
-                    return launch_dense_tiles<MODE, 2, 2, 2, 2, KTB, 1, 3>(p, pl, stream);
-                }
-            }
-            return launch_dense_tiles<MODE, 2, 2, 2, 2, KTB, 2>(p, pl, stream);
-        }
-        if constexpr (MODE == MODE_A8W8)
-            if (pl.geo == GEO_128x64) {
-                if (one_round) {
-                    if (pl.kt_split >= 6) return launch_dense_tiles<MODE, 4, 1, 1, 2, KTB, 1, 6>(p, pl, stream);
-                    return launch_dense_tiles<MODE, 4, 1, 1, 2, KTB, 1, 3>(p, pl, stream);
-                }
-                return launch_dense_tiles<MODE, 4, 1, 1, 2, KTB, 2>(p, pl, stream);
-            }
-    }
-    return launch_dense_whole<MODE, KTB>(p, stream);
+    if (mode != MODE_A8W8 || M < 1 || kbytes % 128 != 0 || kbytes / 128 > NARROW_MAX_STEPS) return false;
+    const int64_t wgs = batch * ((N + 15) / 16);
+    return M <= (wgs <= ncu ? NARROW_MAX_M : wgs > 4 * ncu ? 4 : 1) && 16 * ldb < (1ll << 31) && 16 * lda < (1ll << 31);
 }
 
 template <int MODE>
 static int launch_dense(DenseParams& p, void* ws, size_t ws_bytes, hipStream_t stream) {
-    return p.kbytes % 128 == 0 ? launch_dense_ktb<MODE, 128>(p, ws, ws_bytes, stream)
-                               : launch_dense_ktb<MODE, 64>(p, ws, ws_bytes, stream);
+    p.c16 = (p.ldc % 8 == 0) && (reinterpret_cast<uintptr_t>(p.C) % 16 == 0);
+    if (p.M == 0 || p.N == 0) return 0;
+    const int64_t batch = std::max(1, p.batch);
+    if (use_narrow(MODE, p.M, p.N, p.kbytes, p.lda, p.ldb, batch)) {
+        const dim3 grid((unsigned)((p.N + 15) / 16), (unsigned)batch);
+        narrow_gemm_kernel<<<grid, 64 * NARROW_WAVES, 0, stream>>>(p);
+        return hkq_launch_status();
+    }
+    // the split partials and their reduction are per 2-D GEMM without bias
+    DensePlan pl{};
+    bool split = false;
+    if constexpr (MODE != MODE_MXFP4) {
+        pl = dense_plan(MODE, p.M, p.N, p.kbytes);
+        split = p.batch <= 1 && p.bias == nullptr && pl.geo != GEO_SKINNY && pl.splits > 1 && ws != nullptr &&
+                ws_bytes >= pl.ws_bytes;
+    }
+    // 32-bit row offsets of the small tiles (128 activation rows, 256 weight rows)
+    const bool small_ok = 128 * p.lda < (1ll << 31) && 256 * p.ldb < (1ll << 31) && 128 * p.lsa < (1ll << 31) &&
+                          256 * p.lsb < (1ll << 31);
+    constexpr int M4 = MODE == MODE_MXFP4;  // the e8m0 blocks take LDS from the ring
+    switch (dense_tile_plan(MODE, p.M, p.N, p.kbytes, batch, small_ok, split ? &pl : nullptr)) {
+        case DT_32x32: return launch_dense_kgroup<KgCfg<MODE, 1, 1, 4, 1, 1, 4>>(p, stream);
+        case DT_32x64: return launch_dense_kgroup<KgCfg<MODE, 1, 1, 4, 1, 2, 3 - M4>>(p, stream);
+        case DT_32x128: return launch_dense_kgroup<KgCfg<MODE, 1, 1, 4 - M4, 1, 4, 2>>(p, stream);
+        case DT_64x64: return launch_dense_kgroup<KgCfg<MODE, 1, 1, 4, 2, 2, 2>>(p, stream);
+        case DT_128x64: return launch_dense_kgroup<KgCfg<MODE, 4, 1, 2, 1, 2, 3 - M4>>(p, stream);
+        case DT_128x128: return launch_dense_kgroup<KgCfg<MODE, 4, 2, 1, 1, 2, 4>>(p, stream);
+        case DT_128x256:
+            if constexpr (!M4) return launch_dense_kgroup<KgCfg<MODE, 2, 4, 1, 2, 2, 3>>(p, stream);
+            break;
+        case DT_128x128_PAIR:
+            return launch_dense_tiles<MODE, 2, 2, 2, 2, 128, 2>(p, 1, p.kbytes / 128, nullptr, stream);
+        case DT_SPLIT:
+            // one workgroup per CU where the splits allow, on a deeper ring
+            // (two K-tiles of loads in flight or more)
+            if constexpr (!M4) {
+                const int ncu = cu_count() > 0 ? cu_count() : 256;
+                const bool one_round = pl.tiles * pl.splits <= ncu;
+                const int S = pl.splits, kt = pl.kt_split;
+                if constexpr (MODE == MODE_A8W8)
+                    if (pl.geo == GEO_128x64) {
+                        if (!one_round) return launch_dense_tiles<MODE, 4, 1, 1, 2, 128, 2>(p, S, kt, ws, stream);
+                        if (kt >= 6) return launch_dense_tiles<MODE, 4, 1, 1, 2, 128, 1, 6>(p, S, kt, ws, stream);
+                        return launch_dense_tiles<MODE, 4, 1, 1, 2, 128, 1, 3>(p, S, kt, ws, stream);
+                    }
+                if (!one_round) return launch_dense_tiles<MODE, 2, 2, 2, 2, 128, 2>(p, S, kt, ws, stream);
+                return launch_dense_tiles<MODE, 2, 2, 2, 2, 128, 1, 4>(p, S, kt, ws, stream);
+            }
+            break;
+    }
+    // 128-byte K-tiles of this kernel need whole ones in every row: a partial
+    // last K-tile would read the next row's bytes instead of zeros
+    return p.kbytes % 128 == 0 ? launch_dense_whole<MODE, 128>(p, stream) : launch_dense_whole<MODE, 64>(p, stream);
 }
 
 }  // namespace hkq
@@ -983,11 +1006,20 @@ static int check_common(int64_t M, int64_t N, int64_t K, int64_t ldc, const void
     return 0;
 }
 
+// Shapes that the workspace queries answer with 0: M <= 16, and M <= 32 with
+// fewer than two 16-column slices per CU and at most 32 K-steps of 128 values
+// (`step` bytes each), whose rows hold whole K-steps.
+static bool no_split(int64_t M, int64_t N, int64_t kbytes, int64_t step) {
+    if (M > 32 || kbytes % step != 0 || 64 * kbytes >= (1ll << 31)) return false;
+    const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
+    return M <= 16 || ((N + 15) / 16 < 2 * ncu && kbytes / step <= 32);
+}
+
 extern "C" {
 
 size_t hkq_gemm_a8w8_workspace(int64_t M, int64_t N, int64_t K) {
-    if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || use_narrow(MODE_A8W8, M, N, K, K, K, 1)) return 0;
-    return dense_plan(MODE_A8W8, M, N, K, true).ws_bytes;
+    if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || no_split(M, N, K, 128)) return 0;
+    return dense_plan(MODE_A8W8, M, N, K).ws_bytes;
 }
 
 int hkq_gemm_a8w8_ws(const void* A, const void* B, const float* sa, const float* sb, void* C, int64_t M, int64_t N,
@@ -1075,8 +1107,8 @@ int hkq_gemm_a8w8_noalloc(const void* A, const void* B, const float* sa, const f
 }
 
 size_t hkq_gemm_mxfp4_workspace(int64_t M, int64_t N, int64_t K) {
-    if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0 || use_narrow(MODE_MXFP4, M, N, K / 2, K / 2, K / 2, 1)) return 0;
-    return dense_plan(MODE_MXFP4, M, N, K / 2, true).ws_bytes;
+    if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0 || no_split(M, N, K / 2, 64)) return 0;
+    return dense_plan(MODE_MXFP4, M, N, K / 2).ws_bytes;
 }
 
 int hkq_gemm_mxfp4_ws(const void* A, const void* As, const void* B, const void* Bs, void* C, int64_t M, int64_t N,
@@ -1146,7 +1178,7 @@ int hkq_batched_gemm_a8w8(const void* A, const void* B, const float* sa, const f
 
 size_t hkq_gemm_bf16_workspace(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 32 != 0) return 0;
-    return dense_plan(MODE_BF16, M, N, 2 * K, true).ws_bytes;
+    return dense_plan(MODE_BF16, M, N, 2 * K).ws_bytes;
 }
 
 int hkq_batched_gemm_bf16(const void* A, const void* B, const void* bias, void* C, int64_t batch, int64_t M, int64_t N,

@@ -11,7 +11,7 @@
 // wave's LDS reads, promotions and waits run under another's MFMAs without
 // fragment double-buffering, and the loop stays small enough for deep rings.
 //
-// K-tiles are 128 bytes per row (KTile<128>), staged with LDS-direct loads
+// K-tiles are 128 bytes per row (KTile<128>; the last one may hold 64), staged with LDS-direct loads
 // into an NS-stage ring per group. Groups of one wave (WM * WN == 1) need no
 // barrier: a wave waits for its own loads, reads its fragments and refills
 // the stage at once. Groups of several waves share one barrier per K-tile
@@ -91,6 +91,9 @@ struct KgSrc {
     uint32_t bs_step;
     int sc_shift;
     int KT;  // K-tiles
+    // the last K-tile holds 64 bytes of K per row (linear operands): the lanes
+    // that carry its upper four chunks read nothing, so the LDS holds zeros there
+    bool half_tail = false;
 };
 
 __device__ __forceinline__ uint32_t clamp_bytes(int64_t n) {
@@ -143,6 +146,13 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
     // this group's K-tiles
     const int k0 = kg * src.KT / KG, mine = (kg + 1) * src.KT / KG - k0;
 
+    // OOB in the lanes that carry chunks 4 .. 7 of a row
+    uint32_t upper[GATHER ? 1 : Cfg::SWP];
+    if constexpr (!GATHER) {
+#pragma unroll
+        for (int i = 0; i < Cfg::SWP; ++i)
+            upper[i] = KT::load_chunk(lane, kg_row<Cfg>(i, wg, lane)) >= 4 ? OOB : 0u;
+    }
     // the loads of round t (K-tile k0 + t); past the group's last they read
     // nothing. A scale block goes out before the first K-tile that uses it, so
     // the wait for that K-tile covers it; the waits count operand loads only.
@@ -168,14 +178,16 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
         HKQ_LDS uint8_t* st = gbase + stage * STAGE;
         const uint32_t kb = live ? (uint32_t)kt * 128u : OOB;
         constexpr int SWP = Cfg::SWP;
+        const uint32_t tail = src.half_tail && kt == src.KT - 1 ? OOB : 0u;
         if (idx < LB) {
-            lds_load16_s(src.b, st + Cfg::BM * 128 + (idx * GW + wg) * 1024, src.b_off[idx % SWP],
+            const uint32_t off = GATHER ? src.b_off[idx % SWP] : src.b_off[idx % SWP] | (upper[GATHER ? 0 : idx % SWP] & tail);
+            lds_load16_s(src.b, st + Cfg::BM * 128 + (idx * GW + wg) * 1024, off,
                          live ? kb + (uint32_t)(idx / SWP) * src.b_step : OOB);
         } else if (idx < LB + LA) {
             const int i = idx - LB;
             if constexpr (GATHER) lds_load16_s(src.a, st + (i * GW + wg) * 1024, src.a_off[i], kb);
             else
-                lds_load16_s(src.a, st + (i * GW + wg) * 1024, src.a_off[i % SWP],
+                lds_load16_s(src.a, st + (i * GW + wg) * 1024, src.a_off[i % SWP] | (upper[i % SWP] & tail),
                              live ? kb + (uint32_t)(i / SWP) * src.a_step : OOB);
         } else {
             const int i = idx - LB - LA, q = (i * GW + wg) % Cfg::PC;  // repeated where there are fewer loads than waves
@@ -222,8 +234,9 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
         for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
             for (int q = 0; q < 2; ++q) (isb ? f.b[isb ? i : 0] : f.a[isb ? 0 : i])[ks][q] = lds_read16(base + lo[ks][q]);
-        // the scales of a round past the group's last one are stale: zeros
-        const bool live = t < mine;
+        // the scales of a round past the group's last one are stale, those of a
+        // half last K-tile's upper blocks the next row's: zeros
+        const bool live = t < mine && !(FP4 && src.half_tail && k0 + t == src.KT - 1 && khalf);
         if constexpr (FP4) {
             const int kt = k0 + t;
             const HKQ_LDS uint8_t* sl = sblk + ((kt / Cfg::SBK) & 1) * Cfg::SBLK + r * 32 +

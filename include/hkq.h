@@ -121,14 +121,15 @@ int hkq_gemm_a8w8(const void* A, const void* B, const float* sa, const float* sb
                   int64_t K, int64_t lda, int64_t ldb, int64_t ldc, hkq_stream_t stream);
 
 /* hkq_gemm_a8w8 with a caller-provided device workspace (16-byte aligned).
- * Shapes whose tiles would fill at most half of the CUs (256 x 256 tiles
- * become 128 x 128 or 128 x 64, or (32 or 64) x 256 for M <= 64, first) split
- * K over several workgroups in one launch: each writes its fp32 partial sums
- * to the workspace, and the last split of a tile to finish adds all of them in
- * split order and writes C (bit-identical whichever split finishes last).
- * That needs hkq_gemm_a8w8_workspace(M, N, K) bytes (0: no split for this
- * shape; M <= 16 runs a single-launch streaming kernel that needs none). With
- * a smaller workspace (or NULL) the call runs unsplit. Same results either way
+ * Shapes whose 128 x 128 or 128 x 64 tiles would fill at most half of the CUs
+ * may split K over several workgroups in one launch where that is the faster
+ * plan (a long K): each writes its fp32 partial sums to the workspace, and the
+ * last split of a tile to finish adds all of them in split order and writes C
+ * (bit-identical whichever split finishes last). hkq_gemm_a8w8_workspace(M, N,
+ * K) bytes cover every such plan (0: no split for this shape); many shapes
+ * with a size run small tiles that split K inside a workgroup and leave the
+ * workspace alone. With a smaller workspace (or NULL) the call runs without
+ * the split across workgroups. Same results either way
  * up to fp32 summation order. The workspace needs no clearing: its first 4 KB
  * hold per-tile arrival counters that each call leaves marked idle (a
  * workspace that held other data is claimed on first use, at the cost of one
@@ -163,9 +164,10 @@ int hkq_gemm_a8w8_noalloc(const void* A, const void* B, const float* sa, const f
 int hkq_gemm_mxfp4(const void* A, const void* As, const void* B, const void* Bs, void* C, int64_t M, int64_t N,
                    int64_t K, int64_t lda, int64_t ldb, int64_t ldsa, int64_t ldsb, int64_t ldc, hkq_stream_t stream);
 
-/* hkq_gemm_mxfp4 with a caller-provided workspace: the split-K plan of
- * hkq_gemm_a8w8_ws for the MXFP4 GEMM (no counterpart in the reference;
- * gemm_afp4wfp4_tk calls it with a workspace from torch's allocator). */
+/* hkq_gemm_mxfp4 with a caller-provided workspace, the interface of
+ * hkq_gemm_a8w8_ws (no counterpart in the reference; gemm_afp4wfp4_tk calls it
+ * with a workspace from torch's allocator). The plans of the MXFP4 GEMM split K
+ * inside a workgroup only and leave the workspace alone. */
 size_t hkq_gemm_mxfp4_workspace(int64_t M, int64_t N, int64_t K);
 int hkq_gemm_mxfp4_ws(const void* A, const void* As, const void* B, const void* Bs, void* C, int64_t M, int64_t N,
                       int64_t K, int64_t lda, int64_t ldb, int64_t ldsa, int64_t ldsb, int64_t ldc, void* workspace,

@@ -469,3 +469,47 @@ def test_gemm_bf16_stream_tiles(orc, M, N, K):
     a = torch.from_numpy(orc.bf16_bits_to_f32(A))
     b = torch.from_numpy(orc.bf16_bits_to_f32(B))
     assert_gemm_close(host_bf16_f32(C), (a @ b.T).numpy(), f"bf16 stream {M}x{N}x{K}")
+
+
+# The small tiles of the dense GEMMs with K split over the workgroup's waves:
+# odd counts of K-tiles (uneven shares of the wave groups, a last scale block
+# of 1 or 3 K-tiles) and a half last K-tile, ragged M and N, rows of A (and of its
+# scales) padded with NaN codes, C's padding untouched. K is in 128-byte K-tiles
+# per row; on 256
+# CUs the sizes are 32x32, 32x64, 32x128, 64x64, 128x64, 128x128, 128x256 or
+# two 128x128 workgroups per CU, as the operand format's costs decide.
+@pytest.mark.parametrize("mode", ["a8w8", "mxfp4", "bf16"])
+@pytest.mark.parametrize("M,N,KT", [(17, 300, 5), (9, 40, 1), (31, 8196, 9), (30, 16388, 5), (130, 4100, 15),
+                                    (161, 7172, 9), (333, 7172, 9), (1000, 7172, 5), (900, 10244, 3),
+                                    (6, 1964, 20.5), (40, 1000, 0.5), (100, 4100, 4.5), (333, 7172, 8.5),
+                                    (700, 7172, 2.5)])
+def test_gemm_small_tiles(orc, mode, M, N, KT):
+    require_gpu()
+    Cp = torch.full((M, N + 4), 7.0, dtype=torch.bfloat16, device="cuda")
+    C = Cp[:, :N]
+    if mode == "bf16":
+        K = int(64 * KT)
+        xa, xw = orc.randn_bf16((M, K), seed=M), orc.randn_bf16((N, K), seed=N, std=0.02)
+        Ap = torch.full((M, K + 24), float("nan"), dtype=torch.bfloat16, device="cuda")
+        Ap[:, :K] = torch.from_numpy(xa.view(np.int16)).cuda().view(torch.bfloat16)
+        hkq.gemm_bf16(Ap[:, :K], torch.from_numpy(xw.view(np.int16)).cuda().view(torch.bfloat16), C)
+        ref = orc.gemm_bf16_ref(xa, xw)
+    elif mode == "a8w8":
+        K = int(128 * KT)
+        A, B, sa, sb = a8w8_inputs(orc, M, N, K, seed=M + N + K)
+        Ap = torch.full((M, K + 48), 0x7F, dtype=torch.uint8, device="cuda")
+        Ap[:, :K] = dev_u8(A)
+        hkq.gemm_a8w8(Ap[:, :K], dev_u8(B), dev_f32(sa), dev_f32(sb), C)
+        ref = orc.gemm_a8w8_ref_f32(A, B, sa, sb)
+    else:
+        K = int(256 * KT)
+        Aq, As, Bq, Bs = mx_inputs(orc, M, N, K, seed=M * 3 + K)
+        Ap = torch.full((M, K // 2 + 32), 0x77, dtype=torch.uint8, device="cuda")
+        Ap[:, :K // 2] = dev_u8(Aq)
+        Asp = torch.full((M, K // 32 + 4), 0xFF, dtype=torch.uint8, device="cuda")
+        Asp[:, :K // 32] = dev_u8(As)
+        hkq.gemm_mxfp4(Ap[:, :K // 2], Asp[:, :K // 32], dev_u8(Bq), dev_u8(Bs), C)
+        ref = orc.gemm_mxfp4_ref_f32(Aq, As, Bq, Bs)
+    torch.cuda.synchronize()
+    assert bool((Cp[:, N:] == 7.0).all()), "stores past N reached the row padding"
+    assert_gemm_close(host_bf16_f32(C), ref, f"{mode} small tiles {M}x{N}x{K}")
