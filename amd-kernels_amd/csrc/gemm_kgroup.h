@@ -418,4 +418,26 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
     }
 }
 
+// Tile of a grouped (MoE) GEMM whose experts hold `routed` rows in all, by the
+// mean rows per expert (the counts themselves are on the GPU): a tile's rows
+// should hold an expert's few rows once, and its columns keep the weights of
+// two workgroups per CU in flight. Beyond one routing block per expert the
+// block-pair kernels read the weights once for 256 rows and win. Measured on
+// MI355X, block-scale layers (gate/up and down together; 8 experts of 4096 x
+// 14336, top-2, tokens: us for the four tiles in order, then the pair kernel):
+// 24: 269 / 301 / 317 / 385 / 441; 90: 290 / 316 / 329 / 394 / 456; 150: 456 /
+// 324 / 342 / 403 / 469; 350: 741 / 519 / 376 / 420 / 505; 512: 977 / 631 /
+// 507 / 446 / 530; 1200: - / 1008 / 852 / 743 / 685. With a short K the wider
+// tile's fewer workgroups win earlier, and the pairs too (32 experts of 2048 x
+// 2816, top-4: 512: 261 / 189 / 175 / 169 / 183; 800: - / 233 / 188 / 178 /
+// 197; 1000: 212 on 128 x 256 against 208).
+enum MoeTile { MOET_32x64, MOET_64x128, MOET_128x128, MOET_128x256, MOET_PAIRS };
+inline MoeTile moe_tile(int64_t routed, int64_t experts, int64_t K) {
+    const int64_t r = routed / (experts > 0 ? experts : 1);
+    if (r <= 22) return MOET_32x64;
+    if (r <= 48) return MOET_64x128;
+    if (K <= 3072) return r <= 112 ? MOET_128x256 : MOET_PAIRS;
+    return r <= 96 ? MOET_128x128 : r <= 128 ? MOET_128x256 : MOET_PAIRS;
+}
+
 }  // namespace hkq

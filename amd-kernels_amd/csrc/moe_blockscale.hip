@@ -15,7 +15,8 @@
 //
 // fp32 group scales cannot ride in the MFMA's e8m0 operands, so every K-tile
 // of one scale group is promoted on the VALU: acc += P * xs * ws, P the
-// tile's partial of a 32x32 sub-tile. Two kernels:
+// tile's partial of a 32x32 sub-tile. Three kernels:
+//  - few rows per expert: small tiles of gemm_kgroup.h (moe_bs_tile_kernel);
 //  - group_k = 128 * 2^j and K % 128 == 0: the 8-wave K loop of
 //    blockscale_core.h (128-wide K-tiles, two MFMAs per partial) over
 //    256 x 256 tiles that take two routing blocks of an expert at once;
@@ -33,6 +34,7 @@
 // scales [E, K/32, N], tests/test_moe.py:723-729, 808-815, 909-925) into the
 // K-contiguous [E, N, R] rows the MoE kernels stream into LDS.
 #include "blockscale_core.h"
+#include "gemm_kgroup.h"
 #include "hkq_host.h"
 
 #include <cstdlib>
@@ -569,6 +571,113 @@ __global__ __launch_bounds__(64 * BS_NW, 1) void moe_blockscale8_kernel(const Mo
                                 NoBias{});
 }
 
+// ---------------------------------------------------------------------------
+// Few rows per expert (at most one routing block on average): small tiles with
+// K split over the workgroup's waves (gemm_kgroup.h), a workgroup per routing
+// word and column tile, walking the block's rows BM at a time. Bound by the
+// weights' way from HBM: 256-row tiles gave every 16-row block the loads,
+// barriers and LDS of 256 rows, and one workgroup per CU left it idle between
+// tiles. With 32-row tiles two workgroups share a CU (78 KB of LDS each), so
+// one's prologue and epilogue run under the other's stream. Measured on MI355X
+// (8 experts of 4096 x 14336, top-2, whole layer with 128 x 128 groups, which
+// reads 1.41 GB of weights): 64 tokens 442 -> 281 us (5.0 TB/s), 1 token 222
+// -> 102, 300 tokens 494 -> 350, 512 tokens 530 -> 446.
+template <class Cfg, int MINB>
+__global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_bs_tile_kernel(const MoeBsParams p) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
+    HKQ_LDS uint8_t* smem = (HKQ_LDS uint8_t*)smem_raw;
+    constexpr int BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TMO = Cfg::TMO;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wg = wave % Cfg::GW, kg = wave / Cfg::GW;
+    const int pm = blockIdx.x / p.tiles_n, tn = blockIdx.x % p.tiles_n;
+    const int ed = p.expt_data[pm];
+    const int e = ed & 0xFFFF, b = ed >> 16;
+    if (ed < 0 || e >= p.E) return;  // uniform: -1 or a malformed entry
+    const int m_e = p.hist[e], start = p.offs[e];
+    const int rows = min(m_e - b * 128, 128);
+    if (rows <= 0 || start < 0) return;
+    const int n0 = tn * BN;
+    const int rows_b = min(p.N - n0, BN);
+
+    KgSrc<Cfg, true> src;
+    src.KT = p.K / 128;
+    src.sc_shift = 31 - __builtin_clz(p.gk / 128);
+    src.a = buffer_desc(p.X, clamp_bytes((int64_t)p.T * p.sxm));
+    src.b = buffer_desc(p.W + (int64_t)e * p.swe + (int64_t)n0 * p.swn, clamp_bytes((int64_t)rows_b * p.swn));
+    src.as = buffer_desc(p.xs, clamp_bytes(p.xs_elems * 4));
+    src.bs = buffer_desc(p.ws + (int64_t)e * p.wse, clamp_bytes((p.ws_elems - (int64_t)e * p.wse) * 4));
+    src.bs_step = (uint32_t)p.wsk * 4u;
+    src.b_step = (uint32_t)(8 * Cfg::GW * Cfg::SWP * p.swn);
+#pragma unroll
+    for (int i = 0; i < Cfg::SWP; ++i) {
+        const int r = kg_row<Cfg>(i, wg, lane);
+        src.b_off[i] = (uint32_t)(r * p.swn) + kg_chunk<Cfg>(r, lane);
+    }
+    const int nw = n0 + wg % Cfg::WN * TN * 32;
+    for (int row0 = b * 128; row0 < b * 128 + rows; row0 += BM) {
+        auto token_of = [&](int r) {
+            const int s = start + row0 + r;
+            if (row0 + r >= b * 128 + rows || r >= BM || s >= p.g_len) return -1;
+            const int t = p.gather ? div_recip(p.gather[s], p.rtopk) : s;
+            return (t >= 0 && t < p.T) ? t : -1;
+        };
+#pragma unroll
+        for (int i = 0; i < Cfg::LA; ++i) {
+            const int r = kg_row<Cfg>(i, wg, lane), t = token_of(r);
+            src.a_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.sxm + kg_chunk<Cfg>(r, lane);
+        }
+#pragma unroll
+        for (int i = 0; i < Cfg::PW; ++i) {
+            const int q = i * Cfg::GW + wg;
+            if (q < Cfg::PA) {
+                const int t = token_of(kg_piece_row<Cfg>(q, lane));
+                src.s_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.xsm * 4u;
+            } else {
+                src.s_off[i] = (uint32_t)(min(n0 + (lane >> 2) * 32, p.N - 1) / p.gn) * (uint32_t)p.wsn * 4u +
+                               (uint32_t)(lane & 3) * src.bs_step;
+            }
+        }
+        v16f acc[TN][TMO];
+        kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
+        if (Cfg::SPREAD || kg == 0) {
+            const int s0 = start + row0;
+            const int mw = (wg / Cfg::WN * Cfg::TM + (Cfg::SPREAD ? kg * TMO : 0)) * 32;
+            const int out_rows = min(min(b * 128 + rows - row0, BM), p.y_rows - s0);
+            auto one = [](int) { return 1.0f; };
+            auto ones = [](int, int) { return make_float4(1.f, 1.f, 1.f, 1.f); };
+            const int ep = Cfg::SPREAD ? wave : wg;
+            uint16_t* Y = p.Y + (int64_t)s0 * p.sym;
+            store_tile_bf16<TMO, TN>(acc, smem, ep, lane, Y, p.sym, out_rows, p.N, mw, nw, p.c16 != 0, one, ones,
+                                     [&](int i, int g) {
+                                         const int n = nw + i * 32 + 8 * g + 4 * (lane >> 5);
+                                         if (!p.bias || n >= p.N) return make_float4(-0.f, -0.f, -0.f, -0.f);
+                                         const float* bp = p.bias + (int64_t)e * p.bias_e + n;
+                                         return make_float4(bp[0], bp[1], bp[2], bp[3]);
+                                     });
+        }
+        __syncthreads();  // the staging is read: the next row group's loads may overwrite it
+    }
+}
+
+template <class Cfg, int MINB>
+static int launch_moe_bs_tile(MoeBsParams& p, hipStream_t stream) {
+    static_assert(Cfg::LDS * MINB <= 160 * 1024, "LDS budget of a CDNA4 CU");
+    auto kern = moe_bs_tile_kernel<Cfg, MINB>;
+    static bool attr_set = false;
+    if (!attr_set) {
+        hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS);
+        if (err != hipSuccess) {
+            set_error("hipFuncSetAttribute(MaxDynamicSharedMemorySize=%d) failed: %s", Cfg::LDS, hipGetErrorString(err));
+            return (int)err;
+        }
+        attr_set = true;
+    }
+    p.tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
+    kern<<<dim3((unsigned)((int64_t)p.grid_m * p.tiles_n)), Cfg::THREADS, Cfg::LDS, stream>>>(p);
+    return hkq_launch_status();
+}
+
 }  // namespace hkq
 
 using namespace hkq;
@@ -673,6 +782,18 @@ static int moe_blockscale_impl(const void* X, const void* W, void* Y, const floa
         const int64_t nblk = grid_m * p.tiles_n;
         if (nblk == 0) return 0;
         const bool ntile = group_n % 32 == 0;
+        // few rows per expert: small tiles over one routing block (K-contiguous
+        // weights, one column scale per 32 columns, K-contiguous row scales)
+        if (ntile && !wt && xs_stride_k == 1) {
+            constexpr int B = MODE_BLOCKSCALE;
+            switch (moe_tile(gather ? T * topk : T, E, K)) {
+                case MOET_32x64: return launch_moe_bs_tile<KgCfg<B, 1, 1, 3, 1, 2, 2>, 2>(p, stream);
+                case MOET_64x128: return launch_moe_bs_tile<KgCfg<B, 2, 2, 1, 1, 2, 3>, 2>(p, stream);
+                case MOET_128x128: return launch_moe_bs_tile<KgCfg<B, 4, 2, 1, 1, 2, 4>, 1>(p, stream);
+                case MOET_128x256: return launch_moe_bs_tile<KgCfg<B, 2, 4, 1, 2, 2, 3>, 1>(p, stream);
+                case MOET_PAIRS: break;
+            }
+        }
         auto kern = ntile ? (wt ? moe_blockscale8_kernel<BS_SB_NTILE, true> : moe_blockscale8_kernel<BS_SB_NTILE>)
                           : (wt ? moe_blockscale8_kernel<BS_SB_COL, true> : moe_blockscale8_kernel<BS_SB_COL>);
         const int v8 = (ntile ? 1 : 0) + (wt ? 2 : 0);

@@ -432,6 +432,38 @@ def test_moe_blockscale(orc, T, E, topk, K, N, gk, gn):
     check_rows(orc, Y, ref)
 
 
+# Few rows per expert: the small tiles by mean rows per expert (10, 33, 75 and
+# 115: 32x64, 64x128, then 128x256 or, from K = 3200, 128x128, then block
+# pairs), routing skewed so that some experts
+# hold several row groups or blocks and some no row, odd counts of K-tiles, one
+# or two K-tiles per scale group, ragged N, a bias, -1 / malformed words between
+# the live ones and scale rows padded with NaN.
+@pytest.mark.parametrize("T,E,topk,K,N,gk", [(40, 8, 2, 640, 300, 128), (3, 8, 2, 128, 1000, 128),
+                                             (100, 6, 2, 1152, 260, 128), (150, 4, 2, 896, 772, 256),
+                                             (150, 4, 2, 3200, 132, 128), (230, 4, 2, 640, 1028, 128)])
+def test_moe_blockscale_small_tiles(orc, T, E, topk, K, N, gk):
+    require_gpu()
+
+    def skewed(rng, T, E, topk):
+        p = np.array([6.0] + [1.0] * (E - 2) + [0.0])
+        return np.stack([rng.choice(E, size=topk, replace=False, p=p / p.sum()) for _ in range(T)])
+
+    _, hist, offs, gather, ed, X, _, W, _ = make_problem(orc, T, E, topk, K, N, T + N, skewed)
+    ed = np.concatenate([[-1, E + 3], ed, [-1]]).astype(np.int32)
+    rng = np.random.default_rng(T)
+    G, C = -(-K // gk), -(-N // 128)
+    xs = (rng.random((T, G)) * 0.02 + 0.005).astype(np.float32)
+    ws = (rng.random((E, G, C)) * 0.002 + 0.0005).astype(np.float32)
+    bias = (rng.standard_normal((E, N)) * 0.1).astype(np.float32) if T % 4 == 0 else None
+    xsp = torch.full((T, G + 3), float("nan"), dtype=torch.float32, device="cuda")
+    xsp[:, :G] = dev_f32(xs)
+    Y = hkq.moe_a8w8_blockscale(dev_u8(X), dev_u8(W), dev_i32(hist), dev_i32(offs), dev_i32(ed), topk, xsp[:, :G],
+                                dev_f32(ws), gk, 128, gather=dev_i32(gather),
+                                bias=dev_f32(bias) if bias is not None else None)
+    torch.cuda.synchronize()
+    check_rows(orc, host_bf16_f32(Y), orc.moe_blockscale_ref(X, W, xs, ws, bias, gather, hist, offs, ed, topk, gk, 128))
+
+
 # N-contiguous [E, K, N] weights through both block-scale kernels (the 8-wave
 # one for group_k = 128 * 2^j, the 64-wide one otherwise), read in place: the
 # same bits as the K-contiguous weights, ragged N and padded rows of K
