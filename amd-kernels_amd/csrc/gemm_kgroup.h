@@ -90,7 +90,8 @@ struct KgSrc {
     uint32_t s_off[Cfg::PW > 0 ? Cfg::PW : 1], c_off[Cfg::LC > 0 ? Cfg::LC : 1];
     uint32_t bs_step;
     int sc_shift;
-    int KT;  // K-tiles
+    int KT;       // K-tiles
+    int rot = 0;  // the first one's index (kg_rotation); the order wraps at KT
     // the last K-tile holds 64 bytes of K per row (linear operands): the lanes
     // that carry its upper four chunks read nothing, so the LDS holds zeros there
     bool half_tail = false;
@@ -109,6 +110,22 @@ __device__ __forceinline__ uint32_t kg_chunk(int r, int lane) { return (uint32_t
 template <class Cfg>
 __device__ __forceinline__ int kg_piece_row(int q, int lane) { return Cfg::FP4 ? q * 32 + (lane >> 1) : q * 64 + lane; }
 __device__ __forceinline__ uint32_t kg_piece_half(int lane) { return (uint32_t)((lane & 1) ^ ((lane >> 4) & 1)) * 16u; }
+
+// K-tile that column tile `tile` starts at, for weights that stream from HBM.
+// Where rows lie a multiple of 4 KiB apart, one K-tile of every row falls on
+// the same few memory channels, and workgroups that start together walk
+// through them together: eight K-tiles (1 KiB) between neighbouring column
+// tiles spread them out. Measured on MI355X (A8W8 gate/up, 8 experts, rows of
+// 4096 bytes, 90 tokens: us without and with it): 64 x 128 tiles 208 -> 177,
+// 128 x 128 213 -> 181, 128 x 256 231 -> 200, 32 x 64 with three K groups,
+// which start apart anyway, 176 -> 174; 4 or 12 K-tiles apart give 182 and 179,
+// 1 gives 191. Rows of 14336 bytes lose 2 % (83 -> 85), rows of 2048 bytes gain
+// nothing, and a dense weight that the last-level cache holds neither (4096 x
+// 4096 bf16, 64 rows: 9.0 -> 9.3): those keep one order. A scale block holds 4
+// << sc_shift K-tiles and starts at a multiple of that.
+static __device__ __forceinline__ int kg_rotation(int64_t stride, int KT, int tile, int sc_shift) {
+    return stride % 4096 == 0 && KT % 8 == 0 && sc_shift <= 1 ? tile * 8 % KT : 0;
+}
 
 // lds_load16 / lds_load4 with a prepared descriptor and a wave-uniform offset
 // (measured on MI355X: the buffer's range check is per dword and includes it)
@@ -153,15 +170,19 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
         for (int i = 0; i < Cfg::SWP; ++i)
             upper[i] = KT::load_chunk(lane, kg_row<Cfg>(i, wg, lane)) >= 4 ? OOB : 0u;
     }
-    // the loads of round t (K-tile k0 + t); past the group's last they read
+    auto at = [&](int t) {
+        const int kt = k0 + t + src.rot;
+        return kt >= src.KT ? kt - src.KT : kt;
+    };
+    // the loads of round t (K-tile at(t)); past the group's last they read
     // nothing. A scale block goes out before the first K-tile that uses it, so
     // the wait for that K-tile covers it; the waits count operand loads only.
     auto issue_scales = [&](int t) {
         if constexpr (Cfg::PIECES > 0) {
             const int kt = k0 + t, c = kt >> src.sc_shift;
             if (t < mine && (t == 0 || ((c & (Cfg::SBK - 1)) == 0 && (c << src.sc_shift) == kt))) {
-                const uint32_t blk = (uint32_t)c / Cfg::SBK;
-                HKQ_LDS uint8_t* sl = sblk + (blk & 1) * Cfg::SBLK;
+                const uint32_t blk = (uint32_t)(at(t) >> src.sc_shift) / Cfg::SBK;
+                HKQ_LDS uint8_t* sl = sblk + (c / Cfg::SBK & 1) * Cfg::SBLK;
 #pragma unroll
                 for (int i = 0; i < Cfg::PW; ++i) {
                     const int q = i * GW + wg;
@@ -173,7 +194,7 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
         }
     };
     auto issue_piece = [&](int t, int stage, int idx) {
-        const int kt = k0 + t;
+        const int kt = at(t);
         const bool live = t < mine;
         HKQ_LDS uint8_t* st = gbase + stage * STAGE;
         const uint32_t kb = live ? (uint32_t)kt * 128u : OOB;
@@ -236,7 +257,7 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
             for (int q = 0; q < 2; ++q) (isb ? f.b[isb ? i : 0] : f.a[isb ? 0 : i])[ks][q] = lds_read16(base + lo[ks][q]);
         // the scales of a round past the group's last one are stale, those of a
         // half last K-tile's upper blocks the next row's: zeros
-        const bool live = t < mine && !(FP4 && src.half_tail && k0 + t == src.KT - 1 && khalf);
+        const bool live = t < mine && !(FP4 && src.half_tail && at(t) == src.KT - 1 && khalf);
         if constexpr (FP4) {
             const int kt = k0 + t;
             const HKQ_LDS uint8_t* sl = sblk + ((kt / Cfg::SBK) & 1) * Cfg::SBLK + r * 32 +
@@ -419,25 +440,34 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
 }
 
 // Tile of a grouped (MoE) GEMM whose experts hold `routed` rows in all, by the
-// mean rows per expert (the counts themselves are on the GPU): a tile's rows
-// should hold an expert's few rows once, and its columns keep the weights of
-// two workgroups per CU in flight. Beyond one routing block per expert the
-// block-pair kernels read the weights once for 256 rows and win. Measured on
-// MI355X, block-scale layers (gate/up and down together; 8 experts of 4096 x
-// 14336, top-2, tokens: us for the four tiles in order, then the pair kernel):
-// 24: 269 / 301 / 317 / 385 / 441; 90: 290 / 316 / 329 / 394 / 456; 150: 456 /
-// 324 / 342 / 403 / 469; 350: 741 / 519 / 376 / 420 / 505; 512: 977 / 631 /
-// 507 / 446 / 530; 1200: - / 1008 / 852 / 743 / 685. With a short K the wider
-// tile's fewer workgroups win earlier, and the pairs too (32 experts of 2048 x
-// 2816, top-4: 512: 261 / 189 / 175 / 169 / 183; 800: - / 233 / 188 / 178 /
-// 197; 1000: 212 on 128 x 256 against 208).
+// mean rows per expert r (the counts themselves are on the GPU): a tile's rows
+// should hold an expert's rows once, also where routing is skewed, and its
+// columns keep the weights of two workgroups per CU in flight. Beyond about one
+// routing block per expert (`pairs_short`, `pairs_long` rows, for K up to 3072
+// and above) the block-pair kernels read the weights once for 256 rows and win.
+// Measured on MI355X (us, gate/up and down together; 32 x 64, 64 x 128, 128 x
+// 128, 128 x 256, pairs), block-scale, 8 experts of 4096 x 14336: r = 2: 226 /
+// 236 / 257 / 322 / 392; 16: 259 / 250 / 272 / 337 / 415; 55: 461 / 261 / 293 /
+// 340 / 440; 75: 629 / 452 / 306 / 343 / 452; 105: 828 / 471 / 324 / 344 / 469;
+// 225: - / 784 / 613 / 530 / 561; 350: - / - / 879 / 740 / 702. A short K has
+// too few rounds to fill 8 waves' rings, and 128 x 256 comes before 128 x 128
+// (32 experts of 2048 x 2816, r = 25: 124 / 111 / 134 / 132 / 138; 80: 273 /
+// 193 / 150 / 138 / 152; 125: - / 236 / 196 / 177 / 169).
+// Where 128-column tiles of the experts that can hold a row would not give every
+// CU one, the narrow tile goes on whatever K is (one token's down projection, 4
+// live experts, N 2048, K 2816: 14.9 us on 32 x 128, 10.2 on 32 x 64).
+constexpr int MOE_CUS = 256;
+inline bool moe_few_tiles(int64_t routed, int64_t experts, int64_t N) {
+    return std::min(routed, experts) * ((N + 127) / 128) < MOE_CUS;
+}
 enum MoeTile { MOET_32x64, MOET_64x128, MOET_128x128, MOET_128x256, MOET_PAIRS };
-inline MoeTile moe_tile(int64_t routed, int64_t experts, int64_t K) {
+inline MoeTile moe_tile(int64_t routed, int64_t experts, int64_t N, int64_t K, int64_t pairs_short, int64_t pairs_long) {
     const int64_t r = routed / (experts > 0 ? experts : 1);
-    if (r <= 22) return MOET_32x64;
-    if (r <= 48) return MOET_64x128;
-    if (K <= 3072) return r <= 112 ? MOET_128x256 : MOET_PAIRS;
-    return r <= 96 ? MOET_128x128 : r <= 128 ? MOET_128x256 : MOET_PAIRS;
+    if (r <= 14 && moe_few_tiles(routed, experts, N)) return MOET_32x64;
+    if (K <= 3072) return r <= 56 ? MOET_64x128 : r <= pairs_short ? MOET_128x256 : MOET_PAIRS;
+    if (r <= 14) return MOET_32x64;
+    if (r <= 56) return MOET_64x128;
+    return r <= 112 ? MOET_128x128 : r <= pairs_long ? MOET_128x256 : MOET_PAIRS;
 }
 
 }  // namespace hkq

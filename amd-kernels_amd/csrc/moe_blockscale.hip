@@ -603,6 +603,7 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_bs
     KgSrc<Cfg, true> src;
     src.KT = p.K / 128;
     src.sc_shift = 31 - __builtin_clz(p.gk / 128);
+    src.rot = kg_rotation(p.swn, src.KT, tn, src.sc_shift);
     src.a = buffer_desc(p.X, clamp_bytes((int64_t)p.T * p.sxm));
     src.b = buffer_desc(p.W + (int64_t)e * p.swe + (int64_t)n0 * p.swn, clamp_bytes((int64_t)rows_b * p.swn));
     src.as = buffer_desc(p.xs, clamp_bytes(p.xs_elems * 4));
@@ -786,7 +787,7 @@ static int moe_blockscale_impl(const void* X, const void* W, void* Y, const floa
         // weights, one column scale per 32 columns, K-contiguous row scales)
         if (ntile && !wt && xs_stride_k == 1) {
             constexpr int B = MODE_BLOCKSCALE;
-            switch (moe_tile(gather ? T * topk : T, E, K)) {
+            switch (moe_tile(gather ? T * topk : T, E, N, K, 112, 256)) {
                 case MOET_32x64: return launch_moe_bs_tile<KgCfg<B, 1, 1, 3, 1, 2, 2>, 2>(p, stream);
                 case MOET_64x128: return launch_moe_bs_tile<KgCfg<B, 2, 2, 1, 1, 2, 3>, 2>(p, stream);
                 case MOET_128x128: return launch_moe_bs_tile<KgCfg<B, 4, 2, 1, 1, 2, 4>, 1>(p, stream);
