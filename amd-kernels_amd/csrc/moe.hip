@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <cstdlib>
 
+#include "gemm_kgroup.h"
 #include "gemm_stream.h"
 #include "hkq_host.h"
 
@@ -271,8 +272,104 @@ __global__ __launch_bounds__(64 * MOE_WM * MOE_WN, 1) void moe_gemm_kernel(const
 }
 
 // ---------------------------------------------------------------------------
-// Decode-size MoE (at most 64 routed rows in all, so at most 64 per block):
-// the streaming layout of the dense GEMMs' narrow path. Workgroup u takes
+// Few rows per expert: small tiles (gemm_kgroup.h), a workgroup per routing word
+// and column tile, walking the block's rows BM at a time. What bounds it is the
+// weights' way from HBM: the tiles and the workgroups per CU are chosen for the
+// bytes in flight (measured on MI355X, 64 tokens on 8 experts of 4096 x 14336:
+// gate/up 203 -> 175 us, 5.4 TB/s; down 174 -> 83 us, 5.7 TB/s).
+template <class Cfg, int MINB>
+__global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_tile_kernel(const MoeParams p) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
+    HKQ_LDS uint8_t* smem = (HKQ_LDS uint8_t*)smem_raw;
+    constexpr int BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TMO = Cfg::TMO;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wg = wave % Cfg::GW, kg = wave / Cfg::GW;
+    const int pm = blockIdx.x / p.tiles_n, tn = blockIdx.x % p.tiles_n;
+    const int ed = p.expt_data[pm];
+    const int e = ed & 0xFFFF, b = ed >> 16;
+    if (ed < 0 || e >= p.E) return;  // uniform: -1 or a malformed entry
+    const int m_e = p.hist[e], start = p.offs[e];
+    const int first = b * MOE_BM, rows = min(m_e - first, MOE_BM);
+    if (rows <= 0 || start < 0) return;
+    const int n0 = tn * BN;
+    const int rows_b = min(p.N - n0, BN);
+
+    KgSrc<Cfg, true> src;
+    src.KT = p.K / 128;
+    src.rot = kg_rotation(p.swn, src.KT, tn, 0);
+    src.sc_shift = 0;
+    src.bs_step = 0;
+    src.a = buffer_desc(p.X, clamp_bytes((int64_t)p.T * p.sxm));
+    src.b = buffer_desc(p.W + (int64_t)e * p.swe + (int64_t)n0 * p.swn, clamp_bytes((int64_t)rows_b * p.swn));
+    src.b_step = (uint32_t)(8 * Cfg::GW * Cfg::SWP * p.swn);
+#pragma unroll
+    for (int i = 0; i < Cfg::SWP; ++i) {
+        const int r = kg_row<Cfg>(i, wg, lane);
+        src.b_off[i] = (uint32_t)(r * p.swn) + kg_chunk<Cfg>(r, lane);
+    }
+    const int nw = n0 + wg % Cfg::WN * TN * 32, mw = (wg / Cfg::WN * Cfg::TM + (Cfg::SPREAD ? kg * TMO : 0)) * 32;
+    for (int row0 = first; row0 < first + rows; row0 += BM) {
+        auto token_of = [&](int r) {
+            const int s = start + row0 + r;
+            if (row0 + r >= first + rows || s >= p.g_len) return -1;
+            const int t = p.gather ? div_recip(p.gather[s], p.rtopk) : s;
+            return (t >= 0 && t < p.T) ? t : -1;
+        };
+#pragma unroll
+        for (int i = 0; i < Cfg::LA; ++i) {
+            const int r = kg_row<Cfg>(i, wg, lane), t = token_of(r);
+            src.a_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.sxm + kg_chunk<Cfg>(r, lane);
+        }
+        float rs[TMO];
+#pragma unroll
+        for (int j = 0; j < TMO; ++j) {
+            const int t = p.xs ? token_of(mw + j * 32 + (lane & 31)) : -1;
+            rs[j] = !p.xs ? 1.0f : (t < 0 ? 0.0f : p.xs[(int64_t)t * p.xs_tok]);
+        }
+        v16f acc[TN][TMO];
+        kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
+        if (Cfg::SPREAD || kg == 0) {
+            const int s0 = start + row0;
+            const int out_rows = min(min(first + rows - row0, BM), p.y_rows - s0);
+            // no bias, column scales absent, one per expert or one per channel (the launcher checks)
+            auto col_scale4 = [&](int i, int g) {
+                const int n = nw + i * 32 + 8 * g + 4 * (lane >> 5);
+                if (!p.ws) return make_float4(1.f, 1.f, 1.f, 1.f);
+                if (n >= p.N) return make_float4(0.f, 0.f, 0.f, 0.f);
+                const float* w = p.ws + (int64_t)e * p.ws_e;
+                if (p.ws_n == 0) return make_float4(w[0], w[0], w[0], w[0]);
+                return *reinterpret_cast<const float4*>(w + n);
+            };
+            store_tile_bf16<TMO, TN>(acc, smem, Cfg::SPREAD ? wave : wg, lane, p.Y + (int64_t)s0 * p.sym, p.sym, out_rows,
+                                     p.N, mw, nw, p.c16 != 0, [&](int j) { return rs[j]; }, col_scale4, NoBias{});
+        }
+        __syncthreads();  // the staging is read: the next row group's loads may overwrite it
+    }
+}
+
+template <class Cfg, int MINB>
+static int launch_moe_tile(MoeParams& p, hipStream_t stream) {
+    static_assert(Cfg::LDS * MINB <= 160 * 1024, "LDS budget of a CDNA4 CU");
+    auto kern = moe_tile_kernel<Cfg, MINB>;
+    static bool attr_set = false;
+    if (!attr_set) {
+        hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS);
+        if (e != hipSuccess) {
+            set_error("hipFuncSetAttribute(MaxDynamicSharedMemorySize=%d) failed: %s", Cfg::LDS, hipGetErrorString(e));
+            return (int)e;
+        }
+        attr_set = true;
+    }
+    p.tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
+    if (p.grid_m == 0 || p.N == 0) return 0;
+    kern<<<dim3((unsigned)((int64_t)p.grid_m * p.tiles_n)), Cfg::THREADS, Cfg::LDS, stream>>>(p);
+    return hkq_launch_status();
+}
+
+// ---------------------------------------------------------------------------
+// Decode-size MoE (at most 64 routed rows in all, so at most 64 per block) with
+// few column tiles, a bias or grouped column scales: the streaming layout of the dense GEMMs' narrow path. Workgroup u takes
 // routing entry u / slices and the 16*NT columns of slice u % slices; its 4
 // waves split K and load fragments from memory straight into registers for
 // the 16x16x128 MFMA (lane l: row l % 16 of each 16-row group, bytes
@@ -974,8 +1071,127 @@ __global__ __launch_bounds__(64 * MOE_WM * MOE_WN, 1) void moe_mxfp4_kernel(cons
 }
 
 // ---------------------------------------------------------------------------
-// Decode-size MXFP4 MoE (at most 32 valid gate ids): the streaming layout of
-// the narrow GEMM. Workgroup u takes block u / slices and the 16*NT columns of
+// Few rows per expert: small tiles as in the A8W8 MoE, over one 128-entry block,
+// walking its entries BM at a time (row groups without a valid entry are
+// passed over: the sorted layout puts them last). Measured on MI355X (gate/up,
+// 8 experts, K 4096, N 28672): 24 tokens 111 -> 97 us (5.2 TB/s with the
+// scales), 300 126 -> 120.
+template <class Cfg, int MINB>
+__global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_fp4_tile_kernel(const MoeFp4Params p) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
+    HKQ_LDS uint8_t* smem = (HKQ_LDS uint8_t*)smem_raw;
+    constexpr int BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TMO = Cfg::TMO;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wg = wave % Cfg::GW, kg = wave / Cfg::GW;
+    const int pm = blockIdx.x / p.tiles_n, tn = blockIdx.x % p.tiles_n;
+    const int n0 = tn * BN;
+    const int32_t* ids = p.sorted + (int64_t)pm * MOE_BM;
+    const int e = p.expert[pm];
+    auto gate_of = [&](int r) {  // gate id of entry r of the block, -1: padding
+        const int id = ids[r];
+        return (id >= 0 && id < p.num_valid) ? id : -1;
+    };
+    if (e < 0 || e >= p.E) {
+        if (e == -1) {  // valid rows of an unassigned block are zeros
+            for (int r = wave; r < MOE_BM; r += Cfg::NW) {
+                const int id = gate_of(r);
+                if (id < 0) continue;
+                for (int n = n0 + lane * 4; n < min(p.N, n0 + BN); n += 256)
+                    *reinterpret_cast<v2i*>(p.C + (int64_t)id * p.scm + n) = v2i{0, 0};
+            }
+        }
+        return;
+    }
+    const int rows_b = min(p.N - n0, BN);
+    KgSrc<Cfg, true> src;
+    src.KT = p.K / 256;
+    src.sc_shift = 0;
+    src.bs_step = 0;
+    src.a = buffer_desc(p.A, clamp_bytes((int64_t)p.tokens * p.sam));
+    src.as = buffer_desc(p.As, clamp_bytes((int64_t)(p.tokens - 1) * p.sas + p.K / 32));
+    src.b = buffer_desc(p.B + (int64_t)e * p.sbe + (int64_t)n0 * p.sbn, clamp_bytes((int64_t)rows_b * p.sbn));
+    src.bs = buffer_desc(p.Bs + (int64_t)e * p.sbse + (int64_t)n0 * p.sbsn,
+                         clamp_bytes((int64_t)(rows_b - 1) * p.sbsn + p.K / 32));
+    src.b_step = (uint32_t)(8 * Cfg::GW * Cfg::SWP * p.sbn);
+#pragma unroll
+    for (int i = 0; i < Cfg::SWP; ++i) {
+        const int r = kg_row<Cfg>(i, wg, lane);
+        src.b_off[i] = (uint32_t)(r * p.sbn) + kg_chunk<Cfg>(r, lane);
+    }
+    const int nw = n0 + wg % Cfg::WN * TN * 32, mw = (wg / Cfg::WN * Cfg::TM + (Cfg::SPREAD ? kg * TMO : 0)) * 32;
+    const float gs = (p.a_scale ? p.a_scale[0] : 1.0f) * (p.b_scale ? p.b_scale[e] : 1.0f);
+    for (int row0 = 0; row0 < MOE_BM; row0 += BM) {
+        // uniform: every wave looks at the group's entries
+        int any = 0;
+        for (int r = lane; r < BM; r += 64) any |= gate_of(row0 + r) >= 0;
+        if (__ballot(any) == 0) continue;
+        auto arow_of = [&](int r) {
+            const int id = gate_of(row0 + r);
+            const int t = id < 0 ? -1 : div_recip(id, p.rtopk);
+            return t < p.tokens ? t : -1;
+        };
+#pragma unroll
+        for (int i = 0; i < Cfg::LA; ++i) {
+            const int r = kg_row<Cfg>(i, wg, lane), t = arow_of(r);
+            src.a_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.sam + kg_chunk<Cfg>(r, lane);
+        }
+#pragma unroll
+        for (int i = 0; i < Cfg::PW; ++i) {
+            const int q = i * Cfg::GW + wg;
+            if (q < Cfg::PA) {
+                const int t = arow_of(kg_piece_row<Cfg>(q, lane));
+                src.s_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.sas + kg_piece_half(lane);
+            } else {
+                src.s_off[i] = (uint32_t)(kg_piece_row<Cfg>(q - Cfg::PA, lane) * p.sbsn) + kg_piece_half(lane);
+            }
+        }
+        // the epilogue's gate ids (scatter rows) and routed weights, ahead of the K loop
+        int rid[(TMO * 32 + 63) / 64];
+#pragma unroll
+        for (int h = 0; h < (TMO * 32 + 63) / 64; ++h) {
+            const int r = h * 64 + lane;
+            rid[h] = r < TMO * 32 ? gate_of(row0 + mw + r) : -1;
+        }
+        float rs[TMO];
+#pragma unroll
+        for (int j = 0; j < TMO; ++j) {
+            const int id = gate_of(row0 + mw + j * 32 + (lane & 31));
+            rs[j] = (p.topk_w && id >= 0) ? gs * p.topk_w[id] : gs;
+        }
+        v16f acc[TN][TMO];
+        kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
+        if (Cfg::SPREAD || kg == 0)
+            store_tile_bf16_rows<TMO, TN>(
+                acc, smem, Cfg::SPREAD ? wave : wg, lane, p.C, p.scm, p.N, nw, p.c16 != 0,
+                [&](int r) { return (int64_t)__shfl(rid[TMO > 2 ? r >> 6 : 0], r & 63); }, [&](int j) { return rs[j]; },
+                [&](int, int) { return make_float4(1.f, 1.f, 1.f, 1.f); }, NoBias{});
+        __syncthreads();  // the staging is read: the next row group's loads may overwrite it
+    }
+}
+
+template <class Cfg, int MINB>
+static int launch_moe_fp4_tile(MoeFp4Params& p, hipStream_t stream) {
+    static_assert(Cfg::LDS * MINB <= 160 * 1024, "LDS budget of a CDNA4 CU");
+    auto kern = moe_fp4_tile_kernel<Cfg, MINB>;
+    static bool attr_set = false;
+    if (!attr_set) {
+        hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS);
+        if (err != hipSuccess) {
+            set_error("hipFuncSetAttribute(MaxDynamicSharedMemorySize=%d) failed: %s", Cfg::LDS, hipGetErrorString(err));
+            return (int)err;
+        }
+        attr_set = true;
+    }
+    p.tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
+    if (p.grid_m == 0 || p.N == 0) return 0;
+    kern<<<dim3((unsigned)((int64_t)p.grid_m * p.tiles_n)), Cfg::THREADS, Cfg::LDS, stream>>>(p);
+    return hkq_launch_status();
+}
+
+// ---------------------------------------------------------------------------
+// Decode-size MXFP4 MoE with K % 256 == 128 (at most 32 valid gate ids): the
+// streaming layout of the narrow GEMM. Workgroup u takes block u / slices and the 16*NT columns of
 // slice u % slices; for every 16-entry group of the block that holds a valid
 // gate id (with the sorted layout that is the first one or two groups) its 4
 // waves stream K through the 16x16x128 MFMA with per-lane e8m0 scales (lane l:
@@ -1189,15 +1405,40 @@ static int moe_a8w8_impl(const void* X, const void* W, void* Y, const float* x_s
                reinterpret_cast<uintptr_t>(w_scale) % 16 == 0;
     p.bias_vec = bias && bias_stride_e % 4 == 0 && reinterpret_cast<uintptr_t>(bias) % 16 == 0;
     p.c16 = (stride_ym % 8 == 0) && (reinterpret_cast<uintptr_t>(Y) % 16 == 0);
-    // Decode sizes take the streaming path: at most 32 routed rows, or 64 with
-    // N <= 4096 (measured: with 64 rows and N = 28672 the tiled kernel is 8%
-    // faster, at N = 4096 the streaming one 1.9x). The routed rows are the
-    // gathered (token, choice) pairs, T * topk, or the T sorted rows without
-    // a gather; every block then holds at most that many rows.
+    // The routed rows are the gathered (token, choice) pairs, T * topk, or the T
+    // sorted rows without a gather. Small tiles (moe_tile) take K-contiguous
+    // weights of whole K-tiles and scales they read as they are stored: none,
+    // one per expert or one float4-readable value per channel. Measured on
+    // MI355X (us, gate/up and down; this kernel against the streaming and
+    // block-pair ones): 8 experts of 4096 x 14336, 8 tokens 233 / 251, 90: 259 /
+    // 383, 300: 284 / 504, 640: 379 / 430, 1400: 632 / 744, 2048: 858 / 823; 32
+    // of 2048 x 2816, 8 tokens 71 / 98, 350: 116 / 154, 1000: 164 / 188, 1400:
+    // 209 / 165. With a short K and up to 12 rows per expert 32 x 128 tiles on
+    // three workgroups per CU win (64 tokens, 32 experts: 105 against 110; a
+    // long K leaves the down projection too few of them: 106 against 83). Decode
+    // sizes with fewer column tiles than CUs keep the streaming kernel (one
+    // token's layer, 8 experts: 96.7 against 101.4).
     const int64_t routed = gather ? T * topk : T;
-    const bool decode = routed <= 32 || (routed <= MOE_NARROW_MAX_ROWS && N <= 4096);
-    if (decode && !wt && K % 128 == 0 && 64 * stride_w < (1ll << 31))
-        return launch_moe_narrow(p, routed, stream);
+    const bool few = moe_few_tiles(routed, E, N);
+    const bool decode = (routed <= 32 || (routed <= MOE_NARROW_MAX_ROWS && N <= 4096)) && !wt && K % 128 == 0 &&
+                        64 * stride_w < (1ll << 31);
+    if (!(few && decode) && !wt && K % 128 == 0 && !bias && (!w_scale || ws_stride_n == 0 || p.ws_vec) &&
+        256 * stride_w < (1ll << 31)) {
+        constexpr int B = MODE_A8W8;
+        if (K <= 3072 && !few && routed <= 12 * E) return launch_moe_tile<KgCfg<B, 1, 4, 1, 1, 1, 2>, 3>(p, stream);
+        switch (moe_tile(routed, E, N, K, 128, 352)) {
+            case MOET_32x64: return launch_moe_tile<KgCfg<B, 1, 1, 3, 1, 2, 2>, 2>(p, stream);
+            case MOET_64x128: return launch_moe_tile<KgCfg<B, 2, 2, 1, 1, 2, 3>, 2>(p, stream);
+            case MOET_128x128: return launch_moe_tile<KgCfg<B, 4, 2, 1, 1, 2, 4>, 1>(p, stream);
+            case MOET_128x256: return launch_moe_tile<KgCfg<B, 2, 4, 1, 2, 2, 3>, 1>(p, stream);
+            case MOET_PAIRS: break;
+        }
+    }
+    // Decode sizes (those with a bias or grouped column scales whatever the
+    // column tiles) take the streaming path: at most 32 routed rows, or 64 with
+    // N <= 4096 (measured: with 64 rows and N = 28672 the tiled kernel is 8%
+    // faster, at N = 4096 the streaming one 1.9x).
+    if (decode) return launch_moe_narrow(p, routed, stream);
     // 128-byte K-tiles (2-stage ring) when every row has whole ones: a partial
     // last K-tile would read the next row's bytes instead of zeros
     return K % 128 == 0 ? launch_moe<128, 2>(p, stream) : launch_moe<64, 4>(p, stream);
@@ -1293,12 +1534,35 @@ static int moe_mxfp4_impl(const void* A, const void* B, void* C, const void* A_m
     p.sbsn = stride_bmxn; p.scm = stride_cm;
     p.wt = wt;
     p.c16 = (stride_cm % 8 == 0) && (reinterpret_cast<uintptr_t>(C) % 16 == 0);
-    // The streaming path when the tiled grid would give fewer than a quarter
-    // of the CUs work and there are at most 32 valid gate ids (measured: one
-    // token's down projection, N = 4096, 56 -> 22 us; with N = 28672 or eight
-    // tokens the tiled kernel is faster). Its scale loads are dwords, and 64
-    // weight rows must span less than 2 GiB.
     const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
+    // Small tiles by the mean valid entries per expert r, as in the A8W8 MoE
+    // (moe_tile) but with the tiles that 4-bit rows and their scale blocks leave
+    // room for. They read whole 256-element K-tiles and 16 scale bytes at a
+    // time at dword offsets. Measured on MI355X (us, gate/up of 8 experts, K
+    // 4096, N 28672; 32 x 128, 64 x 128, 128 x 128, block pairs): r = 6: 97 / 98 /
+    // 110 / 111; 22: 99 / 104 / 111 / 118; 37: 161 / 104 / 113 / 118; 75: 249 /
+    // 183 / 120 / 126; 105: - / - / 125 / 131; 128: - / - / - / 150 (pairs win); 32
+    // experts, K 2048, N 5632: r = 3: 41 / 46 / 51 / 51; 18: 42 / 47 / 52 / 52;
+    // 43: - / 48 / 54 / 54; 64: - / - / 58 / 57. Where 32 x 128 tiles over the live
+    // blocks would not give every CU work, 32 x 32 tiles with K in four: one
+    // token's down projection (K 14336, N 4096) 36 -> 13 us, 8 tokens' 60 -> 46
+    // (the streaming kernel below 21, the pairs 81); with a short K from half
+    // the CUs (N 2048, K 2816: 128 workgroups 11.0 -> 9.4, 256 12.0 -> 14.6).
+    const int64_t r = num_valid_tokens / num_experts, live = std::min(grid_m, num_valid_tokens);
+    if (!wt && K % 256 == 0 && stride_amxm % 4 == 0 && stride_bmxn % 4 == 0 && stride_bmxe % 4 == 0 &&
+        256 * stride_bn < (1ll << 31) && 256 * stride_bmxn < (1ll << 31)) {
+        constexpr int B = MODE_MXFP4;
+        if (r <= 20 && live * ((N + 127) / 128) <= (K > 3072 ? ncu : ncu / 2))
+            return launch_moe_fp4_tile<KgCfg<B, 1, 1, 4, 1, 1, 2>, 2>(p, stream);
+        if (r <= 20) return launch_moe_fp4_tile<KgCfg<B, 1, 4, 1, 1, 1, 2>, 3>(p, stream);
+        if (r <= 56) return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 1, 2, 2>, 2>(p, stream);
+        if (r <= 112 && K > 3072) return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 2, 2, 2>, 2>(p, stream);
+    }
+    // K % 256 == 128 or scales at odd strides: the streaming path when the tiled
+    // grid would give fewer than a quarter of the CUs work and there are at most
+    // 32 valid gate ids (measured: one token's down projection, N = 4096, 56 ->
+    // 22 us; with N = 28672 or eight tokens the tiled kernel is faster). Its
+    // scale loads are dwords, and 64 weight rows must span less than 2 GiB.
     const bool few_tiles = ((grid_m + 1) / 2) * ((N + MOE_BN - 1) / MOE_BN) * 4 < ncu;
     if (!wt && few_tiles && num_valid_tokens <= MOE_FP4_NARROW_MAX_VALID && stride_amxm % 4 == 0 && stride_bmxn % 4 == 0 &&
         stride_bmxe % 4 == 0 && reinterpret_cast<uintptr_t>(A_mx_scale) % 4 == 0 &&

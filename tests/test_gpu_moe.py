@@ -432,15 +432,47 @@ def test_moe_blockscale(orc, T, E, topk, K, N, gk, gn):
     check_rows(orc, Y, ref)
 
 
-# Few rows per expert: the small tiles by mean rows per expert (10, 33, 75 and
-# 115: 32x64, 64x128, then 128x256 or, from K = 3200, 128x128, then block
-# pairs), routing skewed so that some experts
-# hold several row groups or blocks and some no row, odd counts of K-tiles, one
-# or two K-tiles per scale group, ragged N, a bias, -1 / malformed words between
-# the live ones and scale rows padded with NaN.
+# The A8W8 small tiles by mean rows per expert (K up to 3072: 10 on 32x64, or
+# 32x128 with N = 4100, 33 on 64x128, 75 on 128x256; above: 5 on 32x64, 32 on 64x128, 76 on
+# 128x128, 150 on 128x256), routing skewed so that some experts hold several row
+# groups or blocks and some no row, odd counts of K-tiles, rows of 4096 bytes
+# (column tiles start at different K-tiles), ragged N, every scale form, -1 /
+# malformed words between the live ones.
+@pytest.mark.parametrize("T,E,topk,K,N,scales", [
+    (3, 8, 2, 128, 1000, "none"), (40, 8, 2, 640, 300, "channel"), (40, 8, 2, 640, 4100, "expert"), (100, 6, 2, 1152, 260, "expert"),
+    (150, 4, 2, 896, 772, "channel"), (20, 8, 2, 4096, 260, "channel"), (130, 8, 2, 4096, 388, "expert"),
+    (230, 6, 2, 4096, 260, "channel"), (300, 4, 2, 3200, 516, "none")])
+def test_moe_small_tiles(orc, T, E, topk, K, N, scales):
+    require_gpu()
+
+    def skewed(rng, T, E, topk):
+        p = np.array([6.0] + [1.0] * (E - 2) + [0.0])
+        return np.stack([rng.choice(E, size=topk, replace=False, p=p / p.sum()) for _ in range(T)])
+
+    _, hist, offs, gather, ed, X, xs, W, ws = make_problem(orc, T, E, topk, K, N, T + N, skewed)
+    words = np.concatenate([[-1, E + 3], ed, [-1]]).astype(np.int32)
+    if scales == "none":  # codes below 2: sums of the size the absolute bound is meant for
+        X, W = X & 0xBF, W & 0xBF
+    xs, ws = {"none": (None, None), "channel": (xs, ws), "expert": (xs, ws[:, 0].copy())}[scales]
+    Y = run_moe(X, W, hist, offs, gather, words, topk, xs=xs, ws=ws)
+    xs, ws = (1.0, np.ones(E)) if xs is None else (xs, ws)
+    check_rows(orc, Y, orc.moe_ref(X, W, xs, ws, None, gather, hist, offs, ed, topk, 128, "enk"))
+
+
+# Few rows per expert: the small tiles by mean rows per expert (K up to 3072: 0
+# and 10 on 32x64, 33 on 64x128, 75 on 128x256, 115 on block pairs; above: 4 on 32x64, 25
+# on 64x128, 75 on 128x128, 150 on 128x256), routing skewed so that some experts
+# hold several row groups or blocks and some no row, odd counts of K-tiles, rows
+# a multiple of 4 KiB apart (column tiles start at different K-tiles; with four
+# K-tiles per scale group they don't), one to four K-tiles per scale group,
+# ragged N, a bias, -1 / malformed words between the live ones and scale rows
+# padded with NaN.
 @pytest.mark.parametrize("T,E,topk,K,N,gk", [(40, 8, 2, 640, 300, 128), (3, 8, 2, 128, 1000, 128),
                                              (100, 6, 2, 1152, 260, 128), (150, 4, 2, 896, 772, 256),
-                                             (150, 4, 2, 3200, 132, 128), (230, 4, 2, 640, 1028, 128)])
+                                             (150, 4, 2, 3200, 132, 128), (230, 4, 2, 640, 1028, 128),
+                                             (12, 6, 2, 4096, 260, 128), (100, 8, 2, 4096, 388, 256),
+                                             (100, 8, 2, 4096, 260, 512), (152, 4, 2, 4096, 260, 128),
+                                             (300, 4, 2, 4096, 516, 128)])
 def test_moe_blockscale_small_tiles(orc, T, E, topk, K, N, gk):
     require_gpu()
 

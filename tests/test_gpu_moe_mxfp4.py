@@ -117,6 +117,46 @@ def test_moe_mxfp4_decode_layouts(orc):
     assert np.all(got[[4, 5]] == 0.0) and np.all(got[nv:] == 7.0)
 
 
+# The small tiles by mean valid entries per expert and by workgroups (1 and 10 on
+# 32x32 with K in four, 3 on 32x128, 33 on 64x128, 75 on 128x128 from K = 3328),
+# routing skewed so that some experts hold several row groups or blocks, odd
+# counts of K-tiles, ragged N, routed weights, padded scale rows, a block whose
+# entries are scattered over its 128, one of expert -1 (zeros for its valid
+# rows) and one past the last expert (left untouched).
+@pytest.mark.parametrize("T,E,topk,K,N", [(4, 8, 2, 256, 260), (40, 8, 2, 4352, 132), (96, 64, 2, 768, 516),
+                                          (100, 6, 2, 1280, 260), (150, 4, 2, 3328, 388)])
+def test_moe_mxfp4_small_tiles(orc, T, E, topk, K, N):
+    require_gpu()
+    Aq, As, Bq, Bs = problem(orc, T, E, K, N, T + K)
+    rng = np.random.default_rng(T)
+    p = np.array([6.0] + [1.0] * (E - 1)) / (E + 5.0)
+    ids = np.stack([rng.choice(E, size=topk, replace=False, p=p) for _ in range(T)]).astype(np.int32).ravel()
+    s, eids, _, _ = orc.align_block_size(ids, E, 128)
+    s, eids, nv = s.copy(), eids.copy(), T * topk
+    s[:128] = rng.permutation(s[:128])
+    eids[-1], eids[-2] = -1, E + 1
+    w = rng.random(nv).astype(np.float32)
+
+    def padded(x):
+        t = torch.full((*x.shape[:-1], x.shape[-1] + 4), 255, dtype=torch.uint8, device="cuda")
+        t[..., :x.shape[-1]] = dev_u8(x)
+        return t[..., :x.shape[-1]]
+
+    C = torch.full((nv, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    hkq.moe_mxfp4(dev_u8(Aq), padded(As), dev_u8(Bq), padded(Bs), dev_i32(s), dev_i32(eids), nv, topk,
+                  topk_weights=dev_f32(w), C=C)
+    torch.cuda.synchronize()
+    keep = np.concatenate([eids[:-2], eids[-1:]])
+    rows = np.concatenate([s[:-256], s[-128:]])
+    ref = orc.moe_mxfp4_ref(Aq, As, Bq, Bs, None, None, w, rows, keep, N, nv, topk, True, nv)
+    got = C.float().cpu().numpy()
+    written = ~np.isnan(ref).any(axis=1)
+    assert_gemm_close(got[written], ref[written], "moe mxfp4 small tiles")
+    assert (~written).any() and np.all(got[~written] == 7.0)
+    zero = s[-128:][s[-128:] < nv]
+    assert len(zero) and np.all(got[zero] == 0.0)
+
+
 def test_moe_mxfp4_module_reference_call(orc):
     """tests/test_moe.py:902-936 of the reference, argument list unchanged:
     random E2M1 bytes and e8m0 scales in [120, 134), B [E, K/2, N] and B_mx_scale
