@@ -369,7 +369,8 @@ static int launch_moe_tile(MoeParams& p, hipStream_t stream) {
 
 // ---------------------------------------------------------------------------
 // Decode-size MoE (at most 64 routed rows in all, so at most 64 per block) with
-// few column tiles, a bias or grouped column scales: the streaming layout of the dense GEMMs' narrow path. Workgroup u takes
+// few column tiles, a bias or grouped column scales: the streaming layout of
+// the dense GEMMs' narrow path. Workgroup u takes
 // routing entry u / slices and the 16*NT columns of slice u % slices; its 4
 // waves split K and load fragments from memory straight into registers for
 // the 16x16x128 MFMA (lane l: row l % 16 of each 16-row group, bytes
@@ -1191,7 +1192,8 @@ static int launch_moe_fp4_tile(MoeFp4Params& p, hipStream_t stream) {
 
 // ---------------------------------------------------------------------------
 // Decode-size MXFP4 MoE with K % 256 == 128 (at most 32 valid gate ids): the
-// streaming layout of the narrow GEMM. Workgroup u takes block u / slices and the 16*NT columns of
+// streaming layout of the narrow GEMM. Workgroup u takes block u / slices and
+// the 16*NT columns of
 // slice u % slices; for every 16-entry group of the block that holds a valid
 // gate id (with the sorted layout that is the first one or two groups) its 4
 // waves stream K through the 16x16x128 MFMA with per-lane e8m0 scales (lane l:
