@@ -1,6 +1,6 @@
 // gemm_kgroup.h -- the K loop of the small-tile GEMMs: workgroups of KG groups
 // of waves, each group computing the whole BM x BN tile over its own K-tiles
-// (group g takes K-tiles g, g + KG, ...), the groups' sums added through LDS at
+// (group g takes a contiguous share), the groups' sums added through LDS at
 // the end.
 //
 // What it is for: few rows (or few tiles), where the time is the weights'
@@ -91,7 +91,6 @@ struct KgSrc {
     uint32_t bs_step;
     int sc_shift;
     int KT;       // K-tiles
-    int rot = 0;  // the first one's index (kg_rotation); the order wraps at KT
     // the last K-tile holds 64 bytes of K per row (linear operands): the lanes
     // that carry its upper four chunks read nothing, so the LDS holds zeros there
     bool half_tail = false;
@@ -110,22 +109,6 @@ __device__ __forceinline__ uint32_t kg_chunk(int r, int lane) { return (uint32_t
 template <class Cfg>
 __device__ __forceinline__ int kg_piece_row(int q, int lane) { return Cfg::FP4 ? q * 32 + (lane >> 1) : q * 64 + lane; }
 __device__ __forceinline__ uint32_t kg_piece_half(int lane) { return (uint32_t)((lane & 1) ^ ((lane >> 4) & 1)) * 16u; }
-
-// K-tile that column tile `tile` starts at, for weights that stream from HBM.
-// Where rows lie a multiple of 4 KiB apart, one K-tile of every row falls on
-// the same few memory channels, and workgroups that start together walk
-// through them together: eight K-tiles (1 KiB) between neighbouring column
-// tiles spread them out. Measured on MI355X (A8W8 gate/up, 8 experts, rows of
-// 4096 bytes, 90 tokens: us without and with it): 64 x 128 tiles 208 -> 177,
-// 128 x 128 213 -> 181, 128 x 256 231 -> 200, 32 x 64 with three K groups,
-// which start apart anyway, 176 -> 174; 4 or 12 K-tiles apart give 182 and 179,
-// 1 gives 191. Rows of 14336 bytes lose 2 % (83 -> 85), rows of 2048 bytes gain
-// nothing, and a dense weight that the last-level cache holds neither (4096 x
-// 4096 bf16, 64 rows: 9.0 -> 9.3): those keep one order. A scale block holds 4
-// << sc_shift K-tiles and starts at a multiple of that.
-static __device__ __forceinline__ int kg_rotation(int64_t stride, int KT, int tile, int sc_shift) {
-    return stride % 4096 == 0 && KT % 8 == 0 && sc_shift <= 1 ? tile * 8 % KT : 0;
-}
 
 // lds_load16 / lds_load4 with a prepared descriptor and a wave-uniform offset
 // (measured on MI355X: the buffer's range check is per dword and includes it)
@@ -170,20 +153,14 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
         for (int i = 0; i < Cfg::SWP; ++i)
             upper[i] = KT::load_chunk(lane, kg_row<Cfg>(i, wg, lane)) >= 4 ? OOB : 0u;
     }
-    // (GATHER only: the wrap's compare and select cost the linear operands' short
-    // loops 4 to 6 %, 601 x 6144 x 4096 A8W8 and 500 x 7168 x 2048 block-scale)
-    auto at = [&](int t) {
-        const int kt = k0 + t + (GATHER ? src.rot : 0);
-        return GATHER && kt >= src.KT ? kt - src.KT : kt;
-    };
-    // the loads of round t (K-tile at(t)); past the group's last they read
+    // the loads of round t (K-tile k0 + t); past the group's last they read
     // nothing. A scale block goes out before the first K-tile that uses it, so
     // the wait for that K-tile covers it; the waits count operand loads only.
     auto issue_scales = [&](int t) {
         if constexpr (Cfg::PIECES > 0) {
             const int kt = k0 + t, c = kt >> src.sc_shift;
             if (t < mine && (t == 0 || ((c & (Cfg::SBK - 1)) == 0 && (c << src.sc_shift) == kt))) {
-                const uint32_t blk = (uint32_t)(at(t) >> src.sc_shift) / Cfg::SBK;
+                const uint32_t blk = (uint32_t)c / Cfg::SBK;
                 HKQ_LDS uint8_t* sl = sblk + (c / Cfg::SBK & 1) * Cfg::SBLK;
 #pragma unroll
                 for (int i = 0; i < Cfg::PW; ++i) {
@@ -196,7 +173,7 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
         }
     };
     auto issue_piece = [&](int t, int stage, int idx) {
-        const int kt = at(t);
+        const int kt = k0 + t;
         const bool live = t < mine;
         HKQ_LDS uint8_t* st = gbase + stage * STAGE;
         const uint32_t kb = live ? (uint32_t)kt * 128u : OOB;
@@ -224,13 +201,14 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
         for (int i = 0; i < NLD; ++i) issue_piece(t, stage, i);
     };
 
-    // fragment addresses (as gemm_mainloop): lane half h owns chunks 4h .. 4h+3,
-    // K-step ks reads 4h + 2ks + {0, 1}
+    // fragment addresses: K-step ks of lane half h reads chunks 4h + 2ks + {0, 1}
+    // as in gemm_mainloop, block-scale 4ks + 2h + {0, 1} as in blockscale_core
+    // (an MFMA's own sum depends, in the last bit, on which 64 values it holds)
     uint32_t lo[2][2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-        for (int q = 0; q < 2; ++q) lo[ks][q] = (uint32_t)KT::swz(r, 4 * khalf + 2 * ks + q);
+        for (int q = 0; q < 2; ++q) lo[ks][q] = (uint32_t)KT::swz(r, BS ? 4 * ks + 2 * khalf + q : 4 * khalf + 2 * ks + q);
 
     v16f acc[TN][TM];
 #pragma unroll
@@ -259,7 +237,7 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
             for (int q = 0; q < 2; ++q) (isb ? f.b[isb ? i : 0] : f.a[isb ? 0 : i])[ks][q] = lds_read16(base + lo[ks][q]);
         // the scales of a round past the group's last one are stale, those of a
         // half last K-tile's upper blocks the next row's: zeros
-        const bool live = t < mine && !(FP4 && src.half_tail && at(t) == src.KT - 1 && khalf);
+        const bool live = t < mine && !(FP4 && src.half_tail && k0 + t == src.KT - 1 && khalf);
         if constexpr (FP4) {
             const int kt = k0 + t;
             const HKQ_LDS uint8_t* sl = sblk + ((kt / Cfg::SBK) & 1) * Cfg::SBLK + r * 32 +
@@ -442,33 +420,27 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
 }
 
 // Tile of a grouped (MoE) GEMM whose experts hold `routed` rows in all, by the
-// mean rows per expert r (the counts themselves are on the GPU): a tile's rows
-// should hold an expert's rows once, also where routing is skewed, and its
-// columns keep the weights of two workgroups per CU in flight. Beyond about one
-// routing block per expert (`pairs_short`, `pairs_long` rows, for K up to 3072
-// and above) the block-pair kernels read the weights once for 256 rows and win.
-// Measured on MI355X (us, gate/up and down together; 32 x 64, 64 x 128, 128 x
-// 128, 128 x 256, pairs), block-scale, 8 experts of 4096 x 14336: r = 2: 226 /
-// 236 / 257 / 322 / 392; 16: 259 / 250 / 272 / 337 / 415; 55: 461 / 261 / 293 /
-// 340 / 440; 75: 629 / 452 / 306 / 343 / 452; 105: 828 / 471 / 324 / 344 / 469;
-// 225: - / 784 / 613 / 530 / 561; 350: - / - / 879 / 740 / 702. A short K has
-// too few rounds to fill 8 waves' rings, and 128 x 256 comes before 128 x 128
-// (32 experts of 2048 x 2816, r = 25: 124 / 111 / 134 / 132 / 138; 80: 273 /
-// 193 / 150 / 138 / 152; 125: - / 236 / 196 / 177 / 169).
-// Where 128-column tiles of the experts that can hold a row would not give every
-// CU one, the narrow tile goes on whatever K is (one token's down projection, 4
-// live experts, N 2048, K 2816: 14.9 us on 32 x 128, 10.2 on 32 x 64).
-constexpr int MOE_CUS = 256;
-inline bool moe_few_tiles(int64_t routed, int64_t experts, int64_t N) {
-    return std::min(routed, experts) * ((N + 127) / 128) < MOE_CUS;
-}
-enum MoeTile { MOET_32x64, MOET_64x128, MOET_128x128, MOET_128x256, MOET_PAIRS };
-inline MoeTile moe_tile(int64_t routed, int64_t experts, int64_t N, int64_t K, int64_t pairs_short, int64_t pairs_long) {
+// mean rows per expert r (the counts themselves are on the GPU). The tiles of
+// the MoE kernels have one K group: they add K-tile after K-tile in K order, as
+// the block-pair kernels do, so every tile size and both weight layouts give
+// the same bits. Bound by the weights' way from HBM: a tile's rows should hold
+// an expert's rows, and the rings of the workgroups of a CU 120 to 150 KB of
+// K-tiles in flight. Beyond about one routing block per expert (`pairs_short`,
+// `pairs_long` rows, for K up to 3072 and above) the block-pair kernels read
+// the weights once for 256 rows and win.
+// Measured on MI355X (us, gate/up and down together), block-scale, 8 experts of
+// 4096 x 14336; 64 x 64 tiles on 4 waves, 64 x 128 on 8, 128 x 128, 128 x 256,
+// pairs: r = 0: 85 / 90 / 123 / 149 / 155; 2: 258 / 265 / 288 / 355 / 400; 16: 275
+// / 281 / 311 / 367 / 416; 37: 290 / 287 / 324 / 372 / 431; 55: 347 / 340 / 326 /
+// 375 / 441; 75: 489 / 462 / 349 / 386 / 459; 125: 593 / 611 / 470 / 425 / 494;
+// 225: 853 / 752 / 601 / 521 / 557. With a short K (32 experts of 2048 x 2816) the
+// wide tile's fewer, longer rows win: r = 1: 69 / 66 / 96 / 78 / 86; 12: 109 / 105 /
+// 140 / 129 / 131; 50: 124 / 123 / 146 / 136 / 140; 112: 219 / 206 / 178 / 160 / 160.
+enum MoeTile { MOET_64x64, MOET_64x128, MOET_128x128, MOET_128x256, MOET_PAIRS };
+inline MoeTile moe_tile(int64_t routed, int64_t experts, int64_t K, int64_t pairs_short, int64_t pairs_long) {
     const int64_t r = routed / (experts > 0 ? experts : 1);
-    if (r <= 14 && moe_few_tiles(routed, experts, N)) return MOET_32x64;
     if (K <= 3072) return r <= 56 ? MOET_64x128 : r <= pairs_short ? MOET_128x256 : MOET_PAIRS;
-    if (r <= 14) return MOET_32x64;
-    if (r <= 56) return MOET_64x128;
+    if (r <= 48) return MOET_64x64;
     return r <= 112 ? MOET_128x128 : r <= pairs_long ? MOET_128x256 : MOET_PAIRS;
 }
 

@@ -275,8 +275,9 @@ __global__ __launch_bounds__(64 * MOE_WM * MOE_WN, 1) void moe_gemm_kernel(const
 // Few rows per expert: small tiles (gemm_kgroup.h), a workgroup per routing word
 // and column tile, walking the block's rows BM at a time. What bounds it is the
 // weights' way from HBM: the tiles and the workgroups per CU are chosen for the
-// bytes in flight (measured on MI355X, 64 tokens on 8 experts of 4096 x 14336:
-// gate/up 203 -> 175 us, 5.4 TB/s; down 174 -> 83 us, 5.7 TB/s).
+// bytes in flight; K-tiles are added in K order, as in the block-pair kernels
+// (measured on MI355X, 64 tokens on 8 experts of 4096 x 14336: gate/up 199 -> 185
+// us, 5.1 TB/s; down 175 -> 83 us, 5.7 TB/s).
 template <class Cfg, int MINB>
 __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_tile_kernel(const MoeParams p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
@@ -297,7 +298,6 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_ti
 
     KgSrc<Cfg, true> src;
     src.KT = p.K / 128;
-    src.rot = kg_rotation(p.swn, src.KT, tn, 0);
     src.sc_shift = 0;
     src.bs_step = 0;
     src.a = buffer_desc(p.X, clamp_bytes((int64_t)p.T * p.sxm));
@@ -1411,26 +1411,24 @@ static int moe_a8w8_impl(const void* X, const void* W, void* Y, const float* x_s
     // sorted rows without a gather. Small tiles (moe_tile) take K-contiguous
     // weights of whole K-tiles and scales they read as they are stored: none,
     // one per expert or one float4-readable value per channel. Measured on
-    // MI355X (us, gate/up and down; this kernel against the streaming and
-    // block-pair ones): 8 experts of 4096 x 14336, 8 tokens 233 / 251, 90: 259 /
-    // 383, 300: 284 / 504, 640: 379 / 430, 1400: 632 / 744, 2048: 858 / 823; 32
-    // of 2048 x 2816, 8 tokens 71 / 98, 350: 116 / 154, 1000: 164 / 188, 1400:
-    // 209 / 165. With a short K and up to 12 rows per expert 32 x 128 tiles on
-    // three workgroups per CU win (64 tokens, 32 experts: 105 against 110; a
-    // long K leaves the down projection too few of them: 106 against 83). Decode
-    // sizes with fewer column tiles than CUs keep the streaming kernel (one
-    // token's layer, 8 experts: 96.7 against 101.4).
+    // MI355X (us, gate/up and down; the tile taken against the streaming and
+    // block-pair kernels): 8 experts of 4096 x 14336, 8 tokens 257 / 262, 24: 260 /
+    // 345, 64: 268 / 373, 150: 277 / 391, 300: 325 / 506, 500: 388 / 553, 900: 445 /
+    // 464, 1400: 653 / 753; 32 of 2048 x 2816, 8 tokens 64 / 97, 56: 101 / 129, 250:
+    // 107 / 135, 900: 142 / 176. Decode sizes with fewer column tiles than CUs keep
+    // the streaming kernel (one token's down projection, 8 experts: 22 against 38;
+    // 32 experts of 2048 x 2816, one token's layer 26 both).
     const int64_t routed = gather ? T * topk : T;
-    const bool few = moe_few_tiles(routed, E, N);
+    const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
+    const bool few = std::min(routed, E) * ((N + 127) / 128) < ncu;
     const bool decode = (routed <= 32 || (routed <= MOE_NARROW_MAX_ROWS && N <= 4096)) && !wt && K % 128 == 0 &&
                         64 * stride_w < (1ll << 31);
     if (!(few && decode) && !wt && K % 128 == 0 && !bias && (!w_scale || ws_stride_n == 0 || p.ws_vec) &&
         256 * stride_w < (1ll << 31)) {
         constexpr int B = MODE_A8W8;
-        if (K <= 3072 && !few && routed <= 12 * E) return launch_moe_tile<KgCfg<B, 1, 4, 1, 1, 1, 2>, 3>(p, stream);
-        switch (moe_tile(routed, E, N, K, 128, 352)) {
-            case MOET_32x64: return launch_moe_tile<KgCfg<B, 1, 1, 3, 1, 2, 2>, 2>(p, stream);
-            case MOET_64x128: return launch_moe_tile<KgCfg<B, 2, 2, 1, 1, 2, 3>, 2>(p, stream);
+        switch (moe_tile(routed, E, K, 128, 352)) {
+            case MOET_64x64: return launch_moe_tile<KgCfg<B, 2, 2, 1, 1, 1, 3>, 3>(p, stream);
+            case MOET_64x128: return launch_moe_tile<KgCfg<B, 2, 4, 1, 1, 1, 3>, 2>(p, stream);
             case MOET_128x128: return launch_moe_tile<KgCfg<B, 4, 2, 1, 1, 2, 4>, 1>(p, stream);
             case MOET_128x256: return launch_moe_tile<KgCfg<B, 2, 4, 1, 2, 2, 3>, 1>(p, stream);
             case MOET_PAIRS: break;
@@ -1540,33 +1538,32 @@ static int moe_mxfp4_impl(const void* A, const void* B, void* C, const void* A_m
     // Small tiles by the mean valid entries per expert r, as in the A8W8 MoE
     // (moe_tile) but with the tiles that 4-bit rows and their scale blocks leave
     // room for. They read whole 256-element K-tiles and 16 scale bytes at a
-    // time at dword offsets. Measured on MI355X (us, gate/up of 8 experts, K
-    // 4096, N 28672; 32 x 128, 64 x 128, 128 x 128, block pairs): r = 6: 97 / 98 /
-    // 110 / 111; 22: 99 / 104 / 111 / 118; 37: 161 / 104 / 113 / 118; 75: 249 /
-    // 183 / 120 / 126; 105: - / - / 125 / 131; 128: - / - / - / 150 (pairs win); 32
-    // experts, K 2048, N 5632: r = 3: 41 / 46 / 51 / 51; 18: 42 / 47 / 52 / 52;
-    // 43: - / 48 / 54 / 54; 64: - / - / 58 / 57. Where 32 x 128 tiles over the live
-    // blocks would not give every CU work, 32 x 32 tiles with K in four: one
-    // token's down projection (K 14336, N 4096) 36 -> 13 us, 8 tokens' 60 -> 46
-    // (the streaming kernel below 21, the pairs 81); with a short K from half
-    // the CUs (N 2048, K 2816: 128 workgroups 11.0 -> 9.4, 256 12.0 -> 14.6).
-    const int64_t r = num_valid_tokens / num_experts, live = std::min(grid_m, num_valid_tokens);
+    // time at dword offsets. Measured on MI355X (us, gate/up and down together,
+    // 8 experts of 4096 x 14336; 64 x 64, 64 x 128, 128 x 128, block pairs): r = 2:
+    // 136 / 140 / 165 / 164; 14: 142 / 144 / 170 / 178; 22: 146 / 147 / 172 / 184;
+    // 37: 160 / 158 / 184 / 182; 55: 198 / 188 / 177 / 188; 75: 275 / 273 / 181 /
+    // 196; 128: - / - / - / pairs win; 32 experts of 2048 x 2816: r = 1: 41 / 43 /
+    // 50 / 46; 7: 57 / 58 / 68 / 60; 37: 61 / 63 / 73 / 64.
+    // Where the tiled grid gives fewer than a quarter of the CUs work and at most
+    // 32 entries are valid, 32 x 32 tiles with K in four (one token's down
+    // projection, K 14336, N 4096: 14 us, streaming kernel 22, 64 x 64 tiles 33);
+    // everywhere else K-tiles are added in K order.
+    const int64_t r = num_valid_tokens / num_experts;
+    const bool few_tiles = ((grid_m + 1) / 2) * ((N + MOE_BN - 1) / MOE_BN) * 4 < ncu;
+    const bool decode = few_tiles && num_valid_tokens <= MOE_FP4_NARROW_MAX_VALID;
     if (!wt && K % 256 == 0 && stride_amxm % 4 == 0 && stride_bmxn % 4 == 0 && stride_bmxe % 4 == 0 &&
         256 * stride_bn < (1ll << 31) && 256 * stride_bmxn < (1ll << 31)) {
         constexpr int B = MODE_MXFP4;
-        if (r <= 20 && live * ((N + 127) / 128) <= (K > 3072 ? ncu : ncu / 2))
-            return launch_moe_fp4_tile<KgCfg<B, 1, 1, 4, 1, 1, 2>, 2>(p, stream);
-        if (r <= 20) return launch_moe_fp4_tile<KgCfg<B, 1, 4, 1, 1, 1, 2>, 3>(p, stream);
+        if (decode) return launch_moe_fp4_tile<KgCfg<B, 1, 1, 4, 1, 1, 2>, 2>(p, stream);
+        if (r <= 20) return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 1, 1, 2>, 3>(p, stream);
         if (r <= 56) return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 1, 2, 2>, 2>(p, stream);
         if (r <= 112 && K > 3072) return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 2, 2, 2>, 2>(p, stream);
     }
-    // K % 256 == 128 or scales at odd strides: the streaming path when the tiled
-    // grid would give fewer than a quarter of the CUs work and there are at most
-    // 32 valid gate ids (measured: one token's down projection, N = 4096, 56 ->
+    // K % 256 == 128, or weight rows too wide for the small tiles: the streaming
+    // path at decode sizes (measured: one token's down projection, N = 4096, 56 ->
     // 22 us; with N = 28672 or eight tokens the tiled kernel is faster). Its
     // scale loads are dwords, and 64 weight rows must span less than 2 GiB.
-    const bool few_tiles = ((grid_m + 1) / 2) * ((N + MOE_BN - 1) / MOE_BN) * 4 < ncu;
-    if (!wt && few_tiles && num_valid_tokens <= MOE_FP4_NARROW_MAX_VALID && stride_amxm % 4 == 0 && stride_bmxn % 4 == 0 &&
+    if (!wt && decode && stride_amxm % 4 == 0 && stride_bmxn % 4 == 0 &&
         stride_bmxe % 4 == 0 && reinterpret_cast<uintptr_t>(A_mx_scale) % 4 == 0 &&
         reinterpret_cast<uintptr_t>(B_mx_scale) % 4 == 0 && 64 * stride_bn < (1ll << 31) && 64 * stride_bmxn < (1ll << 31))
         return launch_moe_fp4_narrow(p, stream);

@@ -572,16 +572,19 @@ __global__ __launch_bounds__(64 * BS_NW, 1) void moe_blockscale8_kernel(const Mo
 }
 
 // ---------------------------------------------------------------------------
-// Few rows per expert (at most one routing block on average): small tiles with
-// K split over the workgroup's waves (gemm_kgroup.h), a workgroup per routing
-// word and column tile, walking the block's rows BM at a time. Bound by the
-// weights' way from HBM: 256-row tiles gave every 16-row block the loads,
-// barriers and LDS of 256 rows, and one workgroup per CU left it idle between
-// tiles. With 32-row tiles two workgroups share a CU (78 KB of LDS each), so
-// one's prologue and epilogue run under the other's stream. Measured on MI355X
-// (8 experts of 4096 x 14336, top-2, whole layer with 128 x 128 groups, which
-// reads 1.41 GB of weights): 64 tokens 442 -> 281 us (5.0 TB/s), 1 token 222
-// -> 102, 300 tokens 494 -> 350, 512 tokens 530 -> 446.
+// Few rows per expert (at most one routing block on average): small tiles
+// (gemm_kgroup.h), a workgroup per routing word and column tile, walking the
+// block's rows BM at a time. Bound by the weights' way from HBM: 256-row tiles
+// gave every 16-row block the loads, barriers and LDS of 256 rows, and one
+// workgroup per CU left it idle between tiles. Three 64 x 64 tiles share a CU
+// (51 KB of LDS each), so one's prologue and epilogue run under the others'
+// streams. K-tiles are added in K order (one K group), which makes the results
+// those of the block-pair kernel, bit for bit; three groups of waves a tile, or
+// column tiles that start at different K-tiles, were up to 10 % faster with
+// rows of 4 KiB (64 tokens 257 us) but gave other sums. Measured on MI355X (8
+// experts of 4096 x 14336, top-2, gate/up and down with 128 x 128 groups, 1.41
+// GB of weights), block pairs and now: 64 tokens 416 -> 275 us (5.1 TB/s), 1
+// token 155 -> 85, 300 tokens 459 -> 349, 500 tokens 494 -> 425.
 template <class Cfg, int MINB>
 __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_bs_tile_kernel(const MoeBsParams p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
@@ -603,7 +606,6 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_bs
     KgSrc<Cfg, true> src;
     src.KT = p.K / 128;
     src.sc_shift = 31 - __builtin_clz(p.gk / 128);
-    src.rot = kg_rotation(p.swn, src.KT, tn, src.sc_shift);
     src.a = buffer_desc(p.X, clamp_bytes((int64_t)p.T * p.sxm));
     src.b = buffer_desc(p.W + (int64_t)e * p.swe + (int64_t)n0 * p.swn, clamp_bytes((int64_t)rows_b * p.swn));
     src.as = buffer_desc(p.xs, clamp_bytes(p.xs_elems * 4));
@@ -787,9 +789,9 @@ static int moe_blockscale_impl(const void* X, const void* W, void* Y, const floa
         // weights, one column scale per 32 columns, K-contiguous row scales)
         if (ntile && !wt && xs_stride_k == 1) {
             constexpr int B = MODE_BLOCKSCALE;
-            switch (moe_tile(gather ? T * topk : T, E, N, K, 112, 256)) {
-                case MOET_32x64: return launch_moe_bs_tile<KgCfg<B, 1, 1, 3, 1, 2, 2>, 2>(p, stream);
-                case MOET_64x128: return launch_moe_bs_tile<KgCfg<B, 2, 2, 1, 1, 2, 3>, 2>(p, stream);
+            switch (moe_tile(gather ? T * topk : T, E, K, 112, 256)) {
+                case MOET_64x64: return launch_moe_bs_tile<KgCfg<B, 2, 2, 1, 1, 1, 3>, 3>(p, stream);
+                case MOET_64x128: return launch_moe_bs_tile<KgCfg<B, 2, 4, 1, 1, 1, 3>, 2>(p, stream);
                 case MOET_128x128: return launch_moe_bs_tile<KgCfg<B, 4, 2, 1, 1, 2, 4>, 1>(p, stream);
                 case MOET_128x256: return launch_moe_bs_tile<KgCfg<B, 2, 4, 1, 2, 2, 3>, 1>(p, stream);
                 case MOET_PAIRS: break;

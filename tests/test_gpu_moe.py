@@ -432,12 +432,53 @@ def test_moe_blockscale(orc, T, E, topk, K, N, gk, gn):
     check_rows(orc, Y, ref)
 
 
-# The A8W8 small tiles by mean rows per expert (K up to 3072: 10 on 32x64, or
-# 32x128 with N = 4100, 33 on 64x128, 75 on 128x256; above: 5 on 32x64, 32 on 64x128, 76 on
-# 128x128, 150 on 128x256), routing skewed so that some experts hold several row
-# groups or blocks and some no row, odd counts of K-tiles, rows of 4096 bytes
-# (column tiles start at different K-tiles), ragged N, every scale form, -1 /
-# malformed words between the live ones.
+def order_codes(rng, shape):
+    """E4M3FN codes of every exponent (no NaN): fp32 sums of their products
+    depend on the order in which they are added."""
+    c = rng.integers(0, 0x7F, shape, dtype=np.uint8)
+    return c | (rng.integers(0, 2, shape, dtype=np.uint8) << 7)
+
+
+# Every small tile adds K-tile after K-tile in K order, as the block-pair
+# kernels that read [E, K, N] weights do: the same bits for both layouts. By
+# mean rows per expert, K above 3072: 64x64 (10 rows), 128x128 (75), 128x256
+# (150); below: 64x128 (25), 128x256 (75). Weight rows 4 KiB apart and not; codes
+# of every exponent, so that another order of the sums shows.
+@pytest.mark.parametrize("T,E,topk,K,N", [(40, 8, 2, 4096, 2056), (300, 8, 2, 4096, 1028), (300, 4, 2, 3200, 1028),
+                                          (100, 8, 2, 2048, 2056), (150, 4, 2, 896, 1028)])
+@pytest.mark.parametrize("fmt", ["a8w8", "blockscale"])
+def test_moe_small_tiles_k_order(orc, fmt, T, E, topk, K, N):
+    require_gpu()
+    rng = np.random.default_rng(T + K)
+    assigns = np.stack([rng.permutation(E)[:topk] for _ in range(T)])
+    hist, offs, gather, ed = orc.ogs_routing(assigns, E, 128)
+    X, W = order_codes(rng, (T, K)), order_codes(rng, (E, N, K))
+    r = (dev_i32(hist), dev_i32(offs), dev_i32(ed), topk)
+    Wd = dev_u8(W)
+    Wkn = torch.zeros((E, K, (N + 15) // 16 * 16), dtype=torch.uint8, device="cuda")
+    Wkn[:, :, :N] = Wd.transpose(1, 2)
+    Wkn = Wkn[:, :, :N]
+    if fmt == "blockscale":
+        xs = dev_f32(rng.random((T, K // 128)).astype(np.float32))
+        ws = dev_f32(rng.random((E, K // 128, -(-N // 128))).astype(np.float32))
+        Y = hkq.moe_a8w8_blockscale(dev_u8(X), Wd, *r, xs, ws, 128, 128, gather=dev_i32(gather))
+        Ykn = hkq.moe_a8w8_blockscale(dev_u8(X), Wkn, *r, xs, ws, 128, 128, gather=dev_i32(gather), w_kn=True)
+    else:
+        s = dict(gather=dev_i32(gather), x_scale=dev_f32(rng.random(T).astype(np.float32)),
+                 w_scale=dev_f32(rng.random((E, N)).astype(np.float32)))
+        Y = hkq.moe_a8w8(dev_u8(X), Wd, *r, **s)
+        Ykn = hkq.moe_a8w8(dev_u8(X), Wkn, *r, w_kn=True, **s)
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(Y).all())
+    differ = int((Y.view(torch.int16) != Ykn.view(torch.int16)).sum())
+    assert differ == 0, f"{differ} of {Y.numel()} elements differ between the weight layouts"
+
+
+# The A8W8 small tiles by mean rows per expert (K up to 3072: 10 and 33 on
+# 64x128, 75 on 128x256; above: 5 and 32 on 64x64, 76 on 128x128, 150 on 128x256),
+# routing skewed so that some experts hold several row groups or blocks and some
+# no row, odd counts of K-tiles, ragged N, every scale form, -1 / malformed words
+# between the live ones.
 @pytest.mark.parametrize("T,E,topk,K,N,scales", [
     (3, 8, 2, 128, 1000, "none"), (40, 8, 2, 640, 300, "channel"), (40, 8, 2, 640, 4100, "expert"), (100, 6, 2, 1152, 260, "expert"),
     (150, 4, 2, 896, 772, "channel"), (20, 8, 2, 4096, 260, "channel"), (130, 8, 2, 4096, 388, "expert"),
@@ -459,13 +500,11 @@ def test_moe_small_tiles(orc, T, E, topk, K, N, scales):
     check_rows(orc, Y, orc.moe_ref(X, W, xs, ws, None, gather, hist, offs, ed, topk, 128, "enk"))
 
 
-# Few rows per expert: the small tiles by mean rows per expert (K up to 3072: 0
-# and 10 on 32x64, 33 on 64x128, 75 on 128x256, 115 on block pairs; above: 4 on 32x64, 25
-# on 64x128, 75 on 128x128, 150 on 128x256), routing skewed so that some experts
-# hold several row groups or blocks and some no row, odd counts of K-tiles, rows
-# a multiple of 4 KiB apart (column tiles start at different K-tiles; with four
-# K-tiles per scale group they don't), one to four K-tiles per scale group,
-# ragged N, a bias, -1 / malformed words between the live ones and scale rows
+# Few rows per expert: the small tiles by mean rows per expert (K up to 3072: 0,
+# 10 and 33 on 64x128, 75 on 128x256, 115 on block pairs; above: 4 and 25 on 64x64,
+# 75 on 128x128, 150 on 128x256), routing skewed so that some experts hold several
+# row groups or blocks and some no row, odd counts of K-tiles, one to four K-tiles
+# per scale group, ragged N, a bias, -1 / malformed words between the live ones and scale rows
 # padded with NaN.
 @pytest.mark.parametrize("T,E,topk,K,N,gk", [(40, 8, 2, 640, 300, 128), (3, 8, 2, 128, 1000, 128),
                                              (100, 6, 2, 1152, 260, 128), (150, 4, 2, 896, 772, 256),

@@ -117,8 +117,8 @@ def test_moe_mxfp4_decode_layouts(orc):
     assert np.all(got[[4, 5]] == 0.0) and np.all(got[nv:] == 7.0)
 
 
-# The small tiles by mean valid entries per expert and by workgroups (1 and 10 on
-# 32x32 with K in four, 3 on 32x128, 33 on 64x128, 75 on 128x128 from K = 3328),
+# The small tiles by mean valid entries per expert (8 entries in all on 32x32 with
+# K in four, 10 and 3 on 64x64, 33 on 64x128, 75 on 128x128 from K = 3328),
 # routing skewed so that some experts hold several row groups or blocks, odd
 # counts of K-tiles, ragged N, routed weights, padded scale rows, a block whose
 # entries are scattered over its 128, one of expert -1 (zeros for its valid
@@ -232,6 +232,32 @@ def test_moe_mxfp4_kn_matches_kmajor(orc, T, E, topk, K, N, pad):
     got = Ckn.float().cpu().numpy()
     rows = ~np.isnan(ref).any(axis=1)
     assert_gemm_close(got[rows], ref[rows], "moe mxfp4 [E, K/2, N]")
+
+
+# The small tiles add K-tile after K-tile in K order, as the block-pair kernel
+# that reads [E, K/2, N] weights does: the same bits. 64x64 (10 entries per
+# expert), 64x128 (37) and 128x128 (75); block scales over 40 powers of two, so
+# that another order of the sums shows.
+@pytest.mark.parametrize("T,E,topk,K,N", [(40, 8, 2, 4352, 2056), (150, 8, 2, 4096, 1028), (300, 8, 2, 4096, 1028)])
+def test_moe_mxfp4_small_tiles_k_order(orc, T, E, topk, K, N):
+    require_gpu()
+    _, s, eids = routed(orc, T, E, topk, 81)
+    rng = np.random.default_rng(82)
+    Aq, As = rng.integers(0, 256, (T, K // 2), dtype=np.uint8), rng.integers(110, 130, (T, K // 32), dtype=np.uint8)
+    Bd = dev_u8(rng.integers(0, 256, (E, N, K // 2), dtype=np.uint8))
+    Bsd = dev_u8(rng.integers(110, 130, (E, N, K // 32), dtype=np.uint8))
+    Np = (N + 15) // 16 * 16
+    Bkn = torch.zeros((E, K // 2, Np), dtype=torch.uint8, device="cuda")
+    Bskn = torch.zeros((E, K // 32, Np), dtype=torch.uint8, device="cuda")
+    Bkn[:, :, :N] = Bd.transpose(1, 2)
+    Bskn[:, :, :N] = Bsd.transpose(1, 2)
+    args = (dev_i32(s), dev_i32(eids), T * topk, topk)
+    C = hkq.moe_mxfp4(dev_u8(Aq), dev_u8(As), Bd, Bsd, *args)
+    Ckn = hkq.moe_mxfp4(dev_u8(Aq), dev_u8(As), Bkn[:, :, :N], Bskn[:, :, :N], *args, b_kn=True)
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(C).all())
+    differ = int((C.view(torch.int16) != Ckn.view(torch.int16)).sum())
+    assert differ == 0, f"{differ} of {C.numel()} elements differ between the weight layouts"
 
 
 def test_moe_pack_kmajor(orc):
