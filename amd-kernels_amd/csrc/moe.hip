@@ -273,10 +273,10 @@ __global__ __launch_bounds__(64 * MOE_WM * MOE_WN, 1) void moe_gemm_kernel(const
 
 // ---------------------------------------------------------------------------
 // Few rows per expert: small tiles (gemm_kgroup.h), a workgroup per routing word
-// and column tile, walking the block's rows BM at a time. What bounds it is the
-// weights' way from HBM: the tiles and the workgroups per CU are chosen for the
-// bytes in flight; K-tiles are added in K order, as in the block-pair kernels
-// (measured on MI355X, 64 tokens on 8 experts of 4096 x 14336: gate/up 199 -> 185
+// and column tile, and per row group of the block where the tile has fewer than
+// its 128 rows (moe_tile). What bounds it is the weights' way from HBM: the tiles
+// and the workgroups per CU are chosen for the bytes in flight; K-tiles are added
+// in K order, as in the block-pair kernels (measured on MI355X, 64 tokens on 8 experts of 4096 x 14336: gate/up 199 -> 185
 // us, 5.1 TB/s; down 175 -> 83 us, 5.7 TB/s).
 template <class Cfg, int MINB>
 __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_tile_kernel(const MoeParams p) {
@@ -286,12 +286,13 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_ti
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wg = wave % Cfg::GW, kg = wave / Cfg::GW;
-    const int pm = blockIdx.x / p.tiles_n, tn = blockIdx.x % p.tiles_n;
+    const int nt = p.grid_m * p.tiles_n, rg = (int)blockIdx.x / nt, u = (int)blockIdx.x - rg * nt;
+    const int pm = u / p.tiles_n, tn = u % p.tiles_n;
     const int ed = p.expt_data[pm];
     const int e = ed & 0xFFFF, b = ed >> 16;
     if (ed < 0 || e >= p.E) return;  // uniform: -1 or a malformed entry
     const int m_e = p.hist[e], start = p.offs[e];
-    const int first = b * MOE_BM, rows = min(m_e - first, MOE_BM);
+    const int row0 = b * MOE_BM + rg * BM, rows = min(min(m_e, (b + 1) * MOE_BM) - row0, BM);
     if (rows <= 0 || start < 0) return;
     const int n0 = tn * BN;
     const int rows_b = min(p.N - n0, BN);
@@ -309,42 +310,39 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_ti
         src.b_off[i] = (uint32_t)(r * p.swn) + kg_chunk<Cfg>(r, lane);
     }
     const int nw = n0 + wg % Cfg::WN * TN * 32, mw = (wg / Cfg::WN * Cfg::TM + (Cfg::SPREAD ? kg * TMO : 0)) * 32;
-    for (int row0 = first; row0 < first + rows; row0 += BM) {
-        auto token_of = [&](int r) {
-            const int s = start + row0 + r;
-            if (row0 + r >= first + rows || s >= p.g_len) return -1;
-            const int t = p.gather ? div_recip(p.gather[s], p.rtopk) : s;
-            return (t >= 0 && t < p.T) ? t : -1;
+    auto token_of = [&](int r) {
+        const int s = start + row0 + r;
+        if (r >= rows || s >= p.g_len) return -1;
+        const int t = p.gather ? div_recip(p.gather[s], p.rtopk) : s;
+        return (t >= 0 && t < p.T) ? t : -1;
+    };
+#pragma unroll
+    for (int i = 0; i < Cfg::LA; ++i) {
+        const int r = kg_row<Cfg>(i, wg, lane), t = token_of(r);
+        src.a_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.sxm + kg_chunk<Cfg>(r, lane);
+    }
+    float rs[TMO];
+#pragma unroll
+    for (int j = 0; j < TMO; ++j) {
+        const int t = p.xs ? token_of(mw + j * 32 + (lane & 31)) : -1;
+        rs[j] = !p.xs ? 1.0f : (t < 0 ? 0.0f : p.xs[(int64_t)t * p.xs_tok]);
+    }
+    v16f acc[TN][TMO];
+    kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
+    if (Cfg::SPREAD || kg == 0) {
+        const int s0 = start + row0;
+        const int out_rows = min(rows, p.y_rows - s0);
+        // no bias, column scales absent, one per expert or one per channel (the launcher checks)
+        auto col_scale4 = [&](int i, int g) {
+            const int n = nw + i * 32 + 8 * g + 4 * (lane >> 5);
+            if (!p.ws) return make_float4(1.f, 1.f, 1.f, 1.f);
+            if (n >= p.N) return make_float4(0.f, 0.f, 0.f, 0.f);
+            const float* w = p.ws + (int64_t)e * p.ws_e;
+            if (p.ws_n == 0) return make_float4(w[0], w[0], w[0], w[0]);
+            return *reinterpret_cast<const float4*>(w + n);
         };
-#pragma unroll
-        for (int i = 0; i < Cfg::LA; ++i) {
-            const int r = kg_row<Cfg>(i, wg, lane), t = token_of(r);
-            src.a_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.sxm + kg_chunk<Cfg>(r, lane);
-        }
-        float rs[TMO];
-#pragma unroll
-        for (int j = 0; j < TMO; ++j) {
-            const int t = p.xs ? token_of(mw + j * 32 + (lane & 31)) : -1;
-            rs[j] = !p.xs ? 1.0f : (t < 0 ? 0.0f : p.xs[(int64_t)t * p.xs_tok]);
-        }
-        v16f acc[TN][TMO];
-        kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
-        if (Cfg::SPREAD || kg == 0) {
-            const int s0 = start + row0;
-            const int out_rows = min(min(first + rows - row0, BM), p.y_rows - s0);
-            // no bias, column scales absent, one per expert or one per channel (the launcher checks)
-            auto col_scale4 = [&](int i, int g) {
-                const int n = nw + i * 32 + 8 * g + 4 * (lane >> 5);
-                if (!p.ws) return make_float4(1.f, 1.f, 1.f, 1.f);
-                if (n >= p.N) return make_float4(0.f, 0.f, 0.f, 0.f);
-                const float* w = p.ws + (int64_t)e * p.ws_e;
-                if (p.ws_n == 0) return make_float4(w[0], w[0], w[0], w[0]);
-                return *reinterpret_cast<const float4*>(w + n);
-            };
-            store_tile_bf16<TMO, TN>(acc, smem, Cfg::SPREAD ? wave : wg, lane, p.Y + (int64_t)s0 * p.sym, p.sym, out_rows,
-                                     p.N, mw, nw, p.c16 != 0, [&](int j) { return rs[j]; }, col_scale4, NoBias{});
-        }
-        __syncthreads();  // the staging is read: the next row group's loads may overwrite it
+        store_tile_bf16<TMO, TN>(acc, smem, Cfg::SPREAD ? wave : wg, lane, p.Y + (int64_t)s0 * p.sym, p.sym, out_rows,
+                                 p.N, mw, nw, p.c16 != 0, [&](int j) { return rs[j]; }, col_scale4, NoBias{});
     }
 }
 
@@ -363,7 +361,7 @@ static int launch_moe_tile(MoeParams& p, hipStream_t stream) {
     }
     p.tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
     if (p.grid_m == 0 || p.N == 0) return 0;
-    kern<<<dim3((unsigned)((int64_t)p.grid_m * p.tiles_n)), Cfg::THREADS, Cfg::LDS, stream>>>(p);
+    kern<<<dim3((unsigned)((int64_t)p.grid_m * p.tiles_n * (MOE_BM / Cfg::BM))), Cfg::THREADS, Cfg::LDS, stream>>>(p);
     return hkq_launch_status();
 }
 
@@ -1072,11 +1070,11 @@ __global__ __launch_bounds__(64 * MOE_WM * MOE_WN, 1) void moe_mxfp4_kernel(cons
 }
 
 // ---------------------------------------------------------------------------
-// Few rows per expert: small tiles as in the A8W8 MoE, over one 128-entry block,
-// walking its entries BM at a time (row groups without a valid entry are
-// passed over: the sorted layout puts them last). Measured on MI355X (gate/up,
-// 8 experts, K 4096, N 28672): 24 tokens 111 -> 97 us (5.2 TB/s with the
-// scales), 300 126 -> 120.
+// Few rows per expert: small tiles as in the A8W8 MoE, over one 128-entry block
+// and, per workgroup, one group of BM of its entries (moe_tile; groups
+// without a valid entry end at once: the sorted layout puts them last).
+// Measured on MI355X (gate/up, 8 experts, K 4096, N 28672): 24 tokens 111 -> 97
+// us (5.2 TB/s with the scales), 300 126 -> 120.
 template <class Cfg, int MINB>
 __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_fp4_tile_kernel(const MoeFp4Params p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
@@ -1085,7 +1083,8 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_fp
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wg = wave % Cfg::GW, kg = wave / Cfg::GW;
-    const int pm = blockIdx.x / p.tiles_n, tn = blockIdx.x % p.tiles_n;
+    const int nt = p.grid_m * p.tiles_n, rg = (int)blockIdx.x / nt, u = (int)blockIdx.x - rg * nt;
+    const int pm = u / p.tiles_n, tn = u % p.tiles_n;
     const int n0 = tn * BN;
     const int32_t* ids = p.sorted + (int64_t)pm * MOE_BM;
     const int e = p.expert[pm];
@@ -1094,7 +1093,7 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_fp
         return (id >= 0 && id < p.num_valid) ? id : -1;
     };
     if (e < 0 || e >= p.E) {
-        if (e == -1) {  // valid rows of an unassigned block are zeros
+        if (e == -1 && rg == 0) {  // valid rows of an unassigned block are zeros
             for (int r = wave; r < MOE_BM; r += Cfg::NW) {
                 const int id = gate_of(r);
                 if (id < 0) continue;
@@ -1104,6 +1103,10 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_fp
         }
         return;
     }
+    const int row0 = rg * BM;
+    int any = 0;  // uniform: every wave looks at the group's entries
+    for (int r = lane; r < BM; r += 64) any |= gate_of(row0 + r) >= 0;
+    if (__ballot(any) == 0) return;
     const int rows_b = min(p.N - n0, BN);
     KgSrc<Cfg, true> src;
     src.KT = p.K / 256;
@@ -1122,53 +1125,46 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_fp
     }
     const int nw = n0 + wg % Cfg::WN * TN * 32, mw = (wg / Cfg::WN * Cfg::TM + (Cfg::SPREAD ? kg * TMO : 0)) * 32;
     const float gs = (p.a_scale ? p.a_scale[0] : 1.0f) * (p.b_scale ? p.b_scale[e] : 1.0f);
-    for (int row0 = 0; row0 < MOE_BM; row0 += BM) {
-        // uniform: every wave looks at the group's entries
-        int any = 0;
-        for (int r = lane; r < BM; r += 64) any |= gate_of(row0 + r) >= 0;
-        if (__ballot(any) == 0) continue;
-        auto arow_of = [&](int r) {
-            const int id = gate_of(row0 + r);
-            const int t = id < 0 ? -1 : div_recip(id, p.rtopk);
-            return t < p.tokens ? t : -1;
-        };
+    auto arow_of = [&](int r) {
+        const int id = gate_of(row0 + r);
+        const int t = id < 0 ? -1 : div_recip(id, p.rtopk);
+        return t < p.tokens ? t : -1;
+    };
 #pragma unroll
-        for (int i = 0; i < Cfg::LA; ++i) {
-            const int r = kg_row<Cfg>(i, wg, lane), t = arow_of(r);
-            src.a_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.sam + kg_chunk<Cfg>(r, lane);
-        }
-#pragma unroll
-        for (int i = 0; i < Cfg::PW; ++i) {
-            const int q = i * Cfg::GW + wg;
-            if (q < Cfg::PA) {
-                const int t = arow_of(kg_piece_row<Cfg>(q, lane));
-                src.s_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.sas + kg_piece_half(lane);
-            } else {
-                src.s_off[i] = (uint32_t)(kg_piece_row<Cfg>(q - Cfg::PA, lane) * p.sbsn) + kg_piece_half(lane);
-            }
-        }
-        // the epilogue's gate ids (scatter rows) and routed weights, ahead of the K loop
-        int rid[(TMO * 32 + 63) / 64];
-#pragma unroll
-        for (int h = 0; h < (TMO * 32 + 63) / 64; ++h) {
-            const int r = h * 64 + lane;
-            rid[h] = r < TMO * 32 ? gate_of(row0 + mw + r) : -1;
-        }
-        float rs[TMO];
-#pragma unroll
-        for (int j = 0; j < TMO; ++j) {
-            const int id = gate_of(row0 + mw + j * 32 + (lane & 31));
-            rs[j] = (p.topk_w && id >= 0) ? gs * p.topk_w[id] : gs;
-        }
-        v16f acc[TN][TMO];
-        kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
-        if (Cfg::SPREAD || kg == 0)
-            store_tile_bf16_rows<TMO, TN>(
-                acc, smem, Cfg::SPREAD ? wave : wg, lane, p.C, p.scm, p.N, nw, p.c16 != 0,
-                [&](int r) { return (int64_t)__shfl(rid[TMO > 2 ? r >> 6 : 0], r & 63); }, [&](int j) { return rs[j]; },
-                [&](int, int) { return make_float4(1.f, 1.f, 1.f, 1.f); }, NoBias{});
-        __syncthreads();  // the staging is read: the next row group's loads may overwrite it
+    for (int i = 0; i < Cfg::LA; ++i) {
+        const int r = kg_row<Cfg>(i, wg, lane), t = arow_of(r);
+        src.a_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.sam + kg_chunk<Cfg>(r, lane);
     }
+#pragma unroll
+    for (int i = 0; i < Cfg::PW; ++i) {
+        const int q = i * Cfg::GW + wg;
+        if (q < Cfg::PA) {
+            const int t = arow_of(kg_piece_row<Cfg>(q, lane));
+            src.s_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.sas + kg_piece_half(lane);
+        } else {
+            src.s_off[i] = (uint32_t)(kg_piece_row<Cfg>(q - Cfg::PA, lane) * p.sbsn) + kg_piece_half(lane);
+        }
+    }
+    // the epilogue's gate ids (scatter rows) and routed weights, ahead of the K loop
+    int rid[(TMO * 32 + 63) / 64];
+#pragma unroll
+    for (int h = 0; h < (TMO * 32 + 63) / 64; ++h) {
+        const int r = h * 64 + lane;
+        rid[h] = r < TMO * 32 ? gate_of(row0 + mw + r) : -1;
+    }
+    float rs[TMO];
+#pragma unroll
+    for (int j = 0; j < TMO; ++j) {
+        const int id = gate_of(row0 + mw + j * 32 + (lane & 31));
+        rs[j] = (p.topk_w && id >= 0) ? gs * p.topk_w[id] : gs;
+    }
+    v16f acc[TN][TMO];
+    kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
+    if (Cfg::SPREAD || kg == 0)
+        store_tile_bf16_rows<TMO, TN>(
+            acc, smem, Cfg::SPREAD ? wave : wg, lane, p.C, p.scm, p.N, nw, p.c16 != 0,
+            [&](int r) { return (int64_t)__shfl(rid[TMO > 2 ? r >> 6 : 0], r & 63); }, [&](int j) { return rs[j]; },
+            [&](int, int) { return make_float4(1.f, 1.f, 1.f, 1.f); }, NoBias{});
 }
 
 template <class Cfg, int MINB>
@@ -1186,7 +1182,7 @@ static int launch_moe_fp4_tile(MoeFp4Params& p, hipStream_t stream) {
     }
     p.tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
     if (p.grid_m == 0 || p.N == 0) return 0;
-    kern<<<dim3((unsigned)((int64_t)p.grid_m * p.tiles_n)), Cfg::THREADS, Cfg::LDS, stream>>>(p);
+    kern<<<dim3((unsigned)((int64_t)p.grid_m * p.tiles_n * (MOE_BM / Cfg::BM))), Cfg::THREADS, Cfg::LDS, stream>>>(p);
     return hkq_launch_status();
 }
 
@@ -1424,7 +1420,7 @@ static int moe_a8w8_impl(const void* X, const void* W, void* Y, const float* x_s
     const bool decode = (routed <= 32 || (routed <= MOE_NARROW_MAX_ROWS && N <= 4096)) && !wt && K % 128 == 0 &&
                         64 * stride_w < (1ll << 31);
     if (!(few && decode) && !wt && K % 128 == 0 && !bias && (!w_scale || ws_stride_n == 0 || p.ws_vec) &&
-        256 * stride_w < (1ll << 31)) {
+        256 * stride_w < (1ll << 31) && kg_moe_grid(grid_m, N)) {
         constexpr int B = MODE_A8W8;
         switch (moe_tile(routed, E, K, 128, 352)) {
             case MOET_64x64: return launch_moe_tile<KgCfg<B, 2, 2, 1, 1, 1, 3>, 3>(p, stream);
@@ -1552,12 +1548,15 @@ static int moe_mxfp4_impl(const void* A, const void* B, void* C, const void* A_m
     const bool few_tiles = ((grid_m + 1) / 2) * ((N + MOE_BN - 1) / MOE_BN) * 4 < ncu;
     const bool decode = few_tiles && num_valid_tokens <= MOE_FP4_NARROW_MAX_VALID;
     if (!wt && K % 256 == 0 && stride_amxm % 4 == 0 && stride_bmxn % 4 == 0 && stride_bmxe % 4 == 0 &&
-        256 * stride_bn < (1ll << 31) && 256 * stride_bmxn < (1ll << 31)) {
+        256 * stride_bn < (1ll << 31) && 256 * stride_bmxn < (1ll << 31) && kg_moe_grid(grid_m, N)) {
         constexpr int B = MODE_MXFP4;
         if (decode) return launch_moe_fp4_tile<KgCfg<B, 1, 1, 4, 1, 1, 2>, 2>(p, stream);
-        if (r <= 20) return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 1, 1, 2>, 3>(p, stream);
+        if (r <= (K > 3072 ? 20 : 56)) return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 1, 1, 2>, 3>(p, stream);
         if (r <= 56) return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 1, 2, 2>, 2>(p, stream);
-        if (r <= 112 && K > 3072) return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 2, 2, 2>, 2>(p, stream);
+        // with more blocks than experts some expert holds several: the pairs
+        // (half of 300 tokens' entries on one expert, gate/up 122 against 144)
+        if (r <= 112 && K > 3072 && grid_m <= num_experts)
+            return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 2, 2, 2>, 2>(p, stream);
     }
     // K % 256 == 128, or weight rows too wide for the small tiles: the streaming
     // path at decode sizes (measured: one token's down projection, N = 4096, 56 ->

@@ -573,10 +573,10 @@ __global__ __launch_bounds__(64 * BS_NW, 1) void moe_blockscale8_kernel(const Mo
 
 // ---------------------------------------------------------------------------
 // Few rows per expert (at most one routing block on average): small tiles
-// (gemm_kgroup.h), a workgroup per routing word and column tile, walking the
-// block's rows BM at a time. Bound by the weights' way from HBM: 256-row tiles
-// gave every 16-row block the loads, barriers and LDS of 256 rows, and one
-// workgroup per CU left it idle between tiles. Three 64 x 64 tiles share a CU
+// (gemm_kgroup.h), a workgroup per routing word and column tile, and per row
+// group of the block (moe_tile). Bound by the weights' way from HBM: 256-row
+// tiles gave every 16-row block the loads, barriers and LDS of 256 rows, and
+// one workgroup per CU left it idle between tiles. Three 64 x 64 tiles share a CU
 // (51 KB of LDS each), so one's prologue and epilogue run under the others'
 // streams. K-tiles are added in K order (one K group), which makes the results
 // those of the block-pair kernel, bit for bit; three groups of waves a tile, or
@@ -593,12 +593,13 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_bs
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wg = wave % Cfg::GW, kg = wave / Cfg::GW;
-    const int pm = blockIdx.x / p.tiles_n, tn = blockIdx.x % p.tiles_n;
+    const int nt = p.grid_m * p.tiles_n, rg = (int)blockIdx.x / nt, u = (int)blockIdx.x - rg * nt;
+    const int pm = u / p.tiles_n, tn = u % p.tiles_n;
     const int ed = p.expt_data[pm];
     const int e = ed & 0xFFFF, b = ed >> 16;
     if (ed < 0 || e >= p.E) return;  // uniform: -1 or a malformed entry
     const int m_e = p.hist[e], start = p.offs[e];
-    const int rows = min(m_e - b * 128, 128);
+    const int row0 = b * 128 + rg * BM, rows = min(min(m_e, (b + 1) * 128) - row0, BM);
     if (rows <= 0 || start < 0) return;
     const int n0 = tn * BN;
     const int rows_b = min(p.N - n0, BN);
@@ -618,48 +619,45 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_bs
         src.b_off[i] = (uint32_t)(r * p.swn) + kg_chunk<Cfg>(r, lane);
     }
     const int nw = n0 + wg % Cfg::WN * TN * 32;
-    for (int row0 = b * 128; row0 < b * 128 + rows; row0 += BM) {
-        auto token_of = [&](int r) {
-            const int s = start + row0 + r;
-            if (row0 + r >= b * 128 + rows || r >= BM || s >= p.g_len) return -1;
-            const int t = p.gather ? div_recip(p.gather[s], p.rtopk) : s;
-            return (t >= 0 && t < p.T) ? t : -1;
-        };
+    auto token_of = [&](int r) {
+        const int s = start + row0 + r;
+        if (r >= rows || s >= p.g_len) return -1;
+        const int t = p.gather ? div_recip(p.gather[s], p.rtopk) : s;
+        return (t >= 0 && t < p.T) ? t : -1;
+    };
 #pragma unroll
-        for (int i = 0; i < Cfg::LA; ++i) {
-            const int r = kg_row<Cfg>(i, wg, lane), t = token_of(r);
-            src.a_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.sxm + kg_chunk<Cfg>(r, lane);
-        }
+    for (int i = 0; i < Cfg::LA; ++i) {
+        const int r = kg_row<Cfg>(i, wg, lane), t = token_of(r);
+        src.a_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.sxm + kg_chunk<Cfg>(r, lane);
+    }
 #pragma unroll
-        for (int i = 0; i < Cfg::PW; ++i) {
-            const int q = i * Cfg::GW + wg;
-            if (q < Cfg::PA) {
-                const int t = token_of(kg_piece_row<Cfg>(q, lane));
-                src.s_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.xsm * 4u;
-            } else {
-                src.s_off[i] = (uint32_t)(min(n0 + (lane >> 2) * 32, p.N - 1) / p.gn) * (uint32_t)p.wsn * 4u +
-                               (uint32_t)(lane & 3) * src.bs_step;
-            }
+    for (int i = 0; i < Cfg::PW; ++i) {
+        const int q = i * Cfg::GW + wg;
+        if (q < Cfg::PA) {
+            const int t = token_of(kg_piece_row<Cfg>(q, lane));
+            src.s_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.xsm * 4u;
+        } else {
+            src.s_off[i] = (uint32_t)(min(n0 + (lane >> 2) * 32, p.N - 1) / p.gn) * (uint32_t)p.wsn * 4u +
+                           (uint32_t)(lane & 3) * src.bs_step;
         }
-        v16f acc[TN][TMO];
-        kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
-        if (Cfg::SPREAD || kg == 0) {
-            const int s0 = start + row0;
-            const int mw = (wg / Cfg::WN * Cfg::TM + (Cfg::SPREAD ? kg * TMO : 0)) * 32;
-            const int out_rows = min(min(b * 128 + rows - row0, BM), p.y_rows - s0);
-            auto one = [](int) { return 1.0f; };
-            auto ones = [](int, int) { return make_float4(1.f, 1.f, 1.f, 1.f); };
-            const int ep = Cfg::SPREAD ? wave : wg;
-            uint16_t* Y = p.Y + (int64_t)s0 * p.sym;
-            store_tile_bf16<TMO, TN>(acc, smem, ep, lane, Y, p.sym, out_rows, p.N, mw, nw, p.c16 != 0, one, ones,
-                                     [&](int i, int g) {
-                                         const int n = nw + i * 32 + 8 * g + 4 * (lane >> 5);
-                                         if (!p.bias || n >= p.N) return make_float4(-0.f, -0.f, -0.f, -0.f);
-                                         const float* bp = p.bias + (int64_t)e * p.bias_e + n;
-                                         return make_float4(bp[0], bp[1], bp[2], bp[3]);
-                                     });
-        }
-        __syncthreads();  // the staging is read: the next row group's loads may overwrite it
+    }
+    v16f acc[TN][TMO];
+    kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
+    if (Cfg::SPREAD || kg == 0) {
+        const int s0 = start + row0;
+        const int mw = (wg / Cfg::WN * Cfg::TM + (Cfg::SPREAD ? kg * TMO : 0)) * 32;
+        const int out_rows = min(rows, p.y_rows - s0);
+        auto one = [](int) { return 1.0f; };
+        auto ones = [](int, int) { return make_float4(1.f, 1.f, 1.f, 1.f); };
+        const int ep = Cfg::SPREAD ? wave : wg;
+        uint16_t* Y = p.Y + (int64_t)s0 * p.sym;
+        store_tile_bf16<TMO, TN>(acc, smem, ep, lane, Y, p.sym, out_rows, p.N, mw, nw, p.c16 != 0, one, ones,
+                                 [&](int i, int g) {
+                                     const int n = nw + i * 32 + 8 * g + 4 * (lane >> 5);
+                                     if (!p.bias || n >= p.N) return make_float4(-0.f, -0.f, -0.f, -0.f);
+                                     const float* bp = p.bias + (int64_t)e * p.bias_e + n;
+                                     return make_float4(bp[0], bp[1], bp[2], bp[3]);
+                                 });
     }
 }
 
@@ -677,7 +675,7 @@ static int launch_moe_bs_tile(MoeBsParams& p, hipStream_t stream) {
         attr_set = true;
     }
     p.tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
-    kern<<<dim3((unsigned)((int64_t)p.grid_m * p.tiles_n)), Cfg::THREADS, Cfg::LDS, stream>>>(p);
+    kern<<<dim3((unsigned)((int64_t)p.grid_m * p.tiles_n * (128 / Cfg::BM))), Cfg::THREADS, Cfg::LDS, stream>>>(p);
     return hkq_launch_status();
 }
 
@@ -787,7 +785,7 @@ static int moe_blockscale_impl(const void* X, const void* W, void* Y, const floa
         const bool ntile = group_n % 32 == 0;
         // few rows per expert: small tiles over one routing block (K-contiguous
         // weights, one column scale per 32 columns, K-contiguous row scales)
-        if (ntile && !wt && xs_stride_k == 1) {
+        if (ntile && !wt && xs_stride_k == 1 && kg_moe_grid(grid_m, N)) {
             constexpr int B = MODE_BLOCKSCALE;
             switch (moe_tile(gather ? T * topk : T, E, K, 112, 256)) {
                 case MOET_64x64: return launch_moe_bs_tile<KgCfg<B, 2, 2, 1, 1, 1, 3>, 3>(p, stream);

@@ -500,6 +500,32 @@ def test_moe_small_tiles(orc, T, E, topk, K, N, scales):
     check_rows(orc, Y, orc.moe_ref(X, W, xs, ws, None, gather, hist, offs, ed, topk, 128, "enk"))
 
 
+# Row groups of the 64-row tiles (a workgroup each): experts of 1 to 129 rows at
+# the groups' and blocks' edges, 36 in the mean (64x64 with K = 3200, 64x128 below).
+ROW_GROUPS = [0, 1, 63, 64, 65, 127, 128, 129] + [0] * 8
+
+
+@pytest.mark.parametrize("K,N", [(3200, 132), (640, 260)])
+@pytest.mark.parametrize("fmt", ["a8w8", "blockscale"])
+def test_moe_small_tile_row_groups(orc, fmt, K, N):
+    require_gpu()
+    E, T = len(ROW_GROUPS), sum(ROW_GROUPS)
+
+    def counted(rng, T, E, topk):
+        return rng.permutation(np.repeat(np.arange(E), ROW_GROUPS))[:, None]
+
+    _, hist, offs, gather, ed, X, xs, W, ws = make_problem(orc, T, E, 1, K, N, K, counted)
+    if fmt == "a8w8":
+        Y = run_moe(X, W, hist, offs, gather, ed, 1, xs, ws)
+        check_rows(orc, Y, orc.moe_ref(X, W, xs, ws, None, gather, hist, offs, ed, 1, 128, "enk"))
+    else:
+        rng = np.random.default_rng(K)
+        xs = (rng.random((T, K // 128)) * 0.02 + 0.005).astype(np.float32)
+        ws = (rng.random((E, K // 128, -(-N // 128))) * 0.002 + 0.0005).astype(np.float32)
+        Y = run_moe_bs(X, W, hist, offs, gather, ed, 1, xs, ws, 128, 128)
+        check_rows(orc, Y, orc.moe_blockscale_ref(X, W, xs, ws, None, gather, hist, offs, ed, 1, 128, 128))
+
+
 # Few rows per expert: the small tiles by mean rows per expert (K up to 3072: 0,
 # 10 and 33 on 64x128, 75 on 128x256, 115 on block pairs; above: 4 and 25 on 64x64,
 # 75 on 128x128, 150 on 128x256), routing skewed so that some experts hold several

@@ -118,7 +118,7 @@ def test_moe_mxfp4_decode_layouts(orc):
 
 
 # The small tiles by mean valid entries per expert (8 entries in all on 32x32 with
-# K in four, 10 and 3 on 64x64, 33 on 64x128, 75 on 128x128 from K = 3328),
+# K in four, 10, 3 and 33 on 64x64, 75 on block pairs: more blocks than experts),
 # routing skewed so that some experts hold several row groups or blocks, odd
 # counts of K-tiles, ragged N, routed weights, padded scale rows, a block whose
 # entries are scattered over its 128, one of expert -1 (zeros for its valid
@@ -234,9 +234,27 @@ def test_moe_mxfp4_kn_matches_kmajor(orc, T, E, topk, K, N, pad):
     assert_gemm_close(got[rows], ref[rows], "moe mxfp4 [E, K/2, N]")
 
 
+@pytest.mark.parametrize("E,K", [(16, 3328), (32, 1280)])
+def test_moe_mxfp4_small_tile_row_groups(orc, E, K):
+    """Row groups of the 64-row tiles (a workgroup each): experts of 1 to 129
+    entries at the groups' and blocks' edges; 36 in the mean (64x128), 18 (64x64)."""
+    require_gpu()
+    N = 260
+    counts = [0, 1, 63, 64, 65, 127, 128, 129] + [0] * (E - 8)
+    T = sum(counts)
+    Aq, As, Bq, Bs = problem(orc, T, E, K, N, E)
+    ids = np.random.default_rng(E).permutation(np.repeat(np.arange(E), counts)).astype(np.int32)
+    s, eids, _, _ = orc.align_block_size(ids, E, 128)
+    C = hkq.moe_mxfp4(dev_u8(Aq), dev_u8(As), dev_u8(Bq), dev_u8(Bs), dev_i32(s), dev_i32(eids), T, 1)
+    torch.cuda.synchronize()
+    ref = orc.moe_mxfp4_ref(Aq, As, Bq, Bs, None, None, None, s, eids, N, T, 1, False, T)
+    assert not np.isnan(ref).any()
+    assert_gemm_close(C.float().cpu().numpy(), ref, f"moe mxfp4 row groups E={E}")
+
+
 # The small tiles add K-tile after K-tile in K order, as the block-pair kernel
 # that reads [E, K/2, N] weights does: the same bits. 64x64 (10 entries per
-# expert), 64x128 (37) and 128x128 (75); block scales over 40 powers of two, so
+# expert), 64x128 (37) and 128x128 (75, no expert past a block); block scales over 40 powers of two, so
 # that another order of the sums shows.
 @pytest.mark.parametrize("T,E,topk,K,N", [(40, 8, 2, 4352, 2056), (150, 8, 2, 4096, 1028), (300, 8, 2, 4096, 1028)])
 def test_moe_mxfp4_small_tiles_k_order(orc, T, E, topk, K, N):
