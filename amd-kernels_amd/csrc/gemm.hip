@@ -116,12 +116,14 @@ __device__ __forceinline__ void dense_kloop(const DenseParams& p, int m0, int n0
     LoopSrc src;
     src.a = p.A + (int64_t)m0 * p.lda + kb0;
     src.b = p.B + (int64_t)n0 * p.ldb + kb0;
-    src.a_bytes = min((int64_t)rows_a * p.lda - kb0, (int64_t)0x7FFFFFFF);
-    src.b_bytes = min((int64_t)rows_b * p.ldb - kb0, (int64_t)0x7FFFFFFF);
+    // extents end with the last row's K bytes: whatever the pitch, an offset past
+    // the tile's rows that wraps at 32 bits stays inside the operand
+    src.a_bytes = min((int64_t)(rows_a - 1) * p.lda + p.kbytes - kb0, (int64_t)0x7FFFFFFF);
+    src.b_bytes = min((int64_t)(rows_b - 1) * p.ldb + p.kbytes - kb0, (int64_t)0x7FFFFFFF);
     src.as = FP4 ? static_cast<const uint8_t*>(p.sa) + (int64_t)m0 * p.lsa + ks0 : nullptr;
     src.bs = FP4 ? static_cast<const uint8_t*>(p.sb) + (int64_t)n0 * p.lsb + ks0 : nullptr;
-    src.as_bytes = FP4 ? min((int64_t)rows_a * p.lsa - ks0, (int64_t)0x7FFFFFFF) : 0;
-    src.bs_bytes = FP4 ? min((int64_t)rows_b * p.lsb - ks0, (int64_t)0x7FFFFFFF) : 0;
+    src.as_bytes = FP4 ? min((int64_t)(rows_a - 1) * p.lsa + p.K / 32 - ks0, (int64_t)0x7FFFFFFF) : 0;
+    src.bs_bytes = FP4 ? min((int64_t)(rows_b - 1) * p.lsb + p.K / 32 - ks0, (int64_t)0x7FFFFFFF) : 0;
     src.lsa = p.lsa;
     src.lsb = p.lsb;
     src.KT = kt1 - kt0;
@@ -272,8 +274,8 @@ struct DenseSeq {
         StreamSrc s;
         s.a = p->A + (int64_t)m0 * p->lda;
         s.b = p->B + (int64_t)n0 * p->ldb;
-        s.a_bytes = (uint32_t)min((int64_t)rows_a * p->lda, (int64_t)0x7FFFFFFF);
-        s.b_bytes = (uint32_t)min((int64_t)rows_b * p->ldb, (int64_t)0x7FFFFFFF);
+        s.a_bytes = clamp_bytes((int64_t)(rows_a - 1) * p->lda + p->kbytes);
+        s.b_bytes = clamp_bytes((int64_t)(rows_b - 1) * p->ldb + p->kbytes);
         s.as = static_cast<const uint8_t*>(p->sa) + (int64_t)m0 * p->lsa;
         s.bs = static_cast<const uint8_t*>(p->sb) + (int64_t)n0 * p->lsb;
         s.as_bytes = (uint32_t)min((int64_t)rows_a * p->lsa, (int64_t)0x7FFFFFFF);
@@ -807,11 +809,19 @@ static DensePlan dense_plan(int mode, int64_t M, int64_t N, int64_t kbytes) {
 enum DenseTile {
     DT_32x32, DT_32x64, DT_32x128, DT_64x64, DT_128x64, DT_128x128, DT_128x256,
     DT_128x128_PAIR,  // two workgroups per CU (dense_tile_kernel)
-    DT_256, DT_SPLIT
+    DT_256, DT_SPLIT,
+    DT_NONE  // rows too far apart for every size
 };
 struct TileCost { float us, e; };
-static int dense_tile_plan(int mode, int64_t M, int64_t N, int64_t kbytes, int64_t batch, bool small_ok,
-                           const DensePlan* split) {
+static int dense_tile_plan(int mode, const DenseParams& p, int64_t batch, const DensePlan* split) {
+    const int64_t M = p.M, N = p.N, kbytes = p.kbytes;
+    // Tile rows `ld` bytes apart that a 32-bit buffer offset reaches. The 256-row
+    // kernels end their extents with the last live row, so only those count
+    // there; the smaller ones form offsets for all of a tile's rows.
+    auto reach = [](int64_t rows, int64_t ld) { return ld <= 0x7FFFFFFF / rows; };
+    auto fits = [&](int64_t bm, int64_t bn) {
+        return reach(bm, p.lda) && reach(bn, p.ldb) && reach(bm, p.lsa) && reach(bn, p.lsb);
+    };
     static const int BM[] = {32, 32, 32, 64, 128, 128, 128, 128, 256}, BN[] = {32, 64, 128, 64, 64, 128, 256, 128, 256};
     static const TileCost A8W8[] = {{0.082f, 1.8f}, {0.118f, 2.3f}, {0.198f, 3.4f}, {0.145f, 3.5f}, {0.245f, 2.5f},
                                     {0.345f, 2.0f}, {0.54f, 3.0f},  {0.60f, 1.8f}, {0.716f, 4.5f}};
@@ -823,10 +833,11 @@ static int dense_tile_plan(int mode, int64_t M, int64_t N, int64_t kbytes, int64
     const TileCost* T = mode == MODE_A8W8 ? A8W8 : mode == MODE_MXFP4 ? FP4 : BF16;
     const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
     const float KT = (float)((kbytes + 64) / 128);
-    int best = DT_256;
+    int best = DT_NONE;
     float best_us = 0.f;
     for (int t = DT_256; t >= 0; --t) {
-        if (T[t].us < 0.f || (t < DT_256 && !small_ok) || (t == DT_128x128_PAIR && kbytes % 128 != 0)) continue;
+        if (T[t].us < 0.f || (t == DT_128x128_PAIR && kbytes % 128 != 0)) continue;
+        if (!(t == DT_256 ? fits(std::min<int64_t>(M, 256), std::min<int64_t>(N, 256)) : fits(BM[t], BN[t]))) continue;
         const int64_t tiles = batch * ((M + BM[t] - 1) / BM[t]) * ((N + BN[t] - 1) / BN[t]);
         const int64_t slots = t == DT_128x128_PAIR ? 2 * ncu : ncu;
         const float us = (float)((tiles + slots - 1) / slots) * (KT * T[t].us + T[t].e);
@@ -835,11 +846,11 @@ static int dense_tile_plan(int mode, int64_t M, int64_t N, int64_t kbytes, int64
             best_us = us;
         }
     }
-    if (split != nullptr) {
+    if (split != nullptr && fits(128, 128)) {
         const float kt = (float)split->kt_split;
         const float us = split->geo == GEO_128x64 ? kt * 0.345f + 5.7f
                                                   : kt * (mode == MODE_BF16 ? 0.5f : 0.4f) + 4.2f + 1.3f * (float)split->splits;
-        if (us < best_us) best = DT_SPLIT;
+        if (best == DT_NONE || us < best_us) best = DT_SPLIT;
     }
     return best;
 }
@@ -941,6 +952,10 @@ static int launch_dense(DenseParams& p, void* ws, size_t ws_bytes, hipStream_t s
     p.c16 = (p.ldc % 8 == 0) && (reinterpret_cast<uintptr_t>(p.C) % 16 == 0);
     if (p.M == 0 || p.N == 0) return 0;
     const int64_t batch = std::max(1, p.batch);
+    if (p.M == 1) {  // a single row's pitch is never stepped over
+        p.lda = p.kbytes;
+        if (MODE == MODE_MXFP4) p.lsa = p.K / 32;
+    }
     if (use_narrow(MODE, p.M, p.N, p.kbytes, p.lda, p.ldb, batch)) {
         const dim3 grid((unsigned)((p.N + 15) / 16), (unsigned)batch);
         narrow_gemm_kernel<<<grid, 64 * NARROW_WAVES, 0, stream>>>(p);
@@ -954,11 +969,8 @@ static int launch_dense(DenseParams& p, void* ws, size_t ws_bytes, hipStream_t s
         split = p.batch <= 1 && p.bias == nullptr && pl.geo != GEO_SKINNY && pl.splits > 1 && ws != nullptr &&
                 ws_bytes >= pl.ws_bytes;
     }
-    // 32-bit row offsets of the small tiles (128 activation rows, 256 weight rows)
-    const bool small_ok = 128 * p.lda < (1ll << 31) && 256 * p.ldb < (1ll << 31) && 128 * p.lsa < (1ll << 31) &&
-                          256 * p.lsb < (1ll << 31);
     constexpr int M4 = MODE == MODE_MXFP4;  // the e8m0 blocks take LDS from the ring
-    switch (dense_tile_plan(MODE, p.M, p.N, p.kbytes, batch, small_ok, split ? &pl : nullptr)) {
+    switch (dense_tile_plan(MODE, p, batch, split ? &pl : nullptr)) {
         case DT_32x32: return launch_dense_kgroup<KgCfg<MODE, 1, 1, 4, 1, 1, 4>>(p, stream);
         case DT_32x64: return launch_dense_kgroup<KgCfg<MODE, 1, 1, 4, 1, 2, 3 - M4>>(p, stream);
         case DT_32x128: return launch_dense_kgroup<KgCfg<MODE, 1, 1, 4 - M4, 1, 4, 2>>(p, stream);
@@ -987,6 +999,9 @@ static int launch_dense(DenseParams& p, void* ws, size_t ws_bytes, hipStream_t s
                 return launch_dense_tiles<MODE, 2, 2, 2, 2, 128, 1, 4>(p, S, kt, ws, stream);
             }
             break;
+        case DT_NONE:
+            HKQ_CHECK_ARG(false, "row pitches too large: 32 rows of each operand (or all of its rows) and of its scales "
+                                 "must span less than 2^31 bytes");
     }
     // 128-byte K-tiles of this kernel need whole ones in every row: a partial
     // last K-tile would read the next row's bytes instead of zeros

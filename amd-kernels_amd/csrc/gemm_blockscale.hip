@@ -101,14 +101,16 @@ __global__ __launch_bounds__(64 * BS_NW, 1) void blockscale_gemm_kernel(const Bl
     for (int i = 0; i < BS_LB; ++i) b_off[i] = dense_row_off<NW, BS_KT>(i, wave, lane, p.ldb);
     const uint8_t* a_src = p.A + (int64_t)m0 * p.lda;
     const uint8_t* b_src = p.B + (int64_t)n0 * p.ldb;
-    const int64_t a_bytes = min((int64_t)rows_a * p.lda, (int64_t)0x7FFFFFFF);
-    const int64_t b_bytes = min((int64_t)rows_b * p.ldb, (int64_t)0x7FFFFFFF);
+    // extents end with the last row's bytes: whatever the pitch, an offset past
+    // the tile's rows that wraps at 32 bits stays inside the operand
+    const int64_t a_bytes = min((int64_t)(rows_a - 1) * p.lda + p.K, (int64_t)0x7FFFFFFF);
+    const int64_t b_bytes = min((int64_t)(rows_b - 1) * p.ldb + p.K, (int64_t)0x7FFFFFFF);
     // scales: sa rows (wave & 3) * 64 + lane; sb per column: tile column c =
     // (wave & 3)*64 + lane from sb's row of the K-tile (GN 128: its block's
     // value), per block (GN 128, BN 256): blocks n0/128 + {0, 1}. Waves 4-7
     // repeat the loads of 0-3 so that every wave issues the same loads.
     const float* sa_src = p.sa + (int64_t)m0 * p.lsa;
-    const int64_t sa_bytes = min((int64_t)rows_a * p.lsa * 4, (int64_t)0x7FFFFFFF);
+    const int64_t sa_bytes = min(((int64_t)(rows_a - 1) * p.lsa + p.K / 128) * 4, (int64_t)0x7FFFFFFF);
     const uint32_t sa_off = (uint32_t)(((wave & 3) * 64 + lane) * p.lsa * 4);
     constexpr bool PER_COL = GN1 || W224;
     const int sb_row = GN1 ? p.N : (p.N + 127) / 128;  // values per sb row
@@ -279,6 +281,13 @@ __global__ __launch_bounds__(64 * BSN_WAVES) void blockscale_narrow_kernel(const
     }
 }
 
+// 32-bit offsets of the streaming kernel: 16 activation rows, 32 weight rows and
+// the scales
+static bool bs_narrow_fits(const BlockScaleParams& p) {
+    auto reach = [](int64_t rows, int64_t ld) { return ld <= 0x7FFFFFFF / rows; };
+    return reach(32, p.ldb) && reach(BSN_MAX_M, p.lda) && reach(4 * BSN_MAX_M, p.lsa) && reach(8 * (p.K / 128), p.lsb);
+}
+
 // 16-column (NT = 1) or 32-column (NT = 2, when N/16 workgroups exceed the
 // CUs) slices.
 template <bool GN1>
@@ -428,18 +437,29 @@ static int launch_blockscale_bn(BlockScaleParams& p, hipStream_t stream) {
 // tiles of 256 columns, 256 of 224). Column scales per column (GN 1) need 64
 // columns for a whole load and leave 128 x 256 no registers.
 // HKQ_BLOCKSCALE_W224=0 (read at each call) keeps 256-column tiles.
-enum BsTile { BST_32x32, BST_32x64, BST_64x64, BST_128x64, BST_128x128, BST_128x256, BST_256x256, BST_256x224, BST_COUNT };
-static int bs_plan(int64_t M, int64_t N, int64_t K, bool gn1, bool small_ok) {
+enum BsTile { BST_32x32, BST_32x64, BST_64x64, BST_128x64, BST_128x128, BST_128x256, BST_256x256, BST_256x224, BST_COUNT,
+              BST_NONE  // rows too far apart for every size
+};
+static int bs_plan(const BlockScaleParams& p, bool gn1) {
+    const int64_t M = p.M, N = p.N, K = p.K;
+    // Rows `ld` bytes apart that a 32-bit buffer offset reaches: all of a small
+    // tile's, the live ones of a 256-row tile (whose extents end with the last)
+    auto reach = [](int64_t rows, int64_t ld) { return ld <= 0x7FFFFFFF / rows; };
+    auto fits = [&](int t, int64_t bm, int64_t bn) {
+        if (t >= BST_256x256) bm = std::min<int64_t>(M, bm), bn = std::min<int64_t>(N, bn);
+        return reach(bm, p.lda) && reach(bn, p.ldb) && reach(4 * bm, p.lsa) &&
+               (t >= BST_256x256 || reach(8 * (K / 128), p.lsb));
+    };
     static const struct { int bm, bn; float us; bool gn1; } T[BST_COUNT] = {
         {32, 32, 0.10f, false},  {32, 64, 0.18f, true},    {64, 64, 0.24f, true},   {128, 64, 0.38f, true},
         {128, 128, 0.60f, true}, {128, 256, 0.97f, false}, {256, 256, 1.5f, true}, {256, 224, 1.3125f, true}};
     const char* w224_env = std::getenv("HKQ_BLOCKSCALE_W224");
     const bool w224_on = !(w224_env && w224_env[0] == '0');
     const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
-    int best = BST_256x256;
+    int best = BST_NONE;
     float best_us = 0.f;
     for (int t = BST_COUNT - 1; t >= 0; --t) {
-        if ((t < BST_256x256 && (!small_ok || (gn1 && !T[t].gn1))) || (t == BST_256x224 && !w224_on)) continue;
+        if ((gn1 && !T[t].gn1) || (t == BST_256x224 && !w224_on) || !fits(t, T[t].bm, T[t].bn)) continue;
         const int64_t tiles = ((M + T[t].bm - 1) / T[t].bm) * ((N + T[t].bn - 1) / T[t].bn);
         const float us = (float)((tiles + ncu - 1) / ncu) * ((float)(K / 128) * T[t].us + 2.3f);
         if (best_us == 0.f || us < best_us) {
@@ -451,9 +471,9 @@ static int bs_plan(int64_t M, int64_t N, int64_t K, bool gn1, bool small_ok) {
 }
 
 template <bool GN1>
-static int launch_blockscale(BlockScaleParams& p, bool small_ok, hipStream_t stream) {
+static int launch_blockscale(BlockScaleParams& p, hipStream_t stream) {
     constexpr int B = MODE_BLOCKSCALE;
-    switch (bs_plan(p.M, p.N, p.K, GN1, small_ok)) {
+    switch (bs_plan(p, GN1)) {
         case BST_32x32:
             if constexpr (!GN1) return launch_blockscale_tile<KgCfg<B, 1, 1, 4, 1, 1, 4>, false>(p, stream);
             break;
@@ -465,6 +485,25 @@ static int launch_blockscale(BlockScaleParams& p, bool small_ok, hipStream_t str
             if constexpr (!GN1) return launch_blockscale_tile<KgCfg<B, 2, 4, 1, 2, 2, 3>, false>(p, stream);
             break;
         case BST_256x224: return launch_blockscale_bn<GN1, BS_BN - 32>(p, stream);
+        case BST_NONE: {
+            // the streaming kernel over groups of 16 rows
+            HKQ_CHECK_ARG(bs_narrow_fits(p), "row pitches too large: 32 rows of each operand (or all of its rows) and of "
+                                             "its scales must span less than 2^31 bytes");
+            const int M = p.M;
+            for (int m0 = 0; m0 < M; m0 += BSN_MAX_M) {
+                BlockScaleParams q = p;
+                q.A += (int64_t)m0 * p.lda;
+                q.sa += (int64_t)m0 * p.lsa;
+                q.C += (int64_t)m0 * p.ldc;
+                if (p.ca) {
+                    q.ca += (int64_t)m0 * p.ldca;
+                    q.cb += (int64_t)m0 * p.ldcb;
+                }
+                q.M = std::min(BSN_MAX_M, M - m0);
+                if (int e = launch_blockscale_narrow<GN1>(q, stream)) return e;
+            }
+            return 0;
+        }
     }
     return launch_blockscale_bn<GN1, BS_BN>(p, stream);
 }
@@ -527,15 +566,17 @@ static int blockscale_call(const void* A, const void* B, const float* sa, const 
     p.cb = static_cast<const uint16_t*>(cb);
     p.ldca = ldca; p.ldcb = ldcb;
     if (M == 0 || N == 0) return 0;
+    // a stride only counts where there is a second row to step to
+    if (M == 1) {
+        p.lda = K;
+        p.lsa = K / 128;
+    }
+    if (K / 128 == 1) p.lsb = group_n == 1 ? N : (N + 127) / 128;
     // M <= 16 with at most 32 K groups streams the weights through registers
     // (16 x 7168 x 2048: 6.1 us against 5.8 on small tiles, 1 x 24576 x 1536
     // 10.3 against 11; with long K the tiles' deeper rings win: 8 x 7168 x
-    // 18432 29.2 against 25.7, 8 x 2112 x 7168 9.5 against 7.4). The streaming
-    // kernel's 32 weight rows and 16 activation rows, the small tiles' 256
-    // and 128, and the scales must span less than 2 GiB (32-bit offsets).
-    const bool scales32 = 128 * lsa < (1ll << 28) && (K / 128) * lsb < (1ll << 28);
-    if (M <= BSN_MAX_M && K / 128 <= 32 && 32 * ldb < (1ll << 31) && BSN_MAX_M * lda < (1ll << 31) && scales32)
+    // 18432 29.2 against 25.7, 8 x 2112 x 7168 9.5 against 7.4).
+    if (M <= BSN_MAX_M && K / 128 <= 32 && bs_narrow_fits(p))
         return group_n == 1 ? launch_blockscale_narrow<true>(p, stream) : launch_blockscale_narrow<false>(p, stream);
-    const bool small_ok = 256 * ldb < (1ll << 31) && 128 * lda < (1ll << 31) && scales32;
-    return group_n == 1 ? launch_blockscale<true>(p, small_ok, stream) : launch_blockscale<false>(p, small_ok, stream);
+    return group_n == 1 ? launch_blockscale<true>(p, stream) : launch_blockscale<false>(p, stream);
 }

@@ -109,7 +109,9 @@ int hkq_rmsnorm_quant(const void* x, const void* w, void* q, void* s, int64_t M,
 int hkq_swiglu_quant(const void* y, void* q, float* s, int64_t M, int64_t F, int64_t ldy, int64_t ldq, int64_t lds,
                      float alpha, int interleaved, int group, hkq_stream_t stream);
 
-/* ---- dense GEMMs (A [M, K], B [N, K], both K-contiguous; C bf16 [M, ldc]) ---- */
+/* ---- dense GEMMs (A [M, K], B [N, K], both K-contiguous; C bf16 [M, ldc]) ----
+ * Row pitches: min(32, rows) rows of each operand, and of its scales, must span
+ * less than 2^31 bytes; a call that no kernel can address is refused. */
 
 /* C = bf16((A . B^T) * sa[m] * sb[n]); A, B E4M3FN; sa fp32 [M], sb fp32 [N].
  * K % 64 == 0 (as the reference requires), N % 4 == 0, ldc % 4 == 0.

@@ -63,6 +63,19 @@ def test_argument_errors_are_reported_before_launch():
     assert "multiple of 128" in hkq.lib().hkq_last_error().decode()
 
 
+def test_gemm_pitches_beyond_every_tile_are_refused():
+    """Weight (or activation) rows 128 MiB apart put 32 rows past a 32-bit
+    buffer offset: no tile reads them all, and the call says so."""
+    p, M, N, K, wide = 0x1000, 64, 512, 4096, 1 << 27
+    m = "row pitches too large"
+    for lda, ldb in ((K, wide), (wide, K)):
+        _expect_invalid("hkq_gemm_a8w8", p, p, p, p, p, M, N, K, lda, ldb, N, None, match=m)
+        _expect_invalid("hkq_gemm_mxfp4", p, p, p, p, p, M, N, 2 * K, lda, ldb, K // 16, K // 16, N, None, match=m)
+        _expect_invalid("hkq_gemm_bf16", p, p, p, M, N, K, lda, ldb, N, None, match=m)
+        for gn in (128, 1):
+            _expect_invalid("hkq_gemm_blockscale", p, p, p, p, p, M, N, K, lda, ldb, K // 128, N, N, gn, None, match=m)
+
+
 def test_gemm_workspace_queries():
     """Host-side GEMM plans (no GPU needed): the narrow path (M <= 16, and
     M <= 32 on narrow short shapes) and full grids need no workspace; split-K

@@ -513,3 +513,57 @@ def test_gemm_small_tiles(orc, mode, M, N, KT):
     torch.cuda.synchronize()
     assert bool((Cp[:, N:] == 7.0).all()), "stores past N reached the row padding"
     assert_gemm_close(host_bf16_f32(C), ref, f"{mode} small tiles {M}x{N}x{K}")
+
+
+# Rows far apart (a view of a wide buffer): a 256-row tile's rows would lie past
+# its 2 GiB buffer range, so the plans keep to tiles whose rows a 32-bit offset
+# reaches. Weight rows 16 MiB apart with N past one 128-column tile, K above the
+# streaming kernels' 32 steps; the same for 200 activation rows; and
+# block-scaled rows 48 MiB apart, which only the 32-row tile (one scale per 128
+# columns) and the streaming kernel in groups of 16 rows (one per column) reach.
+def wide_rows(codes, pitch):
+    rows, k = codes.shape
+    buf = torch.empty((rows - 1) * pitch + k, dtype=torch.uint8, device="cuda")
+    v = buf.as_strided((rows, k), (pitch, 1))
+    v.copy_(dev_u8(codes))
+    return v
+
+
+@pytest.mark.parametrize("M,N,wide_a,wide_b", [(1, 160, 0, 16 << 20), (20, 160, 0, 16 << 20), (200, 64, 12 << 20, 0)])
+@pytest.mark.parametrize("fmt", ["a8w8", "mxfp4", "bs128", "bs1"])
+def test_gemm_wide_row_pitch(orc, fmt, M, N, wide_a, wide_b):
+    require_gpu()
+    K = 4352
+    a = lambda c: wide_rows(c, wide_a) if wide_a else dev_u8(c)
+    b = lambda c: wide_rows(c, wide_b) if wide_b else dev_u8(c)
+    if fmt == "a8w8":
+        A, B, sa, sb = a8w8_inputs(orc, M, N, K, seed=M)
+        C = hkq.gemm_a8w8(a(A), b(B), dev_f32(sa), dev_f32(sb))
+        ref = orc.gemm_a8w8_ref(A, B, sa, sb)
+    elif fmt == "mxfp4":
+        A, As, B, Bs = mx_inputs(orc, M, N, 2 * K, seed=M)
+        C = hkq.gemm_mxfp4(a(A), dev_u8(As), b(B), dev_u8(Bs))
+        ref = orc.gemm_mxfp4_ref(A, As, B, Bs)
+    else:
+        gn = int(fmt[2:])
+        A, B, sa, sb = blockscale_inputs(orc, M, N, K, M, gn)
+        C = hkq.gemm_blockscale(a(A), b(B), dev_f32(sa), dev_f32(sb), group_n=gn)
+        ref = orc.gemm_blockscale_ref(A, B, sa, sb, 128, gn)
+    torch.cuda.synchronize()
+    assert_gemm_close(host_bf16_f32(C), ref, f"{fmt} {M}x{N}x{K} rows far apart")
+
+
+@pytest.mark.parametrize("group_n", [128, 1])
+def test_gemm_blockscale_wide_row_pitch_48m(orc, group_n):
+    require_gpu()
+    M, N, K = 20, 64, 512
+    A, B, sa, sb = blockscale_inputs(orc, M, N, K, 48, group_n)
+    ca, cb = orc.randn_bf16((M, N), seed=1), orc.randn_bf16((M, N), seed=2)
+    bf = lambda x: torch.from_numpy(x.view(np.int16)).view(torch.bfloat16).cuda()
+    args = (dev_u8(A), wide_rows(B, 48 << 20), dev_f32(sa), dev_f32(sb))
+    C = hkq.gemm_blockscale(*args, group_n=group_n)
+    Cma = hkq.gemm_blockscale_mul_add(*args, bf(ca), bf(cb), group_n=group_n)
+    torch.cuda.synchronize()
+    ref = orc.gemm_blockscale_ref(A, B, sa, sb, 128, group_n)
+    assert_gemm_close(host_bf16_f32(C), ref, f"blockscale rows 48 MiB apart gn{group_n}")
+    assert_gemm_close(host_bf16_f32(Cma), host_bf16_f32(bf(ca)) * ref + host_bf16_f32(bf(cb)), "multiply-add")
