@@ -432,10 +432,13 @@ static int launch_blockscale_bn(BlockScaleParams& p, hipStream_t stream) {
 // 0.32, 0.56, 0.82, 1.3 in the order below) and in HBM (7168, 18432: 0.15,
 // 0.26, 0.33, 0.5, 0.67, 1.03, 1.9). It picks the fastest size at 24 .. 2048
 // rows of those shapes and of 24576, 1536 (the runner-up within 6% in all but
-// the clear cases). 224-column tiles of 256 rows do 7/8 of a 256-column
-// tile's work (they fill CUs that 256 columns leave idle: 2048 x 7168 is 224
-// tiles of 256 columns, 256 of 224). Column scales per column (GN 1) need 64
-// columns for a whole load and leave 128 x 256 no registers.
+// the clear cases). With one scale per column a 128 x 128 K-tile takes 0.66:
+// from there the 256-row tiles win where the CUs hold one round of them (1024 x
+// 7168 x 18432 204 against 218, 1536 x 4096 x 4096 50.5 against 53.9).
+// 224-column tiles of 256 rows do 7/8 of a 256-column tile's work (they fill
+// CUs that 256 columns leave idle: 2048 x 7168 is 224 tiles of 256 columns, 256
+// of 224). Column scales per column (GN 1) need 64 columns for a whole load and
+// leave 128 x 256 no registers.
 // HKQ_BLOCKSCALE_W224=0 (read at each call) keeps 256-column tiles.
 enum BsTile { BST_32x32, BST_32x64, BST_64x64, BST_128x64, BST_128x128, BST_128x256, BST_256x256, BST_256x224, BST_COUNT,
               BST_NONE  // rows too far apart for every size
@@ -461,7 +464,8 @@ static int bs_plan(const BlockScaleParams& p, bool gn1) {
     for (int t = BST_COUNT - 1; t >= 0; --t) {
         if ((gn1 && !T[t].gn1) || (t == BST_256x224 && !w224_on) || !fits(t, T[t].bm, T[t].bn)) continue;
         const int64_t tiles = ((M + T[t].bm - 1) / T[t].bm) * ((N + T[t].bn - 1) / T[t].bn);
-        const float us = (float)((tiles + ncu - 1) / ncu) * ((float)(K / 128) * T[t].us + 2.3f);
+        const float kt_us = gn1 && t == BST_128x128 ? 0.66f : T[t].us;
+        const float us = (float)((tiles + ncu - 1) / ncu) * ((float)(K / 128) * kt_us + 2.3f);
         if (best_us == 0.f || us < best_us) {
             best = t;
             best_us = us;
@@ -574,9 +578,18 @@ static int blockscale_call(const void* A, const void* B, const float* sa, const 
     if (K / 128 == 1) p.lsb = group_n == 1 ? N : (N + 127) / 128;
     // M <= 16 with at most 32 K groups streams the weights through registers
     // (16 x 7168 x 2048: 6.1 us against 5.8 on small tiles, 1 x 24576 x 1536
-    // 10.3 against 11; with long K the tiles' deeper rings win: 8 x 7168 x
-    // 18432 29.2 against 25.7, 8 x 2112 x 7168 9.5 against 7.4).
-    if (M <= BSN_MAX_M && K / 128 <= 32 && bs_narrow_fits(p))
+    // 10.3 against 11). With longer K the tiles' deeper rings win (8 x 7168 x
+    // 18432 28.0 against 21.1, 16384 columns of K 5120 17.3 against 15.7 with
+    // one scale per column) except where one 16-column slice per CU holds all of
+    // N: with one scale per column, whose smallest tile is 64 wide, the stream
+    // wins to 12 rows (1 x 2112 x 7168 7.7 against 11.3, 12 x 4096 x 14336 17.6
+    // against 19.0) and to 16 rows of up to 56 groups (16 x 2112 x 5632 8.6
+    // against 10.1, x 7168 11.3 both); with one per 128, to 2 rows of 48 groups
+    // (2 x 2112 x 5632 6.3 against 6.7, 4 x 2112 x 7168 8.0 against 7.4).
+    const int64_t groups = K / 128, ncu = cu_count() > 0 ? cu_count() : 256;
+    const bool one_slice = (N + 15) / 16 <= ncu;
+    const bool stream_long = group_n == 1 ? M <= 12 || groups <= 56 : M <= 2 && groups <= 48;
+    if (M <= BSN_MAX_M && (groups <= 32 || (one_slice && stream_long)) && bs_narrow_fits(p))
         return group_n == 1 ? launch_blockscale_narrow<true>(p, stream) : launch_blockscale_narrow<false>(p, stream);
     return group_n == 1 ? launch_blockscale<true>(p, stream) : launch_blockscale<false>(p, stream);
 }

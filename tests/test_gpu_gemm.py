@@ -400,6 +400,19 @@ def test_gemm_blockscale_small_tiles(orc, M, N, K, group_n):
                       f"blockscale small tiles {M}x{N}x{K} gn{group_n}")
 
 
+# More than 32 K groups: M <= 12 (GN 1; 16 up to 56 groups) or M <= 2 (GN 128, up
+# to 48 groups) stream where one 16-column slice per CU holds all of N, and the
+# rows around those lines run tiles.
+@pytest.mark.parametrize("group_n", [128, 1])
+@pytest.mark.parametrize("M,N,K", [(1, 132, 4224), (2, 260, 6144), (3, 260, 6272), (12, 1000, 7424), (13, 1000, 7168),
+                                   (13, 132, 7296), (5, 4100, 4224)])
+def test_gemm_blockscale_long_k_stream(orc, M, N, K, group_n):
+    require_gpu()
+    A, B, sa, sb = blockscale_inputs(orc, M, N, K, M + N + K, group_n)
+    C = run_blockscale(A, B, sa, sb, group_n)
+    assert_gemm_close(C, orc.gemm_blockscale_ref(A, B, sa, sb, 128, group_n), f"blockscale {M}x{N}x{K} gn{group_n}")
+
+
 def test_gemm_blockscale_uniform_scales_reduce_to_a8w8(orc):
     """Scales constant over K groups: the block-scale GEMM equals the A8W8 GEMM
     with the same per-row / per-column factors."""
