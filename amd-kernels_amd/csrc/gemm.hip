@@ -796,23 +796,33 @@ static DensePlan dense_plan(int mode, int64_t M, int64_t N, int64_t kbytes) {
     return pl;
 }
 
-// Tile size of a dense GEMM: the least estimated time
-// over the sizes below,
+// Tile size of a dense GEMM: the least estimated time over the sizes below,
 //   rounds of tiles over the CUs * (K-tiles * us + e) + 2.3 us,
-// us and e per size and operand format fitted to MI355X times at 24 .. 2500
-// rows of the benchmark's weights and of 1500 x 1024 (the pick is the fastest
-// size or within 6% of it at all of the 230 shapes). Split K (A8W8 and bf16,
-// a workspace given): one round of its own plan, the partial sums' exchange in
-// the constant. It is still the better one where half of the CUs' worth of
-// tiles meets a long K: 400x4096x14336 31.7 us against 34.7, 128x4096x14336
-// 17.7 against 18.4, bf16 256x2048x14336 29.8 against 32.8.
+// us and e per size and operand format fitted to MI355X times of every size at
+// 1 .. 2048 rows of 17 weights (512 .. 57344 columns, K 128 .. 16384) and 25
+// batches. 128 x 128 tiles on two workgroups per CU run their K-tiles faster
+// while there are no more of them than CUs (`alone`: MXFP4 1024x4096x4096 12.9
+// us, the eight-wave tile 15.4). 32 x 256 tiles are for up to 32 rows of a short
+// K, where every other size takes more rounds (A8W8 batch of 128 1x512x128 4.1
+// us, on 128 x 256 5.2; bf16 batch of 64 32x512x512 6.9, on 128 x 128 9.0); with
+// a longer one their columns starve the CUs of rows in flight (A8W8
+// 300x4096x14336 47 us, on 128 x 64 34). Split K (A8W8 and bf16, a workspace
+// given): one round of its own plan, the partial sums' exchange in the constant.
+// It is still the better one where half of the CUs' worth of tiles meets a long
+// K: 400x4096x14336 31.7 us against 34.7, 128x4096x14336 17.7 against 18.4, bf16
+// 512x4096x14336 64 against 72.
 enum DenseTile {
-    DT_32x32, DT_32x64, DT_32x128, DT_64x64, DT_128x64, DT_128x128, DT_128x256,
+    DT_32x32, DT_32x64, DT_32x128, DT_32x256, DT_64x64, DT_128x64, DT_128x128, DT_128x256,
     DT_128x128_PAIR,  // two workgroups per CU (dense_tile_kernel)
     DT_256, DT_SPLIT,
     DT_NONE  // rows too far apart for every size
 };
 struct TileCost { float us, e; };
+struct TileCosts {
+    TileCost tile[DT_256 + 1], alone;
+    float split64_us, split64_e;           // 128 x 64 tiles: per K-tile, constant
+    float split_us, split_e, split_parts;  // 128 x 128 tiles: per K-tile, constant, per split
+};
 static int dense_tile_plan(int mode, const DenseParams& p, int64_t batch, const DensePlan* split) {
     const int64_t M = p.M, N = p.N, kbytes = p.kbytes;
     // Tile rows `ld` bytes apart that a 32-bit buffer offset reaches. The 256-row
@@ -822,25 +832,31 @@ static int dense_tile_plan(int mode, const DenseParams& p, int64_t batch, const 
     auto fits = [&](int64_t bm, int64_t bn) {
         return reach(bm, p.lda) && reach(bn, p.ldb) && reach(bm, p.lsa) && reach(bn, p.lsb);
     };
-    static const int BM[] = {32, 32, 32, 64, 128, 128, 128, 128, 256}, BN[] = {32, 64, 128, 64, 64, 128, 256, 128, 256};
-    static const TileCost A8W8[] = {{0.082f, 1.8f}, {0.118f, 2.3f}, {0.198f, 3.4f}, {0.145f, 3.5f}, {0.245f, 2.5f},
-                                    {0.345f, 2.0f}, {0.54f, 3.0f},  {0.60f, 1.8f}, {0.716f, 4.5f}};
+    static const int BM[] = {32, 32, 32, 32, 64, 128, 128, 128, 128, 256},
+                     BN[] = {32, 64, 128, 256, 64, 64, 128, 256, 128, 256};
+    static const TileCosts A8W8 = {{{0.082f, 1.8f}, {0.118f, 2.3f}, {0.198f, 3.4f}, {0.36f, 1.5f}, {0.145f, 3.5f},
+                                    {0.245f, 2.5f}, {0.345f, 2.0f}, {0.54f, 3.0f}, {0.60f, 1.8f}, {0.716f, 4.5f}},
+                                   {0.60f, 1.8f}, 0.345f, 5.7f, 0.4f, 4.2f, 1.3f};
     // MXFP4's 128 x 256 tile would cost more than the 256 x 256 one
-    static const TileCost FP4[] = {{0.091f, 1.8f}, {0.125f, 1.9f}, {0.233f, 2.7f}, {0.161f, 3.1f}, {0.431f, 2.0f},
-                                   {0.589f, 2.3f}, {-1.f, 0.f},    {0.717f, 1.2f}, {0.909f, 3.4f}};
-    static const TileCost BF16[] = {{0.098f, 1.0f}, {0.132f, 1.5f}, {0.216f, 1.7f}, {0.156f, 2.4f}, {0.259f, 1.7f},
-                                    {0.393f, 0.9f}, {0.605f, 1.3f}, {0.58f, 1.5f},  {0.757f, 3.0f}};
-    const TileCost* T = mode == MODE_A8W8 ? A8W8 : mode == MODE_MXFP4 ? FP4 : BF16;
+    static const TileCosts FP4 = {{{0.091f, 1.8f}, {0.125f, 1.9f}, {0.233f, 2.7f}, {0.5f, 1.1f}, {0.188f, 2.9f},
+                                   {0.431f, 2.2f}, {0.478f, 2.9f}, {-1.f, 0.f}, {0.717f, 1.2f}, {0.909f, 3.9f}},
+                                  {0.611f, 0.0f}, 0.f, 0.f, 0.f, 0.f, 0.f};
+    static const TileCosts BF16 = {{{0.098f, 1.0f}, {0.132f, 1.5f}, {0.216f, 1.7f}, {0.31f, 0.85f}, {0.162f, 2.2f},
+                                    {0.278f, 1.7f}, {0.347f, 0.6f}, {0.606f, 1.2f}, {0.645f, 0.9f}, {0.647f, 2.1f}},
+                                   {0.559f, 0.6f}, 0.f, 0.f, 0.494f, 5.5f, 1.2f};
+    const TileCosts& T = mode == MODE_A8W8 ? A8W8 : mode == MODE_MXFP4 ? FP4 : BF16;
     const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
     const float KT = (float)((kbytes + 64) / 128);
     int best = DT_NONE;
     float best_us = 0.f;
     for (int t = DT_256; t >= 0; --t) {
-        if (T[t].us < 0.f || (t == DT_128x128_PAIR && kbytes % 128 != 0)) continue;
+        if (T.tile[t].us < 0.f || (t == DT_128x128_PAIR && kbytes % 128 != 0) || (t == DT_32x256 && (M > 32 || KT > 8)))
+            continue;
         if (!(t == DT_256 ? fits(std::min<int64_t>(M, 256), std::min<int64_t>(N, 256)) : fits(BM[t], BN[t]))) continue;
         const int64_t tiles = batch * ((M + BM[t] - 1) / BM[t]) * ((N + BN[t] - 1) / BN[t]);
         const int64_t slots = t == DT_128x128_PAIR ? 2 * ncu : ncu;
-        const float us = (float)((tiles + slots - 1) / slots) * (KT * T[t].us + T[t].e);
+        const TileCost c = t == DT_128x128_PAIR && tiles <= ncu ? T.alone : T.tile[t];
+        const float us = (float)((tiles + slots - 1) / slots) * (KT * c.us + c.e);
         if (best_us == 0.f || us < best_us) {
             best = t;
             best_us = us;
@@ -848,8 +864,8 @@ static int dense_tile_plan(int mode, const DenseParams& p, int64_t batch, const 
     }
     if (split != nullptr && fits(128, 128)) {
         const float kt = (float)split->kt_split;
-        const float us = split->geo == GEO_128x64 ? kt * 0.345f + 5.7f
-                                                  : kt * (mode == MODE_BF16 ? 0.5f : 0.4f) + 4.2f + 1.3f * (float)split->splits;
+        const float us = split->geo == GEO_128x64 ? kt * T.split64_us + T.split64_e
+                                                  : kt * T.split_us + T.split_e + T.split_parts * (float)split->splits;
         if (best == DT_NONE || us < best_us) best = DT_SPLIT;
     }
     return best;
@@ -934,17 +950,20 @@ static int launch_dense_whole(DenseParams& p, hipStream_t stream) {
 }
 
 // The narrow path: A8W8 with at most 32 K-steps, and at most 16 rows where the
-// 16-column workgroups fit one per CU, 4 where they come to more than four
-// rounds, 1 between (measured on MI355X against the small tiles: 1x4096x4096
-// 4.4 us and 5.9, 16x4096x4096 5.7 and 6.1, 4x28672x4096 23.1 and 25.0,
-// 8x28672x4096 26.1 and 25.2, 1x14336x4096 11.4 and 11.7, 4x6144x4096 7.4 and
-// 7.1; with 128 K-steps 4x512x16384 12.0 and 10.4). Its buffer offsets are
-// 32-bit.
+// 16-column workgroups fit one per CU (measured on MI355X against the small
+// tiles: 1x4096x4096 4.0 us and 5.4, 16x4096x4096 5.4 both). More workgroups
+// start one after another, 0.9 us per round of them whatever K is (1x28672x128
+// 8.3 us, 4.0 on small tiles; 1x6144x4096 6.2, 5.4), which only a stream that is
+// long by itself hides: from 24 K-steps on, 1 row from two rounds (1x9216x4096
+// 8.5, 8.9; 4 rows 9.4, 9.0) and 4 rows from three (4x12288x4096 9.6, 10.6;
+// 4x28672x4096 19.8, 20.6; 8x28672x4096 22.0, 20.6; 4x28672x2048 14.6, 12.8).
+// Its buffer offsets are 32-bit.
 static bool use_narrow(int mode, int64_t M, int64_t N, int64_t kbytes, int64_t lda, int64_t ldb, int64_t batch) {
     const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
     if (mode != MODE_A8W8 || M < 1 || kbytes % 128 != 0 || kbytes / 128 > NARROW_MAX_STEPS) return false;
     const int64_t wgs = batch * ((N + 15) / 16);
-    return M <= (wgs <= ncu ? NARROW_MAX_M : wgs > 4 * ncu ? 4 : 1) && 16 * ldb < (1ll << 31) && 16 * lda < (1ll << 31);
+    const int64_t rows = wgs <= ncu ? NARROW_MAX_M : kbytes / 128 < 24 || wgs < 2 * ncu ? 0 : wgs < 3 * ncu ? 1 : 4;
+    return M <= rows && 16 * ldb < (1ll << 31) && 16 * lda < (1ll << 31);
 }
 
 template <int MODE>
@@ -974,6 +993,7 @@ static int launch_dense(DenseParams& p, void* ws, size_t ws_bytes, hipStream_t s
         case DT_32x32: return launch_dense_kgroup<KgCfg<MODE, 1, 1, 4, 1, 1, 4>>(p, stream);
         case DT_32x64: return launch_dense_kgroup<KgCfg<MODE, 1, 1, 4, 1, 2, 3 - M4>>(p, stream);
         case DT_32x128: return launch_dense_kgroup<KgCfg<MODE, 1, 1, 4 - M4, 1, 4, 2>>(p, stream);
+        case DT_32x256: return launch_dense_kgroup<KgCfg<MODE, 1, 4, 1, 1, 2, 3>>(p, stream);
         case DT_64x64: return launch_dense_kgroup<KgCfg<MODE, 1, 1, 4, 2, 2, 2>>(p, stream);
         case DT_128x64: return launch_dense_kgroup<KgCfg<MODE, 4, 1, 2, 1, 2, 3 - M4>>(p, stream);
         case DT_128x128: return launch_dense_kgroup<KgCfg<MODE, 4, 2, 1, 1, 2, 4>>(p, stream);

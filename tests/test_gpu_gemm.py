@@ -528,6 +528,29 @@ def test_gemm_small_tiles(orc, mode, M, N, KT):
     assert_gemm_close(host_bf16_f32(C), ref, f"{mode} small tiles {M}x{N}x{K}")
 
 
+# Up to 32 rows of a short K with many columns (32 x 256 tiles; one half K-tile,
+# whole ones, a ragged last tile), and the A8W8 streaming kernel's limits: one
+# 16-column workgroup per CU, 24 K-steps on two and on three per CU.
+@pytest.mark.parametrize("mode,M,N,K", [("a8w8", 30, 28676, 320), ("a8w8", 1, 28676, 1024), ("a8w8", 32, 28676, 128),
+                                        ("mxfp4", 17, 28676, 640), ("mxfp4", 32, 28676, 2048), ("bf16", 9, 28676, 160),
+                                        ("bf16", 32, 28676, 512), ("a8w8", 2, 8196, 3072), ("a8w8", 1, 8196, 3072),
+                                        ("a8w8", 4, 12292, 3072), ("a8w8", 5, 12292, 3072), ("a8w8", 1, 12292, 2944)])
+def test_gemm_few_rows_wide(orc, mode, M, N, K):
+    require_gpu()
+    if mode == "bf16":
+        xa, xw = orc.randn_bf16((M, K), seed=M), orc.randn_bf16((N, K), seed=N, std=0.02)
+        bf = lambda x: torch.from_numpy(x.view(np.int16)).view(torch.bfloat16).cuda()
+        C = host_bf16_f32(hkq.gemm_bf16(bf(xa), bf(xw)))
+        ref = orc.gemm_bf16_ref(xa, xw)
+    elif mode == "a8w8":
+        A, B, sa, sb = a8w8_inputs(orc, M, N, K, seed=M + N + K)
+        C, ref = run_a8w8(A, B, sa, sb), orc.gemm_a8w8_ref_f32(A, B, sa, sb)
+    else:
+        ops = mx_inputs(orc, M, N, K, seed=M * 3 + K)
+        C, ref = run_mxfp4(*ops), orc.gemm_mxfp4_ref_f32(*ops)
+    assert_gemm_close(C, ref, f"{mode} {M}x{N}x{K}")
+
+
 # Rows far apart (a view of a wide buffer): a 256-row tile's rows would lie past
 # its 2 GiB buffer range, so the plans keep to tiles whose rows a 32-bit offset
 # reaches. Weight rows 16 MiB apart with N past one 128-column tile, K above the
