@@ -571,75 +571,95 @@ __global__ __launch_bounds__(64 * WM * WN, MINB) void dense_tile_kernel(const De
 }
 
 // ---------------------------------------------------------------------------
-// Narrow M (M <= 16 and short K, where 16-column workgroups pay): a streaming
-// path on the 16x16x128 MFMA. Workgroup u owns the 16 columns [16u, 16u + 16) of C for all
-// M rows; its 4 waves split K (wave w takes the 128-value K-steps
-// [w*S/4, (w+1)*S/4) of S) and load their operand fragments from memory
-// straight into registers, all steps at once. The waves' sums meet in LDS, and
-// wave 0 adds them in wave order, applies the scales and writes C.
+// Narrow M (few rows and short K, where 16-column workgroups pay; FP8 and FP4):
+// a streaming path on the 16x16x128 MFMA. Workgroup (u, z) owns the 16 columns
+// [16u, 16u + 16) of C for rows [16z, 16z + 16); its 4 waves split K (wave w
+// takes the 128-value K-steps [w*S/4, (w+1)*S/4) of S) and load their operand
+// fragments from memory straight into registers, all steps at once. The waves'
+// sums meet in LDS, and wave 0 adds them in wave order, applies the scales and
+// writes C.
 //
 // Fragment layout of the 16x16x128 MFMA (verified on gfx950): lane l supplies
-// row l % 16 and 32 K-values of the 128-deep slice; lane l, register i of the
-// result holds D[4*(l/16) + i][l % 16]. The MFMA A operand is the weight rows
-// (n), B the activation rows (m): a lane holds 4 consecutive n of one m. A sum
-// over K does not depend on which lane supplies which K-value as long as both
-// operands agree, so a lane takes bytes [16q, 16q+16) and [64+16q, 64+16q+16)
-// of the step (q = l/16): each 16-byte load covers 64 contiguous bytes of 16
-// rows.
+// row l % 16 and 32 K-values of the 128-deep slice (FP8: 32 bytes; FP4: 16 bytes
+// in the low 4 VGPRs, scaled per lane by its 32-value block's e8m0); lane l,
+// register i of the result holds D[4*(l/16) + i][l % 16]. The MFMA A operand is
+// the weight rows (n), B the activation rows (m): a lane holds 4 consecutive n of
+// one m. An FP8 sum over K does not depend on which lane supplies which K-value
+// as long as both operands agree, so an FP8 lane takes bytes [16q, 16q+16) and
+// [64+16q, 64+16q+16) of the step (q = l/16): each 16-byte load covers 64
+// contiguous bytes of 16 rows.
 //
 // Bound by latency: one memory round trip for everything, then the sums'
 // exchange. All of a wave's steps (at most 8) are in flight at once, the
 // epilogue's scales before them, and no look-ahead load is issued past them:
 // 4x4096x4096 5.75 -> 4.9 us against a loop of 8-step rings whose look-ahead
 // read nothing and whose scales were fetched after the sums.
-constexpr int NARROW_WAVES = 4, NARROW_MAX_M = 16, NARROW_MAX_STEPS = 32;
+constexpr int NARROW_WAVES = 4, NARROW_ROWS = 16, NARROW_MAX_STEPS = 32;
 
-struct NarrowFrag {
-    v4i b0, b1, a0, a1;  // weight row, activation row
-};
-
+template <int MODE>
 __global__ __launch_bounds__(64 * NARROW_WAVES) void narrow_gemm_kernel(const DenseParams pb) {
+    constexpr bool FP4 = MODE == MODE_MXFP4;
+    constexpr int SB = FP4 ? 64 : 128;                      // bytes of a row per K-step
     constexpr int DEPTH = NARROW_MAX_STEPS / NARROW_WAVES;  // K-steps of a wave at most, all in flight together
+    struct Frag {
+        v4i b0, b1, a0, a1;  // weight row, activation row (b1, a1: FP8 only)
+        uint32_t sb, sa;     // FP4: e8m0 scales of the step's 4 blocks (byte q is the lane's)
+    };
     __shared__ v4f red[NARROW_WAVES][64];
     const DenseParams p = batch_slice(pb);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, q = lane >> 4;
-    const int n0 = blockIdx.x * 16;
-    const int S = p.kbytes / 128;
+    const int n0 = blockIdx.x * 16, m0 = blockIdx.z * NARROW_ROWS;
+    const int S = p.kbytes / SB;
     const int s0 = wave * S / NARROW_WAVES, s1 = (wave + 1) * S / NARROW_WAVES;
-    const int rows_b = min(16, p.N - n0);
+    const int rows_a = min(NARROW_ROWS, p.M - m0), rows_b = min(16, p.N - n0);
     const auto rb = make_rsrc(p.B + (int64_t)n0 * p.ldb, (uint32_t)(rows_b * p.ldb));
-    const auto ra = make_rsrc(p.A, (uint32_t)(p.M * p.lda));
+    const auto ra = make_rsrc(p.A + (int64_t)m0 * p.lda, (uint32_t)(rows_a * p.lda));
     const uint32_t b_off = (uint32_t)(r * p.ldb + 16 * q), a_off = (uint32_t)(r * p.lda + 16 * q);
+    const auto rsb = make_rsrc(FP4 ? static_cast<const uint8_t*>(p.sb) + (int64_t)n0 * p.lsb : p.B,
+                               FP4 ? (uint32_t)((rows_b - 1) * p.lsb + 4 * S) : 0u);
+    const auto rsa = make_rsrc(FP4 ? static_cast<const uint8_t*>(p.sa) + (int64_t)m0 * p.lsa : p.A,
+                               FP4 ? (uint32_t)((rows_a - 1) * p.lsa + 4 * S) : 0u);
 
     // Steps at or past s1 read zeros (their MFMAs add nothing): offsets with
     // the OOB bit set are past every buffer's range.
-    auto load = [&](int s, NarrowFrag& f) {
-        const uint32_t kb = (uint32_t)s * 128 | (s < s1 ? 0u : OOB);
+    auto load = [&](int s, Frag& f) {
+        const uint32_t kill = s < s1 ? 0u : OOB, kb = (uint32_t)s * SB | kill;
         f.b0 = __builtin_amdgcn_raw_buffer_load_b128(rb, b_off + kb, 0, 0);
-        f.b1 = __builtin_amdgcn_raw_buffer_load_b128(rb, b_off + kb + 64, 0, 0);
+        if constexpr (!FP4) f.b1 = __builtin_amdgcn_raw_buffer_load_b128(rb, b_off + kb + 64, 0, 0);
         f.a0 = __builtin_amdgcn_raw_buffer_load_b128(ra, a_off + kb, 0, 0);
-        f.a1 = __builtin_amdgcn_raw_buffer_load_b128(ra, a_off + kb + 64, 0, 0);
+        if constexpr (!FP4) f.a1 = __builtin_amdgcn_raw_buffer_load_b128(ra, a_off + kb + 64, 0, 0);
+        if constexpr (FP4) {
+            f.sb = __builtin_amdgcn_raw_buffer_load_b32(rsb, (uint32_t)(r * p.lsb) + ((uint32_t)s * 4 | kill), 0, 0);
+            f.sa = __builtin_amdgcn_raw_buffer_load_b32(rsa, (uint32_t)(r * p.lsa) + ((uint32_t)s * 4 | kill), 0, 0);
+        }
     };
     v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
-    auto mma = [&](const NarrowFrag& f) {
-        const v8i a = v8i{f.b0[0], f.b0[1], f.b0[2], f.b0[3], f.b1[0], f.b1[1], f.b1[2], f.b1[3]};
-        const v8i b = v8i{f.a0[0], f.a0[1], f.a0[2], f.a0[3], f.a1[0], f.a1[1], f.a1[2], f.a1[3]};
-        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, acc, 0, 0, 0, 127, 0, 127);
+    auto mma = [&](const Frag& f) {
+        if constexpr (FP4) {
+            const v8i a = v8i{f.b0[0], f.b0[1], f.b0[2], f.b0[3], 0, 0, 0, 0};
+            const v8i b = v8i{f.a0[0], f.a0[1], f.a0[2], f.a0[3], 0, 0, 0, 0};
+            acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, acc, 4, 4, 0, (int)(f.sb >> (8 * q)), 0,
+                                                                   (int)(f.sa >> (8 * q)));
+        } else {
+            const v8i a = v8i{f.b0[0], f.b0[1], f.b0[2], f.b0[3], f.b1[0], f.b1[1], f.b1[2], f.b1[3]};
+            const v8i b = v8i{f.a0[0], f.a0[1], f.a0[2], f.a0[3], f.a1[0], f.a1[1], f.a1[2], f.a1[3]};
+            acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, acc, 0, 0, 0, 127, 0, 127);
+        }
     };
     // the epilogue's scales go out before the operands: no memory latency
     // follows the K loop
-    const int n = n0 + 4 * q, m = r;
+    const int n = n0 + 4 * q, m = m0 + r;
     const bool in = n < p.N && m < p.M;  // N % 4 == 0: n .. n+3 all in or all out
-    float4 cs = make_float4(0.f, 0.f, 0.f, 0.f);
-    float a = 0.f;
-    if (in) {
+    float4 cs = make_float4(1.f, 1.f, 1.f, 1.f);
+    float a = 1.f;
+    if (!FP4 && in) {
         cs = *reinterpret_cast<const float4*>(static_cast<const float*>(p.sb) + n);
         a = static_cast<const float*>(p.sa)[m];
     }
     const float4 c = bias4(p, n);
-    NarrowFrag f[DEPTH];
+    Frag f[DEPTH];
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) load(s0 + d, f[d]);
 #pragma unroll
@@ -949,21 +969,28 @@ static int launch_dense_whole(DenseParams& p, hipStream_t stream) {
     return hkq_launch_status();
 }
 
-// The narrow path: A8W8 with at most 32 K-steps, and at most 16 rows where the
-// 16-column workgroups fit one per CU (measured on MI355X against the small
-// tiles: 1x4096x4096 4.0 us and 5.4, 16x4096x4096 5.4 both). More workgroups
-// start one after another, 0.9 us per round of them whatever K is (1x28672x128
-// 8.3 us, 4.0 on small tiles; 1x6144x4096 6.2, 5.4), which only a stream that is
-// long by itself hides: from 24 K-steps on, 1 row from two rounds (1x9216x4096
-// 8.5, 8.9; 4 rows 9.4, 9.0) and 4 rows from three (4x12288x4096 9.6, 10.6;
-// 4x28672x4096 19.8, 20.6; 8x28672x4096 22.0, 20.6; 4x28672x2048 14.6, 12.8).
-// Its buffer offsets are 32-bit.
-static bool use_narrow(int mode, int64_t M, int64_t N, int64_t kbytes, int64_t lda, int64_t ldb, int64_t batch) {
+// The narrow path: FP8 and FP4 with at most 32 K-steps, up to 64 rows in groups
+// of 16 while there is a CU for every 16-column workgroup of every group; the
+// groups' activation loads grow with K, so FP4, whose small tiles are the
+// cheaper ones, takes more than 16 steps to 8 rows only. Measured on MI355X
+// against the small tiles, us: A8W8 1x4096x4096 4.0 and 5.3, 16x4096x4096 5.4
+// both, 32x1000x256 3.7 and 4.1, 64x1000x4096 5.6 and 5.7; MXFP4 1x1000x256 3.7
+// and 3.9, 32x1000x1024 3.7 and 4.2, 8x2048x4096 4.6 and 4.7, 16x2048x3072 4.8
+// and 4.5. More workgroups start one after another, 0.9 us per round of them
+// whatever K is (A8W8 1x28672x128 8.3 us, 4.0 on small tiles; 1x6144x4096 6.2,
+// 5.4), which only a stream that is long by itself hides: A8W8 from 24 K-steps
+// on, 1 row from two rounds (1x9216x4096 8.5, 8.9; 4 rows 9.4, 9.0) and 4 rows
+// from three (4x12288x4096 9.6, 10.6; 4x28672x4096 19.8, 20.6; 8x28672x4096
+// 22.0, 20.6; 4x28672x2048 14.6, 12.8). Its buffer offsets are 32-bit.
+static bool use_narrow(int mode, const DenseParams& p, int64_t batch) {
+    const int64_t step = mode == MODE_MXFP4 ? 64 : 128, S = p.kbytes / step;
+    if (p.M < 1 || p.kbytes % step != 0 || S > NARROW_MAX_STEPS) return false;
+    const int64_t wide = (1ll << 31) / NARROW_ROWS;
+    if (p.lda >= wide || p.ldb >= wide || p.lsa >= wide || p.lsb >= wide) return false;
     const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
-    if (mode != MODE_A8W8 || M < 1 || kbytes % 128 != 0 || kbytes / 128 > NARROW_MAX_STEPS) return false;
-    const int64_t wgs = batch * ((N + 15) / 16);
-    const int64_t rows = wgs <= ncu ? NARROW_MAX_M : kbytes / 128 < 24 || wgs < 2 * ncu ? 0 : wgs < 3 * ncu ? 1 : 4;
-    return M <= rows && 16 * ldb < (1ll << 31) && 16 * lda < (1ll << 31);
+    const int64_t groups = (p.M + NARROW_ROWS - 1) / NARROW_ROWS, wgs = batch * ((p.N + 15) / 16);
+    if (groups <= 4 && groups * wgs <= ncu) return mode == MODE_A8W8 || S <= 16 || p.M <= 8;
+    return mode == MODE_A8W8 && S >= 24 && p.M <= (wgs >= 3 * ncu ? 4 : wgs >= 2 * ncu ? 1 : 0);
 }
 
 template <int MODE>
@@ -975,10 +1002,12 @@ static int launch_dense(DenseParams& p, void* ws, size_t ws_bytes, hipStream_t s
         p.lda = p.kbytes;
         if (MODE == MODE_MXFP4) p.lsa = p.K / 32;
     }
-    if (use_narrow(MODE, p.M, p.N, p.kbytes, p.lda, p.ldb, batch)) {
-        const dim3 grid((unsigned)((p.N + 15) / 16), (unsigned)batch);
-        narrow_gemm_kernel<<<grid, 64 * NARROW_WAVES, 0, stream>>>(p);
-        return hkq_launch_status();
+    if constexpr (MODE != MODE_BF16) {
+        if (use_narrow(MODE, p, batch)) {
+            const dim3 grid((unsigned)((p.N + 15) / 16), (unsigned)batch, (unsigned)((p.M + NARROW_ROWS - 1) / NARROW_ROWS));
+            narrow_gemm_kernel<MODE><<<grid, 64 * NARROW_WAVES, 0, stream>>>(p);
+            return hkq_launch_status();
+        }
     }
     // the split partials and their reduction are per 2-D GEMM without bias
     DensePlan pl{};

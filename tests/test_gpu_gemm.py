@@ -529,12 +529,15 @@ def test_gemm_small_tiles(orc, mode, M, N, KT):
 
 
 # Up to 32 rows of a short K with many columns (32 x 256 tiles; one half K-tile,
-# whole ones, a ragged last tile), and the A8W8 streaming kernel's limits: one
-# 16-column workgroup per CU, 24 K-steps on two and on three per CU.
+# whole ones, a ragged last tile), and the streaming kernel's limits: a CU for
+# every 16-column workgroup of up to four groups of 16 rows (FP4 past 16 K-steps:
+# 8 rows), and for A8W8 24 K-steps on two and on three rounds of workgroups.
 @pytest.mark.parametrize("mode,M,N,K", [("a8w8", 30, 28676, 320), ("a8w8", 1, 28676, 1024), ("a8w8", 32, 28676, 128),
                                         ("mxfp4", 17, 28676, 640), ("mxfp4", 32, 28676, 2048), ("bf16", 9, 28676, 160),
                                         ("bf16", 32, 28676, 512), ("a8w8", 2, 8196, 3072), ("a8w8", 1, 8196, 3072),
-                                        ("a8w8", 4, 12292, 3072), ("a8w8", 5, 12292, 3072), ("a8w8", 1, 12292, 2944)])
+                                        ("a8w8", 4, 12292, 3072), ("a8w8", 5, 12292, 3072), ("a8w8", 1, 12292, 2944),
+                                        ("a8w8", 33, 1000, 4096), ("a8w8", 64, 1020, 384), ("mxfp4", 17, 1000, 2048),
+                                        ("mxfp4", 64, 1020, 128), ("mxfp4", 8, 4096, 4096), ("mxfp4", 9, 4092, 2176)])
 def test_gemm_few_rows_wide(orc, mode, M, N, K):
     require_gpu()
     if mode == "bf16":
