@@ -424,6 +424,11 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
 // the MoE kernels have one K group: they add K-tile after K-tile in K order, as
 // the block-pair kernels do, so every tile size and both weight layouts give
 // the same bits. Bound by the weights' way from HBM: a tile's rows should hold
+//
+// A short K's 64 x 128 tiles that give the CUs no more than one round of two get
+// a second one from the experts with more than 64 rows: they end at `rows_short`
+// mean rows there (block-scale down projection of 32 experts, K 2816, N 2048,
+// 400 tokens: r = 50, 43.0 us on 64 x 128, 36.5 on 128 x 256, pairs 38.1).
 // an expert's rows, and the rings of the workgroups of a CU 120 to 150 KB of
 // K-tiles in flight. Beyond about one routing block per expert (`pairs_short`,
 // `pairs_long` rows, for K up to 3072 and above) the block-pair kernels read
@@ -449,11 +454,15 @@ enum MoeTile { MOET_64x64, MOET_64x128, MOET_128x128, MOET_128x256, MOET_PAIRS }
 // workgroups (at most 512 threads each) of the widest small-tile grid: within
 // what one launch can hold
 inline bool kg_moe_grid(int64_t grid_m, int64_t N) { return grid_m * ((N + 63) / 64) * 2 < (1ll << 23); }
-inline MoeTile moe_tile(int64_t routed, int64_t experts, int64_t K, int64_t pairs_short, int64_t pairs_long) {
+inline MoeTile moe_tile(int64_t routed, int64_t experts, int64_t N, int64_t K, int64_t ncu, int64_t rows_short,
+                        int64_t pairs_short, int64_t pairs_long) {
     const int64_t r = routed / (experts > 0 ? experts : 1);
-    if (K <= 3072) return r <= 56 ? MOET_64x128 : r <= pairs_short ? MOET_128x256 : MOET_PAIRS;
+    if (K <= 3072) {
+        const bool one_round = experts * ((N + 127) / 128) <= 2 * ncu;
+        return r <= (one_round ? rows_short : 52) ? MOET_64x128 : r <= pairs_short ? MOET_128x256 : MOET_PAIRS;
+    }
     if (r <= 48) return MOET_64x64;
-    return r <= 112 ? MOET_128x128 : r <= pairs_long ? MOET_128x256 : MOET_PAIRS;
+    return r > pairs_long ? MOET_PAIRS : r <= 112 ? MOET_128x128 : MOET_128x256;
 }
 
 }  // namespace hkq

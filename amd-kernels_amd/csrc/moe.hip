@@ -1416,13 +1416,22 @@ static int moe_a8w8_impl(const void* X, const void* W, void* Y, const float* x_s
     // 32 experts of 2048 x 2816, one token's layer 26 both).
     const int64_t routed = gather ? T * topk : T;
     const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
-    const bool few = std::min(routed, E) * ((N + 127) / 128) < ncu;
+    // So do those with one or two rows per expert over a long K, where the
+    // stream's 16-row workgroups keep as much in flight and no tile is padded
+    // (16 experts, K 8192, N 5120, 16 rows 89 us against 105, 28 rows 93 and 106;
+    // 8 of K 14336, N 4096, 8 rows 49.5 and 52; 16 rows 78 and 72).
+    const bool few = std::min(routed, E) * ((N + 127) / 128) < ncu || (K > 6144 && 2 * routed > E && routed < 2 * E);
     const bool decode = (routed <= 32 || (routed <= MOE_NARROW_MAX_ROWS && N <= 4096)) && !wt && K % 128 == 0 &&
                         64 * stride_w < (1ll << 31);
     if (!(few && decode) && !wt && K % 128 == 0 && !bias && (!w_scale || ws_stride_n == 0 || p.ws_vec) &&
         256 * stride_w < (1ll << 31) && kg_moe_grid(grid_m, N)) {
         constexpr int B = MODE_A8W8;
-        switch (moe_tile(routed, E, K, 128, 352)) {
+        // from two rounds of pair tiles on, a long K gains nothing on 128-row
+        // tiles and skewed routing loses: gate/up of 8 experts of 4096 x 14336,
+        // 1000 tokens 280 us on pairs, 302 on 128 x 256; half of the rows on one
+        // expert 298 and 345
+        const bool many = E * ((N + MOE_BN - 1) / MOE_BN) >= 2 * ncu;
+        switch (moe_tile(routed, E, N, K, ncu, 56, 128, many ? 48 : 352)) {
             case MOET_64x64: return launch_moe_tile<KgCfg<B, 2, 2, 1, 1, 1, 3>, 3>(p, stream);
             case MOET_64x128: return launch_moe_tile<KgCfg<B, 2, 4, 1, 1, 1, 3>, 2>(p, stream);
             case MOET_128x128: return launch_moe_tile<KgCfg<B, 4, 2, 1, 1, 2, 4>, 1>(p, stream);
@@ -1540,6 +1549,11 @@ static int moe_mxfp4_impl(const void* A, const void* B, void* C, const void* A_m
     // 37: 160 / 158 / 184 / 182; 55: 198 / 188 / 177 / 188; 75: 275 / 273 / 181 /
     // 196; 128: - / - / - / pairs win; 32 experts of 2048 x 2816: r = 1: 41 / 43 /
     // 50 / 46; 7: 57 / 58 / 68 / 60; 37: 61 / 63 / 73 / 64.
+    // A short K's down projections in no more than one round of 64-column tiles
+    // (`one_round`) end at 28, their experts of more than 64 rows adding a second
+    // round (32 experts, K 2816, N 2048, 300 tokens 21.4 against 20.5 on pairs, 400
+    // 27.0 and 23.8); from four rounds of pair tiles on (`many`) those win from 48
+    // (128 experts, K 4096, N 3072, 850 tokens 192 and 183, 1000 195 and 188).
     // Where the tiled grid gives fewer than a quarter of the CUs work and at most
     // 32 entries are valid, 32 x 32 tiles with K in four (one token's down
     // projection, K 14336, N 4096: 14 us, streaming kernel 22, 64 x 64 tiles 33);
@@ -1551,11 +1565,13 @@ static int moe_mxfp4_impl(const void* A, const void* B, void* C, const void* A_m
         256 * stride_bn < (1ll << 31) && 256 * stride_bmxn < (1ll << 31) && kg_moe_grid(grid_m, N)) {
         constexpr int B = MODE_MXFP4;
         if (decode) return launch_moe_fp4_tile<KgCfg<B, 1, 1, 4, 1, 1, 2>, 2>(p, stream);
-        if (r <= (K > 3072 ? 20 : 56)) return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 1, 1, 2>, 3>(p, stream);
-        if (r <= 56) return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 1, 2, 2>, 2>(p, stream);
+        const bool one_round = num_experts * ((N + 127) / 128) <= 2 * ncu;
+        if (r <= (K > 3072 ? 20 : one_round ? 28 : 56)) return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 1, 1, 2>, 3>(p, stream);
+        const bool many = num_experts * ((N + MOE_BN - 1) / MOE_BN) >= 4 * ncu;
+        if (r <= (many ? 48 : 56) && K > 3072) return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 1, 2, 2>, 2>(p, stream);
         // with more blocks than experts some expert holds several: the pairs
         // (half of 300 tokens' entries on one expert, gate/up 122 against 144)
-        if (r <= 112 && K > 3072 && grid_m <= num_experts)
+        if (r <= 112 && K > 3072 && grid_m <= num_experts && !many)
             return launch_moe_fp4_tile<KgCfg<B, 2, 2, 1, 2, 2, 2>, 2>(p, stream);
     }
     // K % 256 == 128, or weight rows too wide for the small tiles: the streaming

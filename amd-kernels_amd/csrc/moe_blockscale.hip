@@ -787,7 +787,7 @@ static int moe_blockscale_impl(const void* X, const void* W, void* Y, const floa
         // weights, one column scale per 32 columns, K-contiguous row scales)
         if (ntile && !wt && xs_stride_k == 1 && kg_moe_grid(grid_m, N)) {
             constexpr int B = MODE_BLOCKSCALE;
-            switch (moe_tile(gather ? T * topk : T, E, K, 112, 256)) {
+            switch (moe_tile(gather ? T * topk : T, E, N, K, p.ncu > 0 ? p.ncu : 256, 44, 112, 256)) {
                 case MOET_64x64: return launch_moe_bs_tile<KgCfg<B, 2, 2, 1, 1, 1, 3>, 3>(p, stream);
                 case MOET_64x128: return launch_moe_bs_tile<KgCfg<B, 2, 4, 1, 1, 1, 3>, 2>(p, stream);
                 case MOET_128x128: return launch_moe_bs_tile<KgCfg<B, 4, 2, 1, 1, 2, 4>, 1>(p, stream);
