@@ -702,7 +702,7 @@ template <class Cfg>
 __global__ __launch_bounds__(Cfg::THREADS, 1) void dense_kgroup_kernel(const DenseParams pb) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
     HKQ_LDS uint8_t* smem = (HKQ_LDS uint8_t*)smem_raw;
-    constexpr int MODE = Cfg::MODE, BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TMO = Cfg::TMO;
+    constexpr int MODE = Cfg::MODE, BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TM = Cfg::TM;
     const DenseParams p = batch_slice(pb);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -739,14 +739,14 @@ __global__ __launch_bounds__(Cfg::THREADS, 1) void dense_kgroup_kernel(const Den
             src.s_off[i] = (uint32_t)(r * (q < Cfg::PA ? p.lsa : p.lsb)) + kg_piece_half(lane);
         }
     }
-    const int mw = m0 + (wg / Cfg::WN * Cfg::TM + (Cfg::SPREAD ? kg * TMO : 0)) * 32, nw = n0 + wg % Cfg::WN * TN * 32;
-    EpiScales<MODE, TMO, TN> sc;
+    const int mw = m0 + wg / Cfg::WN * TM * 32, nw = n0 + wg % Cfg::WN * TN * 32;
+    EpiScales<MODE, TM, TN> sc;
     sc.load(p, lane, mw, nw);
 
-    v16f acc[TN][TMO];
+    v16f acc[TN][TM];
     kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
-    if (!Cfg::SPREAD && kg != 0) return;
-    dense_epilogue_global<MODE, 0, 0, TMO, TN>(p, acc, sc, smem, Cfg::SPREAD ? wave : wg, lane, mw, nw);
+    if (kg != 0) return;
+    dense_epilogue_global<MODE, 0, 0, TM, TN>(p, acc, sc, smem, wg, lane, mw, nw);
 }
 
 template <class Cfg>

@@ -316,7 +316,7 @@ template <class Cfg, bool GN1>
 __global__ __launch_bounds__(Cfg::THREADS, 1) void blockscale_tile_kernel(const BlockScaleParams p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
     HKQ_LDS uint8_t* smem = (HKQ_LDS uint8_t*)smem_raw;
-    constexpr int BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TMO = Cfg::TMO;
+    constexpr int BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TM = Cfg::TM;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wg = wave % Cfg::GW, kg = wave / Cfg::GW;
@@ -357,16 +357,15 @@ __global__ __launch_bounds__(Cfg::THREADS, 1) void blockscale_tile_kernel(const 
         src.c_off[i] = c < rows_b ? (uint32_t)(n0 + c) * 4u : OOB;
     }
 
-    v16f acc[TN][TMO];
+    v16f acc[TN][TM];
     kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
-    if (!Cfg::SPREAD && kg != 0) return;
+    if (kg != 0) return;
 
-    const int mw = m0 + (wg / Cfg::WN * Cfg::TM + (Cfg::SPREAD ? kg * TMO : 0)) * 32, nw = n0 + wg % Cfg::WN * TN * 32;
+    const int mw = m0 + wg / Cfg::WN * TM * 32, nw = n0 + wg % Cfg::WN * TN * 32;
     auto one = [](int) { return 1.0f; };
     auto ones = [](int, int) { return make_float4(1.f, 1.f, 1.f, 1.f); };
-    const int ep = Cfg::SPREAD ? wave : wg;
     if (p.ca) {
-        MulAddElem<TMO> e;
+        MulAddElem<TM> e;
         e.ca = p.ca;
         e.cb = p.cb;
         e.ldca = p.ldca;
@@ -376,9 +375,9 @@ __global__ __launch_bounds__(Cfg::THREADS, 1) void blockscale_tile_kernel(const 
         e.mw = mw;
         e.nw = nw;
         e.lane = lane;
-        store_tile_bf16<TMO, TN>(acc, smem, ep, lane, p.C, p.ldc, p.M, p.N, mw, nw, p.c16 != 0, one, ones, NoBias{}, e);
+        store_tile_bf16<TM, TN>(acc, smem, wg, lane, p.C, p.ldc, p.M, p.N, mw, nw, p.c16 != 0, one, ones, NoBias{}, e);
     } else {
-        store_tile_bf16<TMO, TN>(acc, smem, ep, lane, p.C, p.ldc, p.M, p.N, mw, nw, p.c16 != 0, one, ones, NoBias{});
+        store_tile_bf16<TM, TN>(acc, smem, wg, lane, p.C, p.ldc, p.M, p.N, mw, nw, p.c16 != 0, one, ones, NoBias{});
     }
 }
 

@@ -59,14 +59,10 @@ struct KgCfg {
     static constexpr int RING = SC_AT + 2 * KG * SBLK;
     static_assert(NS >= 2 && (NS - 1) * NLD <= 63, "vmcnt range");
     static_assert(PIECES == 0 || NS <= SBK + 1, "a block is read out before the ring's look-ahead refills its slot");
-    // Sums: with TM % KG == 0 group g keeps m-tiles [g*TMO, (g+1)*TMO) of every
-    // wave tile and receives them from the other groups; otherwise group 0
-    // keeps all.
-    static constexpr bool SPREAD = KG > 1 && TM % KG == 0;
-    static constexpr int TMO = SPREAD ? TM / KG : TM;
-    static constexpr int RED = KG == 1 ? 0 : GW * (KG - 1) * (SPREAD ? KG : 1) * TMO * TN * 4096;
-    // waves that store, and their staging (store_tile_bf16)
-    static constexpr int EP = (SPREAD ? NW : GW) * TMO * 32 * (TN * 64 + 16);
+    // the sums of groups 1 .. KG-1, added by group 0
+    static constexpr int RED = GW * (KG - 1) * TM * TN * 4096;
+    // staging of group 0's waves (store_tile_bf16)
+    static constexpr int EP = GW * TM * 32 * (TN * 64 + 16);
     static constexpr int LDS = RING > RED ? (RING > EP ? RING : EP) : (RED > EP ? RED : EP);
     static_assert(LDS <= 160 * 1024, "LDS budget of a CDNA4 CU");
 };
@@ -127,13 +123,12 @@ __device__ __forceinline__ void lds_load4_s(const v4i& desc, HKQ_LDS void* dst, 
                  : "memory", "m0");
 }
 
-// The K loop. On return group g of the workgroup holds its m-tiles' sums in
-// out[n-tile][0 .. TMO), the LDS is free and every load has landed; with
-// SPREAD every group stores, otherwise only group 0's sums are complete.
+// The K loop. On return group 0 of the workgroup holds the sums in
+// out[n-tile][m-tile], the LDS is free and every load has landed.
 // wg: the wave's index in its group, kg: its group.
 template <class Cfg, bool GATHER>
 __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_LDS uint8_t* smem, int lane, int wg, int kg,
-                                             v16f (&out)[Cfg::TN][Cfg::TMO]) {
+                                             v16f (&out)[Cfg::TN][Cfg::TM]) {
     using KT = typename Cfg::KT;
     constexpr int TM = Cfg::TM, TN = Cfg::TN, NS = Cfg::NS, KG = Cfg::KG, GW = Cfg::GW, NLD = Cfg::NLD;
     constexpr int LA = Cfg::LA, LB = Cfg::LB;
@@ -369,48 +364,32 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
 #pragma unroll
             for (int j = 0; j < TM; ++j) out[i][j] = acc[i][j];
     } else {
-        constexpr int TMO = Cfg::TMO;
         HKQ_LDS v4f* red = reinterpret_cast<HKQ_LDS v4f*>(smem);
-        // sums of m-tiles [m0, m0 + TMO) for the group `to`, from this group
-        // (slot: the sender's rank among the other groups)
-        auto slot = [&](int to, int from) {
-            const int s = from < to ? from : from - 1;
-            return red + ((to * (KG - 1) + s) * GW + wg) * (TMO * TN * 4 * 64) + lane;
-        };
-#pragma unroll
-        for (int to = 0; to < (Cfg::SPREAD ? KG : 1); ++to) {
-            if (kg == to) continue;
-            HKQ_LDS v4f* d = slot(to, kg);
+        auto slot = [&](int from) { return red + ((from - 1) * GW + wg) * (TM * TN * 4 * 64) + lane; };
+        if (kg != 0) {
+            HKQ_LDS v4f* d = slot(kg);
 #pragma unroll
             for (int i = 0; i < TN; ++i)
 #pragma unroll
-                for (int j = 0; j < TMO; ++j)
+                for (int j = 0; j < TM; ++j)
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
-                        const v16f& v = acc[i][to * TMO + j];
-                        d[((i * TMO + j) * 4 + g) * 64] = v4f{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
+                        const v16f& v = acc[i][j];
+                        d[((i * TM + j) * 4 + g) * 64] = v4f{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
                     }
         }
         __syncthreads();
-        // group order, the own sums in their place: the same bits whichever
-        // group a row belongs to
-#pragma unroll
-        for (int me = 0; me < (Cfg::SPREAD ? KG : 1); ++me) {
-            if (kg != me) continue;
+        if (kg == 0) {
 #pragma unroll
             for (int i = 0; i < TN; ++i)
 #pragma unroll
-                for (int j = 0; j < TMO; ++j)
+                for (int j = 0; j < TM; ++j)
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
-                        v4f v = v4f{0.f, 0.f, 0.f, 0.f};
+                        const v16f& o = acc[i][j];
+                        v4f v = v4f{o[4 * g], o[4 * g + 1], o[4 * g + 2], o[4 * g + 3]};
 #pragma unroll
-                        for (int from = 0; from < KG; ++from) {
-                            const v16f& o = acc[i][me * TMO + j];
-                            const v4f x = from == me ? v4f{o[4 * g], o[4 * g + 1], o[4 * g + 2], o[4 * g + 3]}
-                                                     : slot(me, from)[((i * TMO + j) * 4 + g) * 64];
-                            v = from == 0 ? x : v + x;
-                        }
+                        for (int from = 1; from < KG; ++from) v = v + slot(from)[((i * TM + j) * 4 + g) * 64];
 #pragma unroll
                         for (int e = 0; e < 4; ++e) out[i][j][4 * g + e] = v[e];
                     }
@@ -424,11 +403,6 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
 // the MoE kernels have one K group: they add K-tile after K-tile in K order, as
 // the block-pair kernels do, so every tile size and both weight layouts give
 // the same bits. Bound by the weights' way from HBM: a tile's rows should hold
-//
-// A short K's 64 x 128 tiles that give the CUs no more than one round of two get
-// a second one from the experts with more than 64 rows: they end at `rows_short`
-// mean rows there (block-scale down projection of 32 experts, K 2816, N 2048,
-// 400 tokens: r = 50, 43.0 us on 64 x 128, 36.5 on 128 x 256, pairs 38.1).
 // an expert's rows, and the rings of the workgroups of a CU 120 to 150 KB of
 // K-tiles in flight. Beyond about one routing block per expert (`pairs_short`,
 // `pairs_long` rows, for K up to 3072 and above) the block-pair kernels read
@@ -450,6 +424,11 @@ __device__ __forceinline__ void kgroup_kloop(const KgSrc<Cfg, GATHER>& src, HKQ_
 // x 14336, half of the rows on one expert, 90 tokens 315 -> 302 us, 150 tokens 354
 // -> 340; MXFP4 down projection, 150 tokens 73 -> 49), and an even one loses less
 // than 1 %.
+//
+// A short K's 64 x 128 tiles that give the CUs no more than one round of two get
+// a second one from the experts with more than 64 rows: they end at `rows_short`
+// mean rows there (block-scale down projection of 32 experts, K 2816, N 2048,
+// 400 tokens: r = 50, 43.0 us on 64 x 128, 36.5 on 128 x 256, pairs 38.1).
 enum MoeTile { MOET_64x64, MOET_64x128, MOET_128x128, MOET_128x256, MOET_PAIRS };
 // workgroups (at most 512 threads each) of the widest small-tile grid: within
 // what one launch can hold

@@ -282,7 +282,7 @@ template <class Cfg, int MINB>
 __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_tile_kernel(const MoeParams p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
     HKQ_LDS uint8_t* smem = (HKQ_LDS uint8_t*)smem_raw;
-    constexpr int BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TMO = Cfg::TMO;
+    constexpr int BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TM = Cfg::TM;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wg = wave % Cfg::GW, kg = wave / Cfg::GW;
@@ -309,7 +309,7 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_ti
         const int r = kg_row<Cfg>(i, wg, lane);
         src.b_off[i] = (uint32_t)(r * p.swn) + kg_chunk<Cfg>(r, lane);
     }
-    const int nw = n0 + wg % Cfg::WN * TN * 32, mw = (wg / Cfg::WN * Cfg::TM + (Cfg::SPREAD ? kg * TMO : 0)) * 32;
+    const int nw = n0 + wg % Cfg::WN * TN * 32, mw = wg / Cfg::WN * TM * 32;
     auto token_of = [&](int r) {
         const int s = start + row0 + r;
         if (r >= rows || s >= p.g_len) return -1;
@@ -321,15 +321,15 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_ti
         const int r = kg_row<Cfg>(i, wg, lane), t = token_of(r);
         src.a_off[i] = t < 0 ? OOB : (uint32_t)t * (uint32_t)p.sxm + kg_chunk<Cfg>(r, lane);
     }
-    float rs[TMO];
+    float rs[TM];
 #pragma unroll
-    for (int j = 0; j < TMO; ++j) {
+    for (int j = 0; j < TM; ++j) {
         const int t = p.xs ? token_of(mw + j * 32 + (lane & 31)) : -1;
         rs[j] = !p.xs ? 1.0f : (t < 0 ? 0.0f : p.xs[(int64_t)t * p.xs_tok]);
     }
-    v16f acc[TN][TMO];
+    v16f acc[TN][TM];
     kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
-    if (Cfg::SPREAD || kg == 0) {
+    if (kg == 0) {
         const int s0 = start + row0;
         const int out_rows = min(rows, p.y_rows - s0);
         // no bias, column scales absent, one per expert or one per channel (the launcher checks)
@@ -341,7 +341,7 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_ti
             if (p.ws_n == 0) return make_float4(w[0], w[0], w[0], w[0]);
             return *reinterpret_cast<const float4*>(w + n);
         };
-        store_tile_bf16<TMO, TN>(acc, smem, Cfg::SPREAD ? wave : wg, lane, p.Y + (int64_t)s0 * p.sym, p.sym, out_rows,
+        store_tile_bf16<TM, TN>(acc, smem, wg, lane, p.Y + (int64_t)s0 * p.sym, p.sym, out_rows,
                                  p.N, mw, nw, p.c16 != 0, [&](int j) { return rs[j]; }, col_scale4, NoBias{});
     }
 }
@@ -1079,7 +1079,7 @@ template <class Cfg, int MINB>
 __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_fp4_tile_kernel(const MoeFp4Params p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
     HKQ_LDS uint8_t* smem = (HKQ_LDS uint8_t*)smem_raw;
-    constexpr int BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TMO = Cfg::TMO;
+    constexpr int BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TM = Cfg::TM;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wg = wave % Cfg::GW, kg = wave / Cfg::GW;
@@ -1123,7 +1123,7 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_fp
         const int r = kg_row<Cfg>(i, wg, lane);
         src.b_off[i] = (uint32_t)(r * p.sbn) + kg_chunk<Cfg>(r, lane);
     }
-    const int nw = n0 + wg % Cfg::WN * TN * 32, mw = (wg / Cfg::WN * Cfg::TM + (Cfg::SPREAD ? kg * TMO : 0)) * 32;
+    const int nw = n0 + wg % Cfg::WN * TN * 32, mw = wg / Cfg::WN * TM * 32;
     const float gs = (p.a_scale ? p.a_scale[0] : 1.0f) * (p.b_scale ? p.b_scale[e] : 1.0f);
     auto arow_of = [&](int r) {
         const int id = gate_of(row0 + r);
@@ -1146,24 +1146,24 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_fp
         }
     }
     // the epilogue's gate ids (scatter rows) and routed weights, ahead of the K loop
-    int rid[(TMO * 32 + 63) / 64];
+    int rid[(TM * 32 + 63) / 64];
 #pragma unroll
-    for (int h = 0; h < (TMO * 32 + 63) / 64; ++h) {
+    for (int h = 0; h < (TM * 32 + 63) / 64; ++h) {
         const int r = h * 64 + lane;
-        rid[h] = r < TMO * 32 ? gate_of(row0 + mw + r) : -1;
+        rid[h] = r < TM * 32 ? gate_of(row0 + mw + r) : -1;
     }
-    float rs[TMO];
+    float rs[TM];
 #pragma unroll
-    for (int j = 0; j < TMO; ++j) {
+    for (int j = 0; j < TM; ++j) {
         const int id = gate_of(row0 + mw + j * 32 + (lane & 31));
         rs[j] = (p.topk_w && id >= 0) ? gs * p.topk_w[id] : gs;
     }
-    v16f acc[TN][TMO];
+    v16f acc[TN][TM];
     kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
-    if (Cfg::SPREAD || kg == 0)
-        store_tile_bf16_rows<TMO, TN>(
-            acc, smem, Cfg::SPREAD ? wave : wg, lane, p.C, p.scm, p.N, nw, p.c16 != 0,
-            [&](int r) { return (int64_t)__shfl(rid[TMO > 2 ? r >> 6 : 0], r & 63); }, [&](int j) { return rs[j]; },
+    if (kg == 0)
+        store_tile_bf16_rows<TM, TN>(
+            acc, smem, wg, lane, p.C, p.scm, p.N, nw, p.c16 != 0,
+            [&](int r) { return (int64_t)__shfl(rid[TM > 2 ? r >> 6 : 0], r & 63); }, [&](int j) { return rs[j]; },
             [&](int, int) { return make_float4(1.f, 1.f, 1.f, 1.f); }, NoBias{});
 }
 

@@ -589,7 +589,7 @@ template <class Cfg, int MINB>
 __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_bs_tile_kernel(const MoeBsParams p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem_raw[];
     HKQ_LDS uint8_t* smem = (HKQ_LDS uint8_t*)smem_raw;
-    constexpr int BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TMO = Cfg::TMO;
+    constexpr int BM = Cfg::BM, BN = Cfg::BN, TN = Cfg::TN, TM = Cfg::TM;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wg = wave % Cfg::GW, kg = wave / Cfg::GW;
@@ -641,17 +641,16 @@ __global__ __launch_bounds__(Cfg::THREADS, (Cfg::NW * MINB + 3) / 4) void moe_bs
                            (uint32_t)(lane & 3) * src.bs_step;
         }
     }
-    v16f acc[TN][TMO];
+    v16f acc[TN][TM];
     kgroup_kloop<Cfg>(src, smem, lane, wg, kg, acc);
-    if (Cfg::SPREAD || kg == 0) {
+    if (kg == 0) {
         const int s0 = start + row0;
-        const int mw = (wg / Cfg::WN * Cfg::TM + (Cfg::SPREAD ? kg * TMO : 0)) * 32;
+        const int mw = wg / Cfg::WN * TM * 32;
         const int out_rows = min(rows, p.y_rows - s0);
         auto one = [](int) { return 1.0f; };
         auto ones = [](int, int) { return make_float4(1.f, 1.f, 1.f, 1.f); };
-        const int ep = Cfg::SPREAD ? wave : wg;
         uint16_t* Y = p.Y + (int64_t)s0 * p.sym;
-        store_tile_bf16<TMO, TN>(acc, smem, ep, lane, Y, p.sym, out_rows, p.N, mw, nw, p.c16 != 0, one, ones,
+        store_tile_bf16<TM, TN>(acc, smem, wg, lane, Y, p.sym, out_rows, p.N, mw, nw, p.c16 != 0, one, ones,
                                  [&](int i, int g) {
                                      const int n = nw + i * 32 + 8 * g + 4 * (lane >> 5);
                                      if (!p.bias || n >= p.N) return make_float4(-0.f, -0.f, -0.f, -0.f);
