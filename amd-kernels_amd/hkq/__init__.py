@@ -249,21 +249,16 @@ def gemm_a8w8(A, B, sa, sb, C=None, stream=None, split: bool = True):
 
 def gemm_mxfp4(A, As, B, Bs, C=None, stream=None, split: bool = True):
     """A u8 [M, K/2], As u8 [M, K/32], B u8 [N, K/2], Bs u8 [N, K/32] -> C bf16 [M, N].
-    split=False runs the plain entry point (no workspace, no split-K)."""
+    Its plans split K inside a workgroup only, so no workspace is allocated
+    whatever `split` says."""
     import torch
 
     M, K = A.shape[0], A.shape[1] * 2
     N = B.shape[0]
     if C is None:
         C = torch.empty((M, N), dtype=torch.bfloat16, device=A.device)
-    if not split:
-        call("hkq_gemm_mxfp4", _ptr(A), _ptr(As), _ptr(B), _ptr(Bs), _ptr(C), M, N, K, A.stride(0), B.stride(0),
-             As.stride(0), Bs.stride(0), C.stride(0), _stream(stream))
-        return C
-    ws = _workspace(lib().hkq_gemm_mxfp4_workspace(M, N, K), A)
-    call("hkq_gemm_mxfp4_ws", _ptr(A), _ptr(As), _ptr(B), _ptr(Bs), _ptr(C), M, N, K, A.stride(0), B.stride(0),
-         As.stride(0), Bs.stride(0), C.stride(0), _ptr(ws) if ws is not None else None,
-         ws.numel() if ws is not None else 0, _stream(stream))
+    call("hkq_gemm_mxfp4", _ptr(A), _ptr(As), _ptr(B), _ptr(Bs), _ptr(C), M, N, K, A.stride(0), B.stride(0),
+         As.stride(0), Bs.stride(0), C.stride(0), _stream(stream))
     return C
 
 

@@ -167,9 +167,10 @@ int hkq_gemm_mxfp4(const void* A, const void* As, const void* B, const void* Bs,
                    int64_t K, int64_t lda, int64_t ldb, int64_t ldsa, int64_t ldsb, int64_t ldc, hkq_stream_t stream);
 
 /* hkq_gemm_mxfp4 with a caller-provided workspace, the interface of
- * hkq_gemm_a8w8_ws (no counterpart in the reference; gemm_afp4wfp4_tk calls it
- * with a workspace from torch's allocator). The plans of the MXFP4 GEMM split K
- * inside a workgroup only and leave the workspace alone. */
+ * hkq_gemm_a8w8_ws (no counterpart in the reference). The plans of the MXFP4
+ * GEMM split K inside a workgroup only and leave the workspace alone: NULL and 0
+ * give the same call. The query answers with the bytes that a split across
+ * workgroups would take. */
 size_t hkq_gemm_mxfp4_workspace(int64_t M, int64_t N, int64_t K);
 int hkq_gemm_mxfp4_ws(const void* A, const void* As, const void* B, const void* Bs, void* C, int64_t M, int64_t N,
                       int64_t K, int64_t lda, int64_t ldb, int64_t ldsa, int64_t ldsb, int64_t ldc, void* workspace,
@@ -264,8 +265,9 @@ int hkq_moe_a8w8(const void* X, const void* W, void* Y, const float* x_scale, in
  * K % 128 == 0; K * stride_wk < 2^31). The kernels stage each K-tile of W as
  * it lies (rows of K) and build the MFMA operand with transposed LDS reads, so
  * no K-major copy is made; every output element is the one hkq_moe_a8w8 gives
- * for the same weights in [E, N, K] (bit for bit). Decode-sized launches run the
- * tiled kernel. Replaces moe_op_gemm_a8w8_tk.moe_a8w8 with stride_wn == 1, the
+ * for the same weights in [E, N, K] (bit for bit; up to fp32 summation order
+ * where that call runs its decode kernel, which splits K over waves).
+ * Decode-sized launches run the tiled kernel. Replaces moe_op_gemm_a8w8_tk.moe_a8w8 with stride_wn == 1, the
  * reference's own call (kernels/moe-gemm/moe_op_gemm_a8w8/kernel.cpp:120, the
  * weight read W[e*stride_we + k*stride_wk + n*stride_wn]; tests/test_moe.py:703-729). */
 int hkq_moe_a8w8_kn(const void* X, const void* W, void* Y, const float* x_scale, int64_t xs_stride_tok,
@@ -350,8 +352,9 @@ int hkq_moe_mxfp4(const void* A, const void* B, void* C, const void* A_mx_scale,
  * (row stride stride_bmxk), read in place by the kernels (K-tiles staged as
  * rows of K, operands and e8m0 scale operands built with transposed LDS
  * reads); every output element is the one hkq_moe_mxfp4 gives for the same
- * values in [E, N, K/2] / [E, N, K/32], bit for bit. K % 256 == 0; stride_bk,
- * stride_bmxk >= N; stride_bk, stride_bmxk, stride_be, stride_bmxe multiples
+ * values in [E, N, K/2] / [E, N, K/32], bit for bit (up to fp32 summation order
+ * where that call is decode-sized and splits K over waves). K % 256 == 0;
+ * stride_bk, stride_bmxk >= N; stride_bk, stride_bmxk, stride_be, stride_bmxe multiples
  * of 16 and B_mx_scale 16-byte aligned. Decode-sized launches run the tiled
  * kernel. Replaces moe_op_mxfp4_tk.moe_mxfp4 with stride_bn == stride_bmxn == 1,
  * the reference's own call (kernels/moe-gemm/moe_op_mxfp4/kernel.cpp:155, the
