@@ -78,8 +78,9 @@ def test_gemm_a8w8_strided_and_out_of_place_rows(orc):
 # 20-shape sweep (N, K) x M, each checked element by element against the fp32
 # dequant matmul of the same codes (oracle.gemm_a8w8_ref_f32, pinned against
 # the fp64 reference in tests/test_oracle_gemm_ext.py). These shapes select
-# every A8W8 plan: narrow (M <= 16), skinny / 128 x 64 tiles with split K
-# (M = 128), 128 x 128 tiles (M = 1024) and 256 x 256 tiles (M = 4096).
+# streaming and 32-row tiles (M <= 16), 32 .. 128-row tiles with K split inside
+# the workgroup or, for the long K, across workgroups (M = 128), 128-row and 256 x
+# 256 tiles (M = 1024) and 256 x 256 tiles (M = 4096).
 SWEEP_NK = [(6144, 4096), (4096, 4096), (28672, 4096), (4096, 14336)]
 SWEEP_M = [1, 16, 128, 1024, 4096]
 BASELINE_A8W8 = [(4096, 14336, 4096)] + [(M, N, K) for (N, K) in SWEEP_NK for M in SWEEP_M]
@@ -107,13 +108,16 @@ def test_gemm_a8w8_baseline_sizes_full(orc, M, N, K):
     assert_gemm_close(C, orc.gemm_a8w8_ref_f32(A, B, sa, sb), f"a8w8 {M}x{N}x{K}")
 
 
-# Smaller-tile and split-K plans: M <= 64 uses (32 or 64) x 256 tiles, few
-# 256 x 256 tiles become 128 x 128 tiles (128 x 64 for FP8 with M <= 128 and
-# K <= 8192), and if those are still few (with a long enough K) K is split
-# into fp32 partials that the last split of each tile to finish adds up.
+# Calls of a few tiles: small tiles that split K inside the workgroup, and, where
+# 128-row tiles would fill at most half of the CUs and K is long, K split into
+# fp32 partials over workgroups that the last split of each tile to finish adds up
+# (SPLIT_ACROSS, on 256 CUs: 128 x 64 tiles up to 128 rows, else 128 x 128 ones;
+# ragged M and N; 2 .. 32 splits).
+SPLIT_ACROSS = [(128, 4096, 14336), (65, 2048, 14336), (100, 2052, 14336), (66, 500, 16384), (400, 4096, 14336),
+                (333, 2052, 14336)]
 SPLIT_SHAPES = [(1, 4096, 14336), (16, 2048, 4096), (48, 1024, 2048), (128, 4096, 4096), (96, 28672, 4096), (24, 28672, 4096),
                 (1024, 4096, 14336), (640, 1000, 8192), (256, 1024, 8192), (300, 2052, 2048), (100, 1000, 2048),
-                (128, 6144, 4096)]
+                (128, 6144, 4096)] + SPLIT_ACROSS
 
 
 @pytest.mark.parametrize("M,N,K", SPLIT_SHAPES)
@@ -139,7 +143,7 @@ def _a8w8_ws_launcher(Ad, Bd, sad, sbd, C, ws):
                             torch.cuda.current_stream().cuda_stream)
 
 
-@pytest.mark.parametrize("M,N,K", [(128, 4096, 4096), (64, 4096, 14336), (1024, 1024, 8192)])
+@pytest.mark.parametrize("M,N,K", SPLIT_ACROSS)
 def test_gemm_a8w8_split_workspace_states(orc, M, N, K):
     """The split plan's per-tile arrival counters live in the workspace and
     need no clearing: a workspace full of 0xFF bytes, one left by a call of
@@ -156,12 +160,18 @@ def test_gemm_a8w8_split_workspace_states(orc, M, N, K):
     run = _a8w8_ws_launcher(Ad, Bd, sad, sbd, C, ws)
     run()
     torch.cuda.synchronize()
+    assert not bool((ws[:8] == 0xFF).all()), "the call ran without its split: no arrival counter was claimed"
     first = C.clone()
     assert_gemm_close(host_bf16_f32(first), orc.gemm_a8w8_ref_f32(A, B, sa, sb), f"a8w8 split {M}x{N}x{K}")
     # another shape's split plan on the same workspace, then this one again, twice
-    A2, B2, sa2, sb2 = a8w8_inputs(orc, 96, 2048, 4096, seed=9)
-    C2 = torch.empty((96, 2048), dtype=torch.bfloat16, device="cuda")
-    _a8w8_ws_launcher(dev_u8(A2), dev_u8(B2), dev_f32(sa2), dev_f32(sb2), C2, ws)()
+    M2, N2, K2 = (65, 1028, 16384) if M > 128 else (300, 4092, 14336)  # the other tile size
+    A2, B2, sa2, sb2 = a8w8_inputs(orc, M2, N2, K2, seed=9)
+    C2 = torch.empty((M2, N2), dtype=torch.bfloat16, device="cuda")
+    A2, B2, sa2, sb2 = dev_u8(A2), dev_u8(B2), dev_f32(sa2), dev_f32(sb2)
+    need2 = hkq.lib().hkq_gemm_a8w8_workspace(M2, N2, K2)
+    ws = ws if need2 <= ws.numel() else torch.cat([ws, torch.full((need2,), 0xFF, dtype=torch.uint8, device="cuda")])
+    run = _a8w8_ws_launcher(Ad, Bd, sad, sbd, C, ws)
+    _a8w8_ws_launcher(A2, B2, sa2, sb2, C2, ws)()
     for _ in range(2):
         C.fill_(0)
         run()
@@ -173,7 +183,7 @@ def test_gemm_a8w8_split_graph_replay(orc):
     """A split GEMM captured in a HIP graph replays with one tag: every replay
     (with eager work and synchronization between them) equals the eager call."""
     require_gpu()
-    M, N, K = 128, 4096, 4096
+    M, N, K = 128, 4096, 14336
     A, B, sa, sb = a8w8_inputs(orc, M, N, K, seed=77)
     Ad, Bd, sad, sbd = dev_u8(A), dev_u8(B), dev_f32(sa), dev_f32(sb)
     ws = torch.empty((hkq.lib().hkq_gemm_a8w8_workspace(M, N, K),), dtype=torch.uint8, device="cuda")
@@ -214,10 +224,10 @@ def test_gemm_workspace_plans():
     assert L.hkq_gemm_mxfp4_workspace(64, 8192, 8192) > 0
 
 
-# Narrow path (M <= 16, and M <= 32 with few columns and a short K): one
-# workgroup per 16 * NT columns, K split over its 4 waves (S = K/128 steps,
-# S < 4 leaves waves idle), NT = 1, 2 or 4 by the number of workgroups,
-# ragged N (rows past N read as zeros), ragged M.
+# Few rows: the streaming kernel (one workgroup per 16 columns and 16 rows, K
+# split over its 4 waves: S = K/128 steps, S < 4 leaves waves idle) and the small
+# tiles that take over where its workgroups outnumber the CUs; ragged N (rows past
+# N read as zeros), ragged M.
 NARROW_SHAPES = [(1, 16, 128), (1, 64, 640), (5, 1000, 4096), (16, 4096, 4096), (13, 6144, 256), (16, 28672, 512),
                  (32, 4096, 4096), (20, 6000, 1024), (3, 200, 384)]
 
@@ -323,10 +333,8 @@ def run_blockscale(A, B, sa, sb, group_n):
     return host_bf16_f32(C)
 
 
-# (1, 256, 1024) and M <= 64 below run the narrow block-scale kernel: 16-row
-# tiles (MT = 1, 2, 4), 16- or 32-column slices (N/16 > CUs), one K group
-# (S = 1 < 4 waves), ragged N; (100, 1000, 512) and (192, 2112, 1024) run it in
-# row groups of 64 (few 256 x 256 tiles).
+# M <= 16 below runs the streaming kernel (16- or 32-column slices, N/16 > CUs; one
+# K group, S = 1 < 4 waves; ragged N), the other shapes small tiles.
 @pytest.mark.parametrize("group_n", [128, 1])
 @pytest.mark.parametrize("M,N,K", [(128, 128, 256), (256, 256, 128), (333, 516, 384), (1, 256, 1024),
                                    (600, 772, 2048), (5, 1000, 512), (16, 4160, 1536), (20, 136, 128),
@@ -338,11 +346,13 @@ def test_gemm_blockscale(orc, M, N, K, group_n):
     assert_gemm_close(C, orc.gemm_blockscale_ref(A, B, sa, sb, 128, group_n), f"blockscale {M}x{N}x{K} gn{group_n}")
 
 
-# The tiled kernel with C rows 16-byte aligned: C with a row pitch of N + pad
+# Tiles with C rows 16-byte aligned: C with a row pitch of N + pad
 # (a multiple of 8) whose extra columns must stay untouched, N % 8 == 4 (the
 # last 16-byte piece of a row straddles N) and ragged M.
+# The first three on small tiles, then 256 x 224 and 256 x 256 ones.
 @pytest.mark.parametrize("M,N,K,pad,group_n", [(600, 772, 2048, 4, 128), (333, 516, 384, 12, 1),
-                                               (520, 1028, 256, 4, 1)])
+                                               (520, 1028, 256, 4, 1), (1290, 7172, 384, 4, 128), (777, 5004, 384, 4, 1),
+                                               (1801, 7172, 384, 4, 128), (777, 14340, 128, 4, 1)])
 def test_gemm_blockscale_padded_rows(orc, M, N, K, pad, group_n):
     require_gpu()
     A, B, sa, sb = blockscale_inputs(orc, M, N, K, M + N + K + 7, group_n)
@@ -358,11 +368,14 @@ def test_gemm_blockscale_padded_rows(orc, M, N, K, pad, group_n):
 # Tile widths: grids that 256-column tiles leave a CU short run 256 x 224
 # tiles (waves 4-7 with three n-tiles); HKQ_BLOCKSCALE_W224=0 forces 256-column
 # tiles. Both compute every element with the same K steps and promotions, so
-# their outputs agree bit for bit. Shapes: ragged N (1000 = 4*224 + 104: the
-# last tile's waves 4-7 lie wholly past N), a 128-block boundary inside a
-# 224-column tile (GN 128), per-column scales, and the 2048 x 7168 BASELINE grid.
+# their outputs agree bit for bit. Shapes: ragged M and N (5000 = 22*224 + 72,
+# 3000 = 13*224 + 88: the last tile's waves 4-7 lie wholly past N), a 128-block
+# boundary inside a 224-column tile (GN 128), per-column scales, and the 2048 x
+# 7168 BASELINE grid.
+# The first four run small tiles whatever the variable says.
 @pytest.mark.parametrize("M,N,K,group_n", [(256, 1000, 512, 1), (600, 772, 2048, 128), (333, 516, 384, 1),
-                                           (520, 1792, 640, 128), (2048, 7168, 2048, 128)])
+                                           (520, 1792, 640, 128), (2048, 7168, 2048, 128), (777, 5000, 384, 1),
+                                           (1290, 3000, 384, 1), (1801, 4484, 640, 128), (1290, 7172, 384, 128)])
 def test_gemm_blockscale_tile_widths(orc, monkeypatch, M, N, K, group_n):
     require_gpu()
     A, B, sa, sb = blockscale_inputs(orc, M, N, K, M + N + K + 11, group_n)
@@ -376,7 +389,7 @@ def test_gemm_blockscale_tile_widths(orc, monkeypatch, M, N, K, group_n):
 # The small tiles, each at ragged M and N with an odd count of K groups (uneven
 # splits over the wave groups, a last scale block of 1 or 3 columns): on 256
 # CUs 32x32 / 32x64 (GN 1), 64x64, 128x64, 128x128, 128x256 / 256x224 (GN 1);
-# then 256-row tiles with a ragged last tile. Row strides of A, sa, sb and C
+# then 256-row tiles with a ragged last tile. Row strides of A, B, sa, sb and C
 # hold more than a row; the padding of C stays untouched and that of sa is NaN
 # (a scale read across its row's end would show). Tolerance: that of every
 # GEMM here.
@@ -388,12 +401,14 @@ def test_gemm_blockscale_small_tiles(orc, M, N, K, group_n):
     A, B, sa, sb = blockscale_inputs(orc, M, N, K, M + N + K + 5, group_n)
     Ap = torch.full((M, K + 64), 0x7F, dtype=torch.uint8, device="cuda")
     Ap[:, :K] = dev_u8(A)
+    Bp = torch.full((N, K + 80), 0x7F, dtype=torch.uint8, device="cuda")
+    Bp[:, :K] = dev_u8(B)
     sap = torch.full((M, K // 128 + 3), float("nan"), dtype=torch.float32, device="cuda")
     sap[:, :K // 128] = dev_f32(sa)
     sbp = torch.full((K // 128, sb.shape[1] + 5), float("nan"), dtype=torch.float32, device="cuda")
     sbp[:, :sb.shape[1]] = dev_f32(sb)
     Cp = torch.full((M, N + 4), 7.0, dtype=torch.bfloat16, device="cuda")
-    C = hkq.gemm_blockscale(Ap[:, :K], dev_u8(B), sap[:, :K // 128], sbp[:, :sb.shape[1]], Cp[:, :N], group_n=group_n)
+    C = hkq.gemm_blockscale(Ap[:, :K], Bp[:, :K], sap[:, :K // 128], sbp[:, :sb.shape[1]], Cp[:, :N], group_n=group_n)
     torch.cuda.synchronize()
     assert bool((Cp[:, N:] == 7.0).all()), "stores past N reached the row padding"
     assert_gemm_close(host_bf16_f32(C), orc.gemm_blockscale_ref_f32(A, B, sa, sb, 128, group_n),
@@ -486,8 +501,8 @@ def test_gemm_bf16_stream_tiles(orc, M, N, K):
 
 # The small tiles of the dense GEMMs with K split over the workgroup's waves:
 # odd counts of K-tiles (uneven shares of the wave groups, a last scale block
-# of 1 or 3 K-tiles) and a half last K-tile, ragged M and N, rows of A (and of its
-# scales) padded with NaN codes, C's padding untouched. K is in 128-byte K-tiles
+# of 1 or 3 K-tiles) and a half last K-tile, ragged M and N, rows of A and B (and of
+# their scales) padded with NaN codes, C's padding untouched. K is in 128-byte K-tiles
 # per row; on 256
 # CUs the sizes are 32x32, 32x64, 32x128, 64x64, 128x64, 128x128, 128x256 or
 # two 128x128 workgroups per CU, as the operand format's costs decide.
@@ -505,14 +520,18 @@ def test_gemm_small_tiles(orc, mode, M, N, KT):
         xa, xw = orc.randn_bf16((M, K), seed=M), orc.randn_bf16((N, K), seed=N, std=0.02)
         Ap = torch.full((M, K + 24), float("nan"), dtype=torch.bfloat16, device="cuda")
         Ap[:, :K] = torch.from_numpy(xa.view(np.int16)).cuda().view(torch.bfloat16)
-        hkq.gemm_bf16(Ap[:, :K], torch.from_numpy(xw.view(np.int16)).cuda().view(torch.bfloat16), C)
+        Bp = torch.full((N, K + 40), float("nan"), dtype=torch.bfloat16, device="cuda")
+        Bp[:, :K] = torch.from_numpy(xw.view(np.int16)).cuda().view(torch.bfloat16)
+        hkq.gemm_bf16(Ap[:, :K], Bp[:, :K], C)
         ref = orc.gemm_bf16_ref(xa, xw)
     elif mode == "a8w8":
         K = int(128 * KT)
         A, B, sa, sb = a8w8_inputs(orc, M, N, K, seed=M + N + K)
         Ap = torch.full((M, K + 48), 0x7F, dtype=torch.uint8, device="cuda")
         Ap[:, :K] = dev_u8(A)
-        hkq.gemm_a8w8(Ap[:, :K], dev_u8(B), dev_f32(sa), dev_f32(sb), C)
+        Bp = torch.full((N, K + 80), 0x7F, dtype=torch.uint8, device="cuda")
+        Bp[:, :K] = dev_u8(B)
+        hkq.gemm_a8w8(Ap[:, :K], Bp[:, :K], dev_f32(sa), dev_f32(sb), C)
         ref = orc.gemm_a8w8_ref_f32(A, B, sa, sb)
     else:
         K = int(256 * KT)
@@ -521,7 +540,11 @@ def test_gemm_small_tiles(orc, mode, M, N, KT):
         Ap[:, :K // 2] = dev_u8(Aq)
         Asp = torch.full((M, K // 32 + 4), 0xFF, dtype=torch.uint8, device="cuda")
         Asp[:, :K // 32] = dev_u8(As)
-        hkq.gemm_mxfp4(Ap[:, :K // 2], Asp[:, :K // 32], dev_u8(Bq), dev_u8(Bs), C)
+        Bp = torch.full((N, K // 2 + 48), 0x77, dtype=torch.uint8, device="cuda")
+        Bp[:, :K // 2] = dev_u8(Bq)
+        Bsp = torch.full((N, K // 32 + 12), 0xFF, dtype=torch.uint8, device="cuda")
+        Bsp[:, :K // 32] = dev_u8(Bs)
+        hkq.gemm_mxfp4(Ap[:, :K // 2], Asp[:, :K // 32], Bp[:, :K // 2], Bsp[:, :K // 32], C)
         ref = orc.gemm_mxfp4_ref_f32(Aq, As, Bq, Bs)
     torch.cuda.synchronize()
     assert bool((Cp[:, N:] == 7.0).all()), "stores past N reached the row padding"

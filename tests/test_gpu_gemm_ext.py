@@ -44,11 +44,12 @@ def test_gemm_bf16(orc, M, N, K):
     assert_gemm_close(host_bf16_f32(C), orc.gemm_bf16_ref(A, B), f"bf16 {M}x{N}x{K}")
 
 
-def test_gemm_bf16_split_equals_unsplit(orc):
-    """A grid small enough to split K (workspace plan) gives the same bits as the
-    unsplit plan up to fp32 summation order: both within the bar, and close."""
+@pytest.mark.parametrize("M,N,K", [(32, 256, 16384), (300, 1024, 14336), (333, 2052, 14336)])
+def test_gemm_bf16_split_equals_unsplit(orc, M, N, K):
+    """With and without a workspace the same up to fp32 summation order: both
+    within the bar. K is split inside the workgroup in the first shape, across
+    workgroups (11 and 6 splits of 128 x 128 tiles on 256 CUs) in the others."""
     require_gpu()
-    M, N, K = 32, 256, 16384
     A = orc.randn_bf16((M, K), seed=1)
     B = orc.randn_bf16((N, K), seed=2, std=0.05)
     C1 = host_bf16_f32(hkq.gemm_bf16(dev_bf16(A), dev_bf16(B), split=True))

@@ -33,8 +33,15 @@ def make_problem(orc, T, E, topk, K, N, seed, skew=None):
     return assigns, hist, offs, gather, ed, X, xs.reshape(-1), Wq.reshape(E, N, K), ws.reshape(E, N)
 
 
-def run_moe(X, W, hist, offs, gather, ed, topk, xs=None, ws=None, bias=None, y_rows=None):
-    Xd, Wd = dev_u8(X), dev_u8(W)
+def padded_rows(codes, pad):
+    """Device codes whose rows lie `pad` bytes further apart, NaN codes between them."""
+    t = torch.full((*codes.shape[:-1], codes.shape[-1] + pad), 0x7F, dtype=torch.uint8, device="cuda")
+    t[..., :codes.shape[-1]] = dev_u8(codes)
+    return t[..., :codes.shape[-1]]
+
+
+def run_moe(X, W, hist, offs, gather, ed, topk, xs=None, ws=None, bias=None, y_rows=None, pad=0):
+    Xd, Wd = padded_rows(X, pad), padded_rows(W, pad)
     args = dict(gather=dev_i32(gather) if gather is not None else None,
                 x_scale=dev_f32(xs) if xs is not None else None,
                 w_scale=dev_f32(ws) if ws is not None else None,
@@ -70,11 +77,13 @@ def test_moe_reference_setup(orc):
 # 16-row groups, ragged N and K-steps uneven over the 4 waves; (24, 2, 2, 384,
 # 4104) has 48 rows and a wide N, so it takes the tiled kernel. N >= 8192 (32
 # or more column tiles) walks the columns in XCD-aligned blocks of 8: 8320 has
-# 33 column tiles (a last block of one), 700 x 3 with topk 2 odd pair groups.
+# 33 column tiles (a last block of one), 700 x 3 with topk 2 odd pair groups;
+# (7, 8, 1, 6272, 4360) streams for its long K and one or two rows per expert.
 @pytest.mark.parametrize("T,E,topk,K,N", [(300, 4, 2, 512, 520), (1, 8, 2, 256, 512), (1000, 8, 2, 1024, 1024),
                                           (257, 3, 1, 384, 260), (77, 4, 2, 320, 256), (5, 8, 2, 512, 4100),
                                           (16, 8, 2, 384, 1000), (16, 4, 2, 640, 4200), (30, 8, 2, 256, 520),
-                                          (24, 2, 2, 384, 4104), (300, 4, 2, 256, 8320), (700, 3, 2, 384, 9216)])
+                                          (24, 2, 2, 384, 4104), (300, 4, 2, 256, 8320), (700, 3, 2, 384, 9216),
+                                          (7, 8, 1, 6272, 4360)])
 def test_moe_per_token_per_channel(orc, T, E, topk, K, N):
     require_gpu()
     _, hist, offs, gather, ed, X, xs, W, ws = make_problem(orc, T, E, topk, K, N, T + N)
@@ -477,8 +486,8 @@ def test_moe_small_tiles_k_order(orc, fmt, T, E, topk, K, N):
 # The A8W8 small tiles by mean rows per expert (K up to 3072: 10 and 33 on
 # 64x128, 75 on 128x256; above: 5 and 32 on 64x64, 76 on 128x128, 150 on 128x256),
 # routing skewed so that some experts hold several row groups or blocks and some
-# no row, odd counts of K-tiles, ragged N, every scale form, -1 / malformed words
-# between the live ones.
+# no row, odd counts of K-tiles, ragged N, padded rows of X and W, every scale form,
+# -1 / malformed words between the live ones.
 @pytest.mark.parametrize("T,E,topk,K,N,scales", [
     (3, 8, 2, 128, 1000, "none"), (40, 8, 2, 640, 300, "channel"), (40, 8, 2, 640, 4100, "expert"), (100, 6, 2, 1152, 260, "expert"),
     (150, 4, 2, 896, 772, "channel"), (20, 8, 2, 4096, 260, "channel"), (130, 8, 2, 4096, 388, "expert"),
@@ -495,7 +504,7 @@ def test_moe_small_tiles(orc, T, E, topk, K, N, scales):
     if scales == "none":  # codes below 2: sums of the size the absolute bound is meant for
         X, W = X & 0xBF, W & 0xBF
     xs, ws = {"none": (None, None), "channel": (xs, ws), "expert": (xs, ws[:, 0].copy())}[scales]
-    Y = run_moe(X, W, hist, offs, gather, words, topk, xs=xs, ws=ws)
+    Y = run_moe(X, W, hist, offs, gather, words, topk, xs=xs, ws=ws, pad=48)
     xs, ws = (1.0, np.ones(E)) if xs is None else (xs, ws)
     check_rows(orc, Y, orc.moe_ref(X, W, xs, ws, None, gather, hist, offs, ed, topk, 128, "enk"))
 
@@ -530,8 +539,8 @@ def test_moe_small_tile_row_groups(orc, fmt, K, N):
 # 10 and 33 on 64x128, 75 on 128x256, 115 on block pairs; above: 4 and 25 on 64x64,
 # 75 on 128x128, 150 on 128x256), routing skewed so that some experts hold several
 # row groups or blocks and some no row, odd counts of K-tiles, one to four K-tiles
-# per scale group, ragged N, a bias, -1 / malformed words between the live ones and scale rows
-# padded with NaN.
+# per scale group, ragged N, a bias, -1 / malformed words between the live ones and
+# rows of X, W and the scales padded with NaN.
 @pytest.mark.parametrize("T,E,topk,K,N,gk", [(40, 8, 2, 640, 300, 128), (3, 8, 2, 128, 1000, 128),
                                              (100, 6, 2, 1152, 260, 128), (150, 4, 2, 896, 772, 256),
                                              (150, 4, 2, 3200, 132, 128), (230, 4, 2, 640, 1028, 128),
@@ -554,7 +563,7 @@ def test_moe_blockscale_small_tiles(orc, T, E, topk, K, N, gk):
     bias = (rng.standard_normal((E, N)) * 0.1).astype(np.float32) if T % 4 == 0 else None
     xsp = torch.full((T, G + 3), float("nan"), dtype=torch.float32, device="cuda")
     xsp[:, :G] = dev_f32(xs)
-    Y = hkq.moe_a8w8_blockscale(dev_u8(X), dev_u8(W), dev_i32(hist), dev_i32(offs), dev_i32(ed), topk, xsp[:, :G],
+    Y = hkq.moe_a8w8_blockscale(padded_rows(X, 48), padded_rows(W, 80), dev_i32(hist), dev_i32(offs), dev_i32(ed), topk, xsp[:, :G],
                                 dev_f32(ws), gk, 128, gather=dev_i32(gather),
                                 bias=dev_f32(bias) if bias is not None else None)
     torch.cuda.synchronize()

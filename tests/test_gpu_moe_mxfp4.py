@@ -120,7 +120,7 @@ def test_moe_mxfp4_decode_layouts(orc):
 # The small tiles by mean valid entries per expert (8 entries in all on 32x32 with
 # K in four, 10, 3 and 33 on 64x64, 75 on block pairs: more blocks than experts),
 # routing skewed so that some experts hold several row groups or blocks, odd
-# counts of K-tiles, ragged N, routed weights, padded scale rows, a block whose
+# counts of K-tiles, ragged N, routed weights, padded code and scale rows, a block whose
 # entries are scattered over its 128, one of expert -1 (zeros for its valid
 # rows) and one past the last expert (left untouched).
 @pytest.mark.parametrize("T,E,topk,K,N", [(4, 8, 2, 256, 260), (40, 8, 2, 4352, 132), (96, 64, 2, 768, 516),
@@ -137,13 +137,13 @@ def test_moe_mxfp4_small_tiles(orc, T, E, topk, K, N):
     eids[-1], eids[-2] = -1, E + 1
     w = rng.random(nv).astype(np.float32)
 
-    def padded(x):
-        t = torch.full((*x.shape[:-1], x.shape[-1] + 4), 255, dtype=torch.uint8, device="cuda")
+    def padded(x, pad=4):
+        t = torch.full((*x.shape[:-1], x.shape[-1] + pad), 255, dtype=torch.uint8, device="cuda")
         t[..., :x.shape[-1]] = dev_u8(x)
         return t[..., :x.shape[-1]]
 
     C = torch.full((nv, N), 7.0, dtype=torch.bfloat16, device="cuda")
-    hkq.moe_mxfp4(dev_u8(Aq), padded(As), dev_u8(Bq), padded(Bs), dev_i32(s), dev_i32(eids), nv, topk,
+    hkq.moe_mxfp4(padded(Aq, 16), padded(As), padded(Bq, 48), padded(Bs), dev_i32(s), dev_i32(eids), nv, topk,
                   topk_weights=dev_f32(w), C=C)
     torch.cuda.synchronize()
     keep = np.concatenate([eids[:-2], eids[-1:]])
