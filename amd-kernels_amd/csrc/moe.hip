@@ -1407,19 +1407,19 @@ static int moe_a8w8_impl(const void* X, const void* W, void* Y, const float* x_s
     // sorted rows without a gather. Small tiles (moe_tile) take K-contiguous
     // weights of whole K-tiles and scales they read as they are stored: none,
     // one per expert or one float4-readable value per channel. Measured on
-    // MI355X (us, gate/up and down; the tile taken against the streaming and
-    // block-pair kernels): 8 experts of 4096 x 14336, 8 tokens 257 / 262, 24: 260 /
-    // 345, 64: 268 / 373, 150: 277 / 391, 300: 325 / 506, 500: 388 / 553, 900: 445 /
-    // 464, 1400: 653 / 753; 32 of 2048 x 2816, 8 tokens 64 / 97, 56: 101 / 129, 250:
-    // 107 / 135, 900: 142 / 176. Decode sizes with fewer column tiles than CUs keep
-    // the streaming kernel (one token's down projection, 8 experts: 22 against 38;
-    // 32 experts of 2048 x 2816, one token's layer 26 both).
+    // MI355X (us, gate/up and down; the kernels taken against the streaming and
+    // block-pair ones): 8 experts of 4096 x 14336, 8 tokens 256 / 259, 24: 257 /
+    // 343, 64: 265 / 368, 150: 268 / 385, 300: 300 / 494, 500: 365 / 538, 850: 371 /
+    // 439, 1400: 625 / 724; 32 of 2048 x 2816, 8 tokens 62 / 94, 48: 98 / 125, 250:
+    // 101 / 130, 850: 127 / 153. Decode sizes with fewer column tiles than CUs keep
+    // the streaming kernel (one token's down projection, 8 experts: 21 against 38;
+    // 32 experts of 2048 x 2816, one token's layer 24 both). So do those with one or
+    // two rows per expert over a long K, where the stream's 16-row workgroups keep
+    // as much in flight and no tile is padded (16 experts, K 8192, N 5120, 16 rows
+    // 89 against 105, 28 rows 93 and 106; 8 of K 14336, N 4096, 8 rows 49.5 and 52,
+    // 16 rows 78 and 72).
     const int64_t routed = gather ? T * topk : T;
     const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
-    // So do those with one or two rows per expert over a long K, where the
-    // stream's 16-row workgroups keep as much in flight and no tile is padded
-    // (16 experts, K 8192, N 5120, 16 rows 89 us against 105, 28 rows 93 and 106;
-    // 8 of K 14336, N 4096, 8 rows 49.5 and 52; 16 rows 78 and 72).
     const bool few = std::min(routed, E) * ((N + 127) / 128) < ncu || (K > 6144 && 2 * routed > E && routed < 2 * E);
     const bool decode = (routed <= 32 || (routed <= MOE_NARROW_MAX_ROWS && N <= 4096)) && !wt && K % 128 == 0 &&
                         64 * stride_w < (1ll << 31);
