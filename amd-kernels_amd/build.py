@@ -32,7 +32,7 @@ PY_INCLUDE = sysconfig.get_paths()["include"]
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 ARCH = "gfx950"
 # Packed-FP32 VALU forms are disabled for all device code (some of their forms
-# have produced wrong results on this pool's MI355X boxes).
+# have produced wrong results on MI355X).
 HIP_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

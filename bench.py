@@ -14,7 +14,7 @@ GEMM): algorithmic flops per launch / average launch duration against the
 MI355X dense FP8 peak; `traffic` is the HBM bytes per launch measured with
 rocprofv3 PMC counters (FETCH_SIZE + WRITE_SIZE) and read from the committed
 profile summary. `cpu_baseline` times the CPU port of the reference formula
-(oracle/cpu_baseline.py) on BASELINE config 0.
+(oracle/cpu_baseline.py) on the smallest configuration.
 """
 from __future__ import annotations
 
@@ -477,7 +477,7 @@ def main():
     sweep = []
     if args.only in (None, "sweep"):
         log("a8w8 sweep")
-        # BASELINE's data: bf16 activations ~N(0,1) and weights ~N(0,0.02),
+        # The benchmark's data: bf16 activations ~N(0,1) and weights ~N(0,0.02),
         # quantized per token / per channel to E4M3FN by this library
         for si, (nn, kk) in enumerate(SWEEP_NK):
             wb, wsb = hkq.per_token_quant(seeded_bf16_dev((nn, kk), 0.02, 100 + si))
@@ -533,7 +533,7 @@ def main():
 
     cpu = None
     if not args.no_cpu:
-        log("cpu baseline (oracle/cpu_baseline.py, BASELINE config 0)")
+        log("cpu baseline (oracle/cpu_baseline.py)")
         from oracle import cpu_baseline
 
         r = cpu_baseline.run()

@@ -30,7 +30,7 @@ def dequant_matmul(q: torch.Tensor, s: torch.Tensor, wq: torch.Tensor, ws: torch
 
 def run(M: int = 128, N: int = 4096, K: int = 4096, seed: int = 0, budget_s: float = 12.0, warmup: int = 3,
         min_reps: int = 10):
-    """Time quant + dequant matmul on config 0 of BASELINE (X [M,K] ~ N(0,1),
+    """Time quant + dequant matmul on the smallest configuration (X [M,K] ~ N(0,1),
     W [N,K] ~ N(0,0.02) quantized per output channel). Returns a dict with the
     median times and TFLOP/s of the total."""
     threads = len(os.sched_getaffinity(0))

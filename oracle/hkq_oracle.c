@@ -3,7 +3,7 @@
  *
  * TEST INFRASTRUCTURE ONLY. Nothing in the product path may link or call this
  * file; only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg
- * use it, and only as the checker (or the timed CPU baseline).
+ * use it, and only as the oracle (or the timed CPU baseline).
  *
  * Plain scalar C, written for clarity, not speed. Every routine cites the
  * reference formula it restates (paths relative to the reference repository).

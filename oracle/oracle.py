@@ -1,7 +1,7 @@
 """CPU oracle for the quantized-GEMM hot path. TEST INFRASTRUCTURE ONLY.
 
 Only ``tests/``, ``__graft_entry__.smoke()`` and ``bench.py``'s ``cpu_baseline``
-leg may import this module, and only as the checker (or the timed CPU
+leg may import this module, and only as the oracle (or the timed CPU
 baseline). The product path (``amd-kernels_amd``) never imports it.
 
 The element-level arithmetic lives in ``hkq_oracle.c`` (plain scalar C, built
@@ -51,7 +51,7 @@ moe_blockscale_ref     per-expert dense gemm_blockscale_ref on the gathered rows
                        with each group's scales (group_k 64 / 128, group_n 1 /
                        64 / 128), and for [E, K, N] weights the same result
                        (tests/test_oracle_moe.py).
-*_ref_f32              fp32 restatements used at BASELINE sizes (gemm_a8w8,
+*_ref_f32              fp32 restatements used at the benchmark's sizes (gemm_a8w8,
                        gemm_blockscale, gemm_mxfp4, moe, moe_mxfp4): against
                        the fp64 references within 2^-16 of the sum of |terms|
                        (tests/test_oracle_gemm_ext.py, tests/test_oracle_moe.py).
@@ -342,7 +342,7 @@ def gemm_blockscale_ref(A, B, sa, sb, group_k: int = 128, group_n: int = 128) ->
     return C
 
 
-# Full-output references at BASELINE sizes: the same formulas with the decoded
+# Full-output references at the benchmark's sizes: the same formulas with the decoded
 # operands multiplied in fp32 by torch on all host threads (seconds instead of
 # minutes for 10^11-10^12 flops). Products of E4M3 / E2M1 values are exact in
 # fp32; the fp32 sums differ from the fp64 ones by ~sqrt(K) * 2^-24 of the sum
@@ -535,7 +535,7 @@ def moe_blockscale_ref(X, W, x_scale, w_scale, bias, gather, hist, offs, expt_da
 
 def moe_ref_f32(X, W, x_scale, w_scale, gather, hist, offs, expt_data, topk, group_k=None, group_n=1,
                 block_m: int = 128):
-    """fp32 full-output MoE reference for BASELINE sizes: per expert one fp32
+    """fp32 full-output MoE reference for the benchmark's sizes: per expert one fp32
     product of pre-scaled operands (W [E, N, K] e4m3 codes). x_scale: [T]
     (per token) or [T, G]; w_scale: [E, N] (per channel) or [E, G, C] with
     group_k / group_n. Rows of the listed tiles only; the rest NaN (float32)."""

@@ -4,7 +4,7 @@
  *
  * TEST INFRASTRUCTURE ONLY. Nothing in the product path may link or call this
  * file; only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg
- * use it, and only as the checker.
+ * use it, and only as the oracle.
  *
  * Plain scalar C following each reference routine step by step. How each one
  * is pinned is listed in oracle/oracle.py's header.

@@ -1,9 +1,9 @@
 """Helpers shared by the GPU parity tests (bf16 bit patterns <-> device tensors,
-seeded inputs, the north-star GEMM tolerance)."""
+seeded inputs, the GEMM tolerance)."""
 import numpy as np
 import torch
 
-# GEMM tolerance of the north star: bf16 output within 1e-2 relative / 2e-2
+# GEMM tolerance: bf16 output within 1e-2 relative / 2e-2
 # absolute of the fp32-dequant matmul, elementwise |C - ref| <= ATOL + RTOL*|ref|.
 GEMM_RTOL = 1e-2
 GEMM_ATOL = 2e-2
@@ -40,7 +40,7 @@ def host_bf16_f32(t: torch.Tensor) -> np.ndarray:
 
 def assert_gemm_close(C: np.ndarray, ref: np.ndarray, what: str = "", rows_per_chunk: int = 512):
     """Elementwise |C - ref| <= ATOL + RTOL |ref| and Frobenius relative error
-    < RTOL, checked in row chunks so that full outputs at BASELINE sizes
+    < RTOL, checked in row chunks so that full outputs at the benchmark's sizes
     (10^8 elements) need no fp64 copies of the whole matrix."""
     C = np.asarray(C)
     ref = np.asarray(ref)

@@ -1,10 +1,10 @@
 """GPU parity of the dense GEMMs against the CPU oracle, through the C ABI.
 
-Bar (north star): bf16 C within |C - ref| <= 2e-2 + 1e-2 |ref| of the fp64
+Bar: bf16 C within |C - ref| <= 2e-2 + 1e-2 |ref| of the fp64
 dequant matmul of the same codes and scales, and Frobenius relative error
-< 1e-2. Inputs follow BASELINE's distributions (acts ~N(0,1), weights
+< 1e-2. Inputs follow the benchmark's distributions (acts ~N(0,1), weights
 ~N(0,0.02)) through the oracle quantizers, so the GEMM test does not depend on
-the GPU quantizer. Small shapes and every BASELINE size (the A8W8 headline and 20-shape sweep,
+the GPU quantizer. Small shapes and every size of the benchmark (the A8W8 headline and 20-shape sweep,
 both MXFP4 sizes, the three block-scale shapes) are compared in full, the
 latter against fp32 products of the decoded operands; plus closed forms.
 """
@@ -74,7 +74,7 @@ def test_gemm_a8w8_strided_and_out_of_place_rows(orc):
     assert np.all(C[:, N:] == 7.0)
 
 
-# Full-output parity at every BASELINE A8W8 size: the headline shape and the
+# Full-output parity at every A8W8 size of the benchmark: the headline shape and the
 # 20-shape sweep (N, K) x M, each checked element by element against the fp32
 # dequant matmul of the same codes (oracle.gemm_a8w8_ref_f32, pinned against
 # the fp64 reference in tests/test_oracle_gemm_ext.py). These shapes select
@@ -83,7 +83,7 @@ def test_gemm_a8w8_strided_and_out_of_place_rows(orc):
 # 256 tiles (M = 1024) and 256 x 256 tiles (M = 4096).
 SWEEP_NK = [(6144, 4096), (4096, 4096), (28672, 4096), (4096, 14336)]
 SWEEP_M = [1, 16, 128, 1024, 4096]
-BASELINE_A8W8 = [(4096, 14336, 4096)] + [(M, N, K) for (N, K) in SWEEP_NK for M in SWEEP_M]
+BENCH_A8W8 = [(4096, 14336, 4096)] + [(M, N, K) for (N, K) in SWEEP_NK for M in SWEEP_M]
 
 _weight_cache = {}
 
@@ -98,7 +98,7 @@ def _weights(orc, N, K, seed):
     return _weight_cache[key]
 
 
-@pytest.mark.parametrize("M,N,K", BASELINE_A8W8)
+@pytest.mark.parametrize("M,N,K", BENCH_A8W8)
 def test_gemm_a8w8_baseline_sizes_full(orc, M, N, K):
     require_gpu()
     A, sa = orc.quant_rowwise(orc.randn_bf16((M, K), seed=M + K), None, "fp8")
@@ -300,7 +300,7 @@ def test_gemm_mxfp4_closed_form_scales(orc):
 
 @pytest.mark.parametrize("M", [128, 4096])
 def test_gemm_mxfp4_baseline_sizes_full(orc, M):
-    """BASELINE MXFP4 sizes, every output element against the fp32 product of
+    """The benchmark's MXFP4 sizes, every output element against the fp32 product of
     the decoded operands (oracle.gemm_mxfp4_ref_f32)."""
     require_gpu()
     N = K = 8192
@@ -371,7 +371,7 @@ def test_gemm_blockscale_padded_rows(orc, M, N, K, pad, group_n):
 # their outputs agree bit for bit. Shapes: ragged M and N (5000 = 22*224 + 72,
 # 3000 = 13*224 + 88: the last tile's waves 4-7 lie wholly past N), a 128-block
 # boundary inside a 224-column tile (GN 128), per-column scales, and the 2048 x
-# 7168 BASELINE grid.
+# 7168 grid.
 # The first four run small tiles whatever the variable says.
 @pytest.mark.parametrize("M,N,K,group_n", [(256, 1000, 512, 1), (600, 772, 2048, 128), (333, 516, 384, 1),
                                            (520, 1792, 640, 128), (2048, 7168, 2048, 128), (777, 5000, 384, 1),

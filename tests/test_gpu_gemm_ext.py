@@ -9,7 +9,7 @@ oracle, through the C ABI and the reference-named modules:
   (fused_gemm_a8w8_blockscale_mul_add_tk; :498-533) and next to a bf16 GEMM
   (fused_gemm_a8w8_blockscale_a16w16_tk; :454-496).
 
-Bar: the north-star GEMM tolerance (|C - ref| <= 2e-2 + 1e-2 |ref|, Frobenius
+Bar: the GEMM tolerance (|C - ref| <= 2e-2 + 1e-2 |ref|, Frobenius
 relative error < 1e-2) against the fp64 oracle on the same codes, scales and
 bf16 values. The reference tests' own inputs are bf16 tensors; the FP8 paths
 take their E4M3FN quantization (oracle quantizers), as the dense modules do.
@@ -72,7 +72,7 @@ def test_gemm_bf16_identity_closed_form(orc):
 
 def test_gemm_a16w16_module_reference_call(orc):
     """tests/test_gemm.py:21-42 as written: M = N = K = 256, torch.randn bf16
-    (seed 42), rel-err bar 0.02 of the reference plus the north-star bar."""
+    (seed 42), rel-err bar 0.02 of the reference plus the GEMM bar."""
     require_gpu()
     import hipkittens as hk
     M, N, K = 256, 256, 256

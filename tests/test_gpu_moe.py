@@ -3,7 +3,7 @@
 C ABI and through the reference-named modules.
 
 Routing metadata follows the OGS contract (tests/test_moe.py:97-128) built by
-oracle.ogs_routing. Bar: the north-star GEMM tolerance on every routed row;
+oracle.ogs_routing. Bar: the GEMM tolerance on every routed row;
 rows that no tile covers stay untouched.
 """
 import numpy as np
@@ -358,7 +358,7 @@ def device_weights_fp8(E, N, K, seed):
 
 @pytest.mark.parametrize("K,N", [(4096, 28672), (14336, 4096)])
 def test_moe_mixtral_full(orc, K, N):
-    """BASELINE MoE shapes (Mixtral-8x7B: T=4096, E=8, top-2; gate/up K=4096,
+    """The benchmark's MoE shapes (Mixtral-8x7B: T=4096, E=8, top-2; gate/up K=4096,
     N=28672 and down K=14336, N=4096), softmax top-2 routing from seeded logits,
     per-token x per-channel scales: every routed output row against the fp32
     oracle (oracle.moe_ref_f32, pinned in tests/test_oracle_moe.py)."""

@@ -1,7 +1,7 @@
 """GPU parity of the MXFP4 MoE GEMM (block-sorted routing) against the CPU
 oracle (oracle.moe_mxfp4_ref: moe-gemm/moe_op_mxfp4/kernel.cpp:90-237
 restated over exactly decoded operands), through the C ABI and the
-reference-named module. Bar: the north-star GEMM tolerance on every written
+reference-named module. Bar: the GEMM tolerance on every written
 row; rows no block names stay untouched."""
 import numpy as np
 import pytest

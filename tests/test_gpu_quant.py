@@ -3,7 +3,7 @@
 Bar: bit-exact codes and scales (integer/byte work). Inputs are seeded on the
 CPU and copied, so both sides see identical bf16 bytes. Edge rows cover what
 the reference kernels meet: all-zero rows/blocks, bf16 subnormals, extreme
-dynamic range, +-inf and NaN, M = 1, ragged K, and BASELINE sizes.
+dynamic range, +-inf and NaN, M = 1, ragged K, and the benchmark's sizes.
 """
 import numpy as np
 import pytest
@@ -192,7 +192,7 @@ def test_static_fp8(orc):
 
 
 def test_per_token_quant_baseline_size(orc):
-    """BASELINE quantizer size: bf16 [4096, 4096], full comparison."""
+    """The benchmark's quantizer size: bf16 [4096, 4096], full comparison."""
     require_gpu()
     xb = orc.randn_bf16((4096, 4096), seed=1)
     q, s = hkq.per_token_quant(dev_bf16(xb), hkq.KIND_FP8)

@@ -94,7 +94,7 @@ def _close_to_fp64(f32, f64, a_abs_b_abs):
 
 
 def test_fp32_references_match_fp64(orc):
-    """The fp32 full-output references (used at BASELINE sizes) against the
+    """The fp32 full-output references (used at the benchmark's sizes) against the
     fp64 ones on ragged shapes with per-row/column/group scales that differ
     everywhere, so a transposed or mis-indexed scale would fail."""
     M, N, K = 200, 260, 1024

@@ -72,7 +72,7 @@ def test_moe_blockscale_ref_matches_dense_per_expert(orc):
 
 
 def test_moe_fp32_references_match_fp64(orc):
-    """The fp32 full-output MoE references (BASELINE sizes) against the fp64
+    """The fp32 full-output MoE references (the benchmark's sizes) against the fp64
     ones: per-token x per-channel, per-K-group scales, and MXFP4."""
     T, E, topk, K, N = 200, 4, 2, 512, 160
     hist, offs, gather, ed = _routing(orc, T, E, topk, 7)
