@@ -861,7 +861,7 @@ static int dense_tile_plan(int mode, const DenseParams& p, int64_t batch, const 
     static const TileCosts FP4 = {{{0.091f, 1.8f}, {0.125f, 1.9f}, {0.233f, 2.7f}, {0.5f, 1.1f}, {0.188f, 2.9f},
                                    {0.431f, 2.2f}, {0.478f, 2.9f}, {-1.f, 0.f}, {0.717f, 1.2f}, {0.909f, 3.9f}},
                                   {0.611f, 0.0f}, 0.f, 0.f, 0.f, 0.f, 0.f};
-    static const TileCosts BF16 = {{{0.098f, 1.0f}, {0.132f, 1.5f}, {0.216f, 1.7f}, {0.31f, 0.85f}, {0.162f, 2.2f},
+    static const TileCosts BF16 = {{{0.098f, 1.0f}, {0.132f, 1.45f}, {0.216f, 1.7f}, {0.31f, 0.85f}, {0.162f, 2.2f},
                                     {0.278f, 1.7f}, {0.347f, 0.6f}, {0.606f, 1.2f}, {0.645f, 0.9f}, {0.647f, 2.1f}},
                                    {0.559f, 0.6f}, 0.f, 0.f, 0.494f, 5.5f, 1.2f};
     const TileCosts& T = mode == MODE_A8W8 ? A8W8 : mode == MODE_MXFP4 ? FP4 : BF16;
